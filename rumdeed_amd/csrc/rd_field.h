@@ -6,54 +6,12 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
+#include "rd_fp64.h"
 #include "rd_internal.h"
 
 namespace rd {
-
-// FP64 device forms of the reference expressions.
-__device__ __forceinline__ void ic_planar64(double z_a, double z_b, double dx, double dy,
-                                            double dxy2, int nic, double dd, double es,
-                                            double& icx, double& icy, double& icz) {
-  double z_ic = -1.0 * z_b;
-  double diff_z = z_a - z_ic;
-  double r = __builtin_sqrt(dxy2 + diff_z * diff_z) + es;
-  double inv_r3 = 1.0 / (r * r * r);
-  double ix = -dx * inv_r3, iy = -dy * inv_r3, iz = -diff_z * inv_r3;
-  for (int n = 1; n <= nic; ++n) {
-    double tnd = 2.0 * n * dd;
-    z_ic = tnd - z_b;
-    diff_z = z_a - z_ic;
-    r = __builtin_sqrt(dxy2 + diff_z * diff_z) + es;
-    inv_r3 = 1.0 / (r * r * r);
-    ix = ix - dx * inv_r3;
-    iy = iy - dy * inv_r3;
-    iz = iz - diff_z * inv_r3;
-    z_ic = -2.0 * n * dd - z_b;
-    diff_z = z_a - z_ic;
-    r = __builtin_sqrt(dxy2 + diff_z * diff_z) + es;
-    inv_r3 = 1.0 / (r * r * r);
-    ix = ix - dx * inv_r3;
-    iy = iy - dy * inv_r3;
-    iz = iz - diff_z * inv_r3;
-    z_ic = tnd + z_b;
-    diff_z = z_a - z_ic;
-    r = __builtin_sqrt(dxy2 + diff_z * diff_z) + es;
-    inv_r3 = 1.0 / (r * r * r);
-    ix = ix + dx * inv_r3;
-    iy = iy + dy * inv_r3;
-    iz = iz + diff_z * inv_r3;
-    z_ic = -2.0 * n * dd + z_b;
-    diff_z = z_a - z_ic;
-    r = __builtin_sqrt(dxy2 + diff_z * diff_z) + es;
-    inv_r3 = 1.0 / (r * r * r);
-    ix = ix + dx * inv_r3;
-    iy = iy + dy * inv_r3;
-    iz = iz + diff_z * inv_r3;
-  }
-  icx = ix;
-  icy = iy;
-  icz = iz;
-}
 
 // Tip vacuum field (acc_tip_field_E.inc:13-34); cos/sin of atan2(y,x) are
 // taken as x/rho, y/rho.
@@ -109,22 +67,6 @@ __device__ __forceinline__ void tip_image_point64(double x_a, double y_a, double
   x_im = (zi - z0) * x_a / dz;
   y_im = (zi - z0) * y_a / dz;
   dis_a = da;
-}
-
-// Sphere image force (acc_tip_ic_force.inc:17-22), t**1.5 = t*sqrt(t).
-__device__ __forceinline__ void tip_ic_force64(double x_a, double y_a, double z_a, double x_b,
-                                               double y_b, double z_b, double dis_a,
-                                               double x_im, double y_im, double z_im, double R,
-                                               double kt, double& icx, double& icy,
-                                               double& icz) {
-  double ta = (x_b - x_a) * (x_b - x_a) + (y_b - y_a) * (y_b - y_a) + (z_b - z_a) * (z_b - z_a);
-  double tb = (x_b - x_im) * (x_b - x_im) + (y_b - y_im) * (y_b - y_im) +
-              (z_b - z_im) * (z_b - z_im);
-  double tda = ta * __builtin_sqrt(ta);
-  double tdb = tb * __builtin_sqrt(tb);
-  icx = kt * ((x_a - x_b) / tda - (R * (x_im - x_b)) / (dis_a * tdb));
-  icy = kt * ((y_a - y_b) / tda - (R * (y_im - y_b)) / (dis_a * tdb));
-  icz = kt * ((z_a - z_b) / tda - (R * (z_im - z_b)) / (dis_a * tdb));
 }
 
 // ------------------------------------------------------------------------
@@ -431,47 +373,50 @@ __device__ __forceinline__ void field_chunks64(const DevGeom& g, bool act, doubl
   const int t = threadIdx.x;
   double da = 0, xim = 0, yim = 0, zim = 0;
   if (KIND == RD_GEOM_TIP && act && g.ic) tip_image_point64(x1, y1, z1, g.z0, g.R, da, xim, yim, zim);
+  const bool mine =
+      f64_ordinary(x1) && f64_ordinary(y1) && f64_ordinary(z1) &&
+      (KIND == RD_GEOM_PLANAR ? f64_ordinary(g.d)
+                              : f64_ordinary(da) && f64_ordinary(xim) && f64_ordinary(yim) &&
+                                    f64_ordinary(zim));
+  // every target of the wavefront on the cathode: the paired-image form
+  const bool surf = KIND == RD_GEOM_PLANAR && g.ic && __all(!act || z1 == 0.0);
   for (int c = c0; c < c1; ++c) {
     const int jb = c * kChunk;
     __syncthreads();
+    bool ord = !act || mine;
     if (jb + t < n) {
       sx[t] = x[jb + t];
       sy[t] = y[jb + t];
       sz[t] = z[jb + t];
-      sq[t] = q[jb + t];
+      sq[t] = q[jb + t] * g.dfc;
+      ord = ord && f64_ordinary(sx[t]) && f64_ordinary(sy[t]) && f64_ordinary(sz[t]);
     }
-    __syncthreads();
+    const bool fast = __syncthreads_and(ord);
     const int cnt = min(kChunk, n - jb);
     double fxs = 0.0, fys = 0.0, fzs = 0.0;
-    if (act) {
+    auto sweep = [&](auto m, auto on_cathode) {
+      using M = decltype(m);
       for (int jj = 0; jj < cnt; ++jj) {
         double x2 = sx[jj], y2 = sy[jj], z2 = sz[jj];
-        double pre = sq[jj] * g.dfc;
+        double pre = sq[jj];
         double dx = x1 - x2, dy = y1 - y2, dz = z1 - z2;
         double ax, ay, az;
-        if (KIND == RD_GEOM_PLANAR) {
-          double dxy2 = dx * dx + dy * dy;
-          double r = __builtin_sqrt(dxy2 + dz * dz) + g.es;
-          double inv_r3 = 1.0 / (r * r * r);
-          ax = pre * inv_r3 * dx;
-          ay = pre * inv_r3 * dy;
-          az = pre * inv_r3 * dz;
-          if (g.ic) {
-            double icx, icy, icz;
-            ic_planar64(z1, z2, dx, dy, dxy2, g.nic, g.d, g.es, icx, icy, icz);
-            ax = ax + pre * icx;
-            ay = ay + pre * icy;
-            az = az + pre * icz;
-          }
+        if (decltype(on_cathode)::value) {
+          surface_pair64<M, false>(g, pre, dx, dy, z2, ax, ay, az);
+        } else if (KIND == RD_GEOM_PLANAR) {
+          planar_pair64<M>(g, pre, dx, dy, dz, z1, z2, ax, ay, az);
         } else {
-          double r = __builtin_sqrt(dx * dx + dy * dy + dz * dz) + g.es;
-          double inv_r3 = 1.0 / (r * r * r);
-          ax = pre * inv_r3 * dx;
-          ay = pre * inv_r3 * dy;
-          az = pre * inv_r3 * dz;
+          const double r2 = M::lift(dx * dx + dy * dy) + dz * dz;
+          const double rt = M::sqrt(r2);
+          const double r = rt + g.es;
+          const double p0 = pre * M::rcp(r * r * r);
+          ax = p0 * dx;
+          ay = p0 * dy;
+          az = p0 * dz;
           if (g.ic) {
             double icx, icy, icz;
-            tip_ic_force64(x1, y1, z1, x2, y2, z2, da, xim, yim, zim, g.R, g.ktip, icx, icy, icz);
+            tip_ic64<M>(dx, dy, dz, r2, rt, xim - x2, yim - y2, zim - z2, da, g.R, g.ktip, icx,
+                        icy, icz);
             ax = ax + pre * icx;
             ay = ay + pre * icy;
             az = az + pre * icz;
@@ -481,6 +426,14 @@ __device__ __forceinline__ void field_chunks64(const DevGeom& g, bool act, doubl
         fys = fys + ay;
         fzs = fzs + az;
       }
+    };
+    if (act) {
+      if (!fast)
+        sweep(Ieee64{}, std::false_type{});
+      else if (surf)
+        sweep(Fast64{}, std::true_type{});
+      else
+        sweep(Fast64{}, std::false_type{});
       P[0 * S + (size_t)(c - cfirst) * m + p] = fxs;
       P[1 * S + (size_t)(c - cfirst) * m + p] = fys;
       P[2 * S + (size_t)(c - cfirst) * m + p] = fzs;

@@ -153,14 +153,21 @@ __global__ __launch_bounds__(kBlock) void k_accel64(const Ent* tab, int ne, cons
       zi1 = img[4 * (size_t)(base + i) + 3];
     }
   }
+  bool mine = !act || (f64_ordinary(x1) && f64_ordinary(y1) && f64_ordinary(z1));
+  if (KIND == RD_GEOM_PLANAR)
+    mine = mine && f64_ordinary(g.d);
+  else
+    mine = mine && f64_ordinary(d1) && f64_ordinary(xi1) && f64_ordinary(yi1) && f64_ordinary(zi1);
   for (int c = c0; c < c1; ++c) {
     const int jb = c * kChunk;
     __syncthreads();
+    bool ord = mine;
     if (jb + t < n) {
       sx[t] = x[jb + t];
       sy[t] = y[jb + t];
       sz[t] = z[jb + t];
       sq[t] = q[jb + t];
+      ord = ord && f64_ordinary(sx[t]) && f64_ordinary(sy[t]) && f64_ordinary(sz[t]);
       if (tts) ssp[t] = SP[base + jb + t];
       if (KIND == RD_GEOM_TIP && g.ic) {
         const size_t gj = 4 * (size_t)(base + jb + t);
@@ -168,12 +175,15 @@ __global__ __launch_bounds__(kBlock) void k_accel64(const Ent* tab, int ne, cons
         sxi[t] = img[gj + 1];
         syi[t] = img[gj + 2];
         szi[t] = img[gj + 3];
+        ord = ord && f64_ordinary(sd[t]) && f64_ordinary(sxi[t]) && f64_ordinary(syi[t]) &&
+              f64_ordinary(szi[t]);
       }
     }
-    __syncthreads();
+    const bool fast = __syncthreads_and(ord);
     const int cnt = min(kChunk, n - jb);
     double px = 0.0, py = 0.0, pz = 0.0;
-    if (act) {
+    auto sweep = [&](auto m) {
+      using M = decltype(m);
       for (int jj = 0; jj < cnt; ++jj) {
         const int j = jb + jj;
         if (j == i) continue;
@@ -186,39 +196,27 @@ __global__ __launch_bounds__(kBlock) void k_accel64(const Ent* tab, int ne, cons
         double dx = x1 - x2, dy = y1 - y2, dz = z1 - z2;
         double axx, ayy, azz;
         if (KIND == RD_GEOM_PLANAR) {
-          double dxy2 = dx * dx + dy * dy;
-          double r = __builtin_sqrt(dxy2 + dz * dz) + g.es;
-          double inv_r3 = 1.0 / (r * r * r);
-          axx = pre * inv_r3 * dx;
-          ayy = pre * inv_r3 * dy;
-          azz = pre * inv_r3 * dz;
-          if (g.ic) {
-            double za = first ? z1 : z2;
-            double zb = first ? z2 : z1;
-            double icx, icy, icz;
-            ic_planar64(za, zb, dx, dy, dxy2, g.nic, g.d, g.es, icx, icy, icz);
-            axx = axx + pre * icx;
-            ayy = ayy + pre * icy;
-            azz = azz + pre * icz;
-          }
+          planar_pair64<M>(g, pre, dx, dy, dz, first ? z1 : z2, first ? z2 : z1, axx, ayy, azz);
         } else {
-          double r = __builtin_sqrt(dx * dx + dy * dy + dz * dz) + g.es;
-          double inv_r3 = 1.0 / (r * r * r);
-          axx = pre * inv_r3 * dx;
-          ayy = pre * inv_r3 * dy;
-          azz = pre * inv_r3 * dz;
+          const double r2 = M::lift(dx * dx + dy * dy) + dz * dz;
+          const double rt = M::sqrt(r2);
+          const double r = rt + g.es;
+          const double p0 = pre * M::rcp(r * r * r);
+          axx = p0 * dx;
+          ayy = p0 * dy;
+          azz = p0 * dz;
           if (g.ic) {
             double icx, icy, icz;
             if (first) {
-              tip_ic_force64(x1, y1, z1, x2, y2, z2, d1, xi1, yi1, zi1, g.R, g.ktip, icx, icy,
-                             icz);
-              axx = axx + pre * 1.0 * icx;
-              ayy = ayy + pre * 1.0 * icy;
+              tip_ic64<M>(dx, dy, dz, r2, rt, xi1 - x2, yi1 - y2, zi1 - z2, d1, g.R, g.ktip, icx,
+                          icy, icz);
+              axx = axx + pre * icx;
+              ayy = ayy + pre * icy;
             } else {
-              tip_ic_force64(x2, y2, z2, x1, y1, z1, sd[jj], sxi[jj], syi[jj], szi[jj], g.R,
-                             g.ktip, icx, icy, icz);
-              axx = axx + pre * -1.0 * icx;
-              ayy = ayy + pre * -1.0 * icy;
+              tip_ic64<M>(-dx, -dy, -dz, r2, rt, sxi[jj] - x1, syi[jj] - y1, szi[jj] - z1, sd[jj],
+                          g.R, g.ktip, icx, icy, icz);
+              axx = axx + -pre * icx;
+              ayy = ayy + -pre * icy;
             }
             azz = azz + pre * icz;
           }
@@ -227,6 +225,12 @@ __global__ __launch_bounds__(kBlock) void k_accel64(const Ent* tab, int ne, cons
         py = py + ayy;
         pz = pz + azz;
       }
+    };
+    if (act) {
+      if (fast)
+        sweep(Fast64{});
+      else
+        sweep(Ieee64{});
       const size_t S = (size_t)tl.e.pslots * tl.e.n_ub;
       const size_t o = (size_t)(c - tl.e.band0) * tl.e.n_ub + i;
       P[0 * S + o] = px;
