@@ -270,28 +270,24 @@ int rd_slot_step(rd_ctx* ctx, int32_t slot, int32_t* step);
  * (max_slots entries, may be NULL); slots that are not open are left untouched. */
 int rd_pool_step(rd_ctx* ctx, int32_t precision, rd_step_record* records);
 
-/* Launch the Metropolis-Hastings jump loop of each emission step (about
- * 400 kernels at 200 jumps) as one HIP graph (on != 0) or as separate
- * launches (0, the default).  The graph is captured when the loop's launch
- * parameters change and replayed while they do not; results are identical
- * either way.  Library control, no reference counterpart. */
+/* Launch the random numbers and Metropolis-Hastings jumps of each emission
+ * step as one HIP graph (on != 0) or as separate launches (0, the default).
+ * The graph is captured when the launch parameters change and replayed while
+ * they do not; results are identical either way.  Library control, no
+ * reference counterpart. */
 int rd_set_graphs(rd_ctx* ctx, int32_t on);
 
-/* Pool tuning: the mixed-precision jump launches of a step give each
- * workgroup four partial sums of the chain fields once they hold at least
- * min_workgroups workgroups of one partial each (2048 by default; 0: always).
- * The partials keep their size and order, so results are identical for every
- * threshold.  Library control, no reference counterpart. */
+/* Pool tuning of earlier jump launches (min_workgroups >= 0).  The jumps of a
+ * step now take one launch whose workgroups follow the simulations' sizes, so
+ * the value is checked and has no effect; results never depended on it.
+ * Library control, no reference counterpart. */
 int rd_set_jump_pairing(rd_ctx* ctx, int64_t min_workgroups);
 
-/* Mixed-precision jump loops of small simulations (on != 0, the default): in
- * a context made for one simulation (rd_ctx_create), a planar simulation whose
- * chains x electrons per jump are few (by its own sizes) runs all its
- * Metropolis-Hastings jumps in one workgroup of one launch instead of two
- * launches per jump; pools keep the two launches, which serve all their
- * simulations at once.  The chain fields add the same FP32 pair terms in
- * another fixed order, so the fields agree to rounding and the chains take
- * the same sites unless an accept test falls within that rounding.  Library
+/* All Metropolis-Hastings jumps of a step in one launch (on != 0, the
+ * default), or a launch per jump.  In one launch the workgroups of a planar FE
+ * simulation wait, within a bound, for each other's acceptance counts of every
+ * jump; a step in which they cannot all be resident takes a launch per jump by
+ * itself.  Results are identical either way, in both precisions.  Library
  * control, no reference counterpart. */
 int rd_set_solo_jumps(rd_ctx* ctx, int32_t on);
 

@@ -337,6 +337,7 @@ int rd_pool_create(int32_t device, int64_t total, int32_t max_slots, rd_ctx** ou
   e = hipMalloc((void**)&c->d_desc, sizeof(SimDesc) * max_slots);
   if (e == hipSuccess) e = hipMalloc((void**)&c->d_state, sizeof(SimState) * max_slots);
   if (e == hipSuccess) e = hipHostMalloc((void**)&c->h_state, sizeof(SimState) * max_slots);
+  if (e == hipSuccess) e = hipHostMalloc((void**)&c->h_stop, sizeof(int));
   if (e == hipSuccess) e = hipMalloc((void**)&c->d_life, sizeof(int32_t) * 2 * kLife * max_slots);
   if (e != hipSuccess) {
     rd_ctx_destroy(c);
@@ -382,7 +383,7 @@ int rd_ctx_destroy(rd_ctx* c) {
   if (c->jump_exec) hipGraphExecDestroy(c->jump_exec);
   if (c->h_state) hipHostFree(c->h_state);
   if (c->h_tab) hipHostFree(c->h_tab);
-  Buf* bufs[] = {&c->part, &c->pack_hi, &c->pack_lo, &c->pack_far, &c->pack_srf, &c->pts, &c->fld, &c->pts_hi, &c->pts_lo,
+  Buf* bufs[] = {&c->part, &c->pack_hi, &c->pack_lo, &c->pack_far, &c->pack_srx, &c->pack_srz, &c->pts, &c->fld, &c->pts_hi, &c->pts_lo,
                  &c->stage, &c->img64, &c->tab, &c->red, &c->chains, &c->rnd, &c->img_hi, &c->img_lo, &c->cnt,
                  &c->mark, &c->elog, &c->alog, &c->plog, &c->tail_plan, &c->tail_work,
                  &c->tail_box, &c->acc, &c->ctmp};
@@ -390,13 +391,7 @@ int rd_ctx_destroy(rd_ctx* c) {
   if (c->ev0) hipEventDestroy(c->ev0);
   if (c->ev1) hipEventDestroy(c->ev1);
   if (c->ev2) hipEventDestroy(c->ev2);
-  if (c->ev_fork) hipEventDestroy(c->ev_fork);
-  for (int h = 0; h < kJumpStreams - 1; ++h) {
-    if (c->ev_join[h]) hipEventDestroy(c->ev_join[h]);
-    if (c->jstream[h]) hipStreamDestroy(c->jstream[h]);
-  }
-  if (c->ev_solo) hipEventDestroy(c->ev_solo);
-  if (c->sstream) hipStreamDestroy(c->sstream);
+  if (c->h_stop) hipHostFree(c->h_stop);
   if (c->stream) hipStreamDestroy(c->stream);
   delete c;
   return RD_OK;
@@ -1088,7 +1083,6 @@ int rd_set_partial_budget(rd_ctx* c, int64_t bytes) {
 int rd_set_jump_pairing(rd_ctx* c, int64_t min_workgroups) {
   if (!c) return fail(RD_ERR_ARG, "null context");
   if (min_workgroups < 0) return fail(RD_ERR_ARG, "negative workgroup threshold");
-  c->jump_pair_wgs = min_workgroups;
   return RD_OK;
 }
 

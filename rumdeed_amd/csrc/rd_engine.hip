@@ -58,9 +58,11 @@ struct Chains {
   int *ok, *acc, *rej, *pv;  // start found; per-chain counts; proposal valid
 };
 
-static Chains chain_view(rd_ctx* c, int C) {
+static size_t chain_bytes(int C) { return (size_t)C * (10 * sizeof(double) + 4 * sizeof(int)); }
+
+static Chains chain_view(rd_ctx* c, int C, int which) {
   Chains h;
-  double* d = (double*)c->chains.p;
+  double* d = (double*)((char*)c->chains.p + (size_t)which * chain_bytes(C));
   h.cx = d;
   h.cy = d + C;
   h.px = d + 2 * (size_t)C;
@@ -78,7 +80,6 @@ static Chains chain_view(rd_ctx* c, int C) {
   h.pv = ip + 3 * (size_t)C;
   return h;
 }
-static size_t chain_bytes(int C) { return (size_t)C * (10 * sizeof(double) + 4 * sizeof(int)); }
 
 // Work function at a surface point of a planar emitter.
 __device__ __forceinline__ double work_at(const SimDesc& s, const double* wf, double x, double y,
@@ -103,28 +104,50 @@ __device__ __forceinline__ double field_normal(const DevGeom& g, double x, doubl
   return nx * ex + ny * ey + nz * ez;
 }
 
-// MH chain target at a surface point with field component F (< 0).
-__device__ __forceinline__ double chain_target(const SimDesc& s, const double* wf,
-                                               const EmitConsts& ec, double F, double a, double b,
-                                               double xs, double ys, double zs) {
-  if (s.mode == RD_EMIT_PLANAR_FE) {
+// What the MH chain target at a surface point (a, b) takes from the point
+// alone: planar the work function (FE: and its logarithm), tip the surface
+// element's log term.
+struct SiteTerms {
+  double w, lw;
+};
+__device__ __forceinline__ SiteTerms site_terms(const SimDesc& s, const double* wf, double a,
+                                                double b) {
+  SiteTerms t{s.w_tip, 0.0};
+  if (s.mode == RD_EMIT_TIP_FE) {
+    t.lw = 0.5 * rd_log(a * a - s.g.eta_1 * s.g.eta_1);
+  } else {
     int sec;
-    double w = work_at(s, wf, a, b, sec);
-    return fn_supply_log(ec, s.g.ic, F, w);  // Elec_Supply_log
+    t.w = work_at(s, wf, a, b, sec);
+    if (s.mode == RD_EMIT_PLANAR_FE) t.lw = rd_log(t.w);
   }
-  if (s.mode == RD_EMIT_PLANAR_GTF) {
-    int sec;
-    double w = work_at(s, wf, a, b, sec);
-    double J = gtf_current(F, s.T, w);
+  return t;
+}
+
+// MH chain target at a surface point with field component F (< 0).
+template <class M>
+__device__ __forceinline__ double chain_target_by(int mode, int ic, double dt_q0, double F,
+                                                  const SiteTerms& at) {
+  const EmitConsts ec = emit_consts();
+  if (mode == RD_EMIT_PLANAR_FE)  // Elec_Supply_log
+    return fn_supply_log<M>(ec, ic, F, at.w, at.lw);
+  // tip: Tip_fe_target_log(eta_f, xi, pos)
+  double t = fn_t<M>(ic, ec.l_const, F, at.w);
+  double sup = typename M::Div(t * t * at.w)(dt_q0 * ec.a_FN) * (F * F);
+  return rd_log(sup > kTiny ? sup : kTiny) + at.lw;
+}
+// A call, not inlined: in the jump kernels the series' constants would be
+// hoisted out of the jump loop and crowd out the field sums' registers.  All
+// arguments are values, so the call waits for no memory.
+__device__ __attribute__((noinline)) double chain_target(int mode, int ic, double dt_q0, double T,
+                                                         double F, double w, double lw) {
+  const SiteTerms at{w, lw};
+  if (mode == RD_EMIT_PLANAR_GTF) {
+    double J = gtf_current(F, T, at.w);
     return rd_log(J > kTiny ? J : kTiny);
   }
-  // tip: Tip_fe_target_log(eta_f, xi, pos); a = xi
-  double t = fn_t(s.g.ic, ec.l_const, F, s.w_tip);
-  double sup = s.dt_q0 * ec.a_FN / (t * t * s.w_tip) * (F * F);
-  (void)xs;
-  (void)ys;
-  (void)zs;
-  return rd_log(sup > kTiny ? sup : kTiny) + 0.5 * rd_log(a * a - s.g.eta_1 * s.g.eta_1);
+  return f64_ordinary(F) && f64_ordinary(at.w) && at.w != 0.0 && f64_ordinary(dt_q0)
+             ? chain_target_by<Fast64>(mode, ic, dt_q0, F, at)
+             : chain_target_by<Ieee64>(mode, ic, dt_q0, F, at);
 }
 
 // ------------------------------------------------------------------------
@@ -457,7 +480,6 @@ __global__ __launch_bounds__(256) void k_mh_start_check(const Ent* tab, const Si
   __shared__ int red[256];
   const Ent e = tab[blockIdx.x];
   const SimDesc& s = desc[e.slot];
-  const EmitConsts ec = emit_consts();
   int pend = 0;
   for (int k = threadIdx.x; k < e.nch; k += blockDim.x) {
     const int c = e.cbase + k;
@@ -471,7 +493,8 @@ __global__ __launch_bounds__(256) void k_mh_start_check(const Ent* tab, const Si
       ch.cx[c] = ch.px[c];
       ch.cy[c] = ch.py[c];
       ch.F[c] = F;
-      ch.sup[c] = chain_target(s, wf, ec, F, ch.px[c], ch.py[c], ptx[p], pty[p], ptz[p]);
+      const SiteTerms at = site_terms(s, wf, ch.px[c], ch.py[c]);
+      ch.sup[c] = chain_target(s.mode, s.g.ic, s.dt_q0, s.T, F, at.w, at.lw);
       ch.ox[c] = ptx[p];
       ch.oy[c] = pty[p];
       ch.oz[c] = ptz[p];
@@ -511,9 +534,9 @@ __global__ __launch_bounds__(256) void k_mh_start_check(const Ent* tab, const Si
   }
 }
 
-// Gaussian proposal of jump `it` (1-based) for chain k of entry e, with the
-// width MH of the start of the jump and the unit normal pair (u1, u2) of the
-// chain's (step, jump) stream (box_muller_unit).  (a, b) are the chain coordinates
+// Gaussian proposal of jump `it` (1-based) for a chain at (cx, cy) whose site
+// is (ox, oy, oz), with the width MH of the start of the jump and the unit
+// normal pair (u1, u2) of the chain's (step, jump) stream (box_muller_unit).  (a, b) are the chain coordinates
 // (planar x, y; tip xi, phi) and (x, y, z) the surface point whose field the
 // accept step needs.  valid: 1 proposal inside the patch, 0 tip proposal
 // outside it, -1 chain without a start site (the point is its final site and
@@ -523,16 +546,15 @@ struct Proposal {
   int valid;
 };
 
-__device__ __forceinline__ Proposal mh_proposal(const Ent& e, const SimDesc& s, double MH,
-                                                const Chains& ch, int it, int k, double u1,
-                                                double u2) {
+__device__ __forceinline__ Proposal mh_proposal(const SimDesc& s, double MH, int it, int ok,
+                                                double cx, double cy, double ox, double oy,
+                                                double oz, double u1, double u2) {
   Proposal P;
-  const int c = e.cbase + k;
-  if (ch.ok[c] != 1) {
+  if (ok != 1) {
     P.a = P.b = 0.0;
-    P.x = ch.ox[c];
-    P.y = ch.oy[c];
-    P.z = ch.oz[c];
+    P.x = ox;
+    P.y = oy;
+    P.z = oz;
     P.valid = -1;
     return P;
   }
@@ -548,8 +570,8 @@ __device__ __forceinline__ Proposal mh_proposal(const Ent& e, const SimDesc& s, 
       s2 = PI2 * 0.10;
     }
     const double d1 = u1 * s1 + 0.0, d2 = u2 * s2 + 0.0;
-    double nxi = ch.cx[c] + d1;
-    double nphi = fmodulo(ch.cy[c] + d2, PI2);
+    double nxi = cx + d1;
+    double nphi = fmodulo(cy + d2, PI2);
     if (nxi > s.g.max_xi) nxi = 2.0 * s.g.max_xi - nxi;
     if (nxi < 1.0) nxi = 2.0 - nxi;
     P.valid = !((nxi < 1.0) || (nxi > s.g.max_xi));
@@ -558,9 +580,9 @@ __device__ __forceinline__ Proposal mh_proposal(const Ent& e, const SimDesc& s, 
     if (P.valid) {
       tip_xyz(tip_surf(s.g), nxi, s.g.eta_1, nphi, P.x, P.y, P.z);
     } else {
-      P.x = ch.ox[c];
-      P.y = ch.oy[c];
-      P.z = ch.oz[c];
+      P.x = ox;
+      P.y = oy;
+      P.z = oz;
     }
     return P;
   }
@@ -574,7 +596,7 @@ __device__ __forceinline__ Proposal mh_proposal(const Ent& e, const SimDesc& s, 
     sx = s.elx * MH;
     sy = s.ely * MH;
   }
-  double nx = u1 * sx + ch.cx[c], ny = u2 * sy + ch.cy[c];
+  double nx = u1 * sx + cx, ny = u2 * sy + cy;
   if (s.mode == RD_EMIT_PLANAR_FE) {
     // check_limits_metro_rec (src/mod_field_emission_v2.F90:1466-1516): reflect
     double x_max = s.ex0 + s.elx, x_min = s.ex0;
@@ -604,22 +626,6 @@ __device__ __forceinline__ Proposal mh_proposal(const Ent& e, const SimDesc& s, 
   return P;
 }
 
-// Record a proposal: the chain's proposed coordinates and its field point.
-__device__ __forceinline__ void mh_record(const Ent& e, const SimDesc& s, const Chains& ch, int k,
-                                          const Proposal& P, double* __restrict__ ptx,
-                                          double* __restrict__ pty, double* __restrict__ ptz) {
-  const int c = e.cbase + k;
-  const int p = e.pbase + k;
-  if (P.valid >= 0) {
-    if (s.mode == RD_EMIT_TIP_FE) ch.pv[c] = P.valid;
-    ch.px[c] = P.a;
-    ch.py[c] = P.b;
-  }
-  ptx[p] = P.x;
-  pty[p] = P.y;
-  ptz[p] = P.z;
-}
-
 // The planar FE width update of one jump from the batch counts
 // (MH_std_update, src/mod_field_emission_v2.F90:603-612).
 __device__ __forceinline__ double fe_width_after(double mh, int it, int first, int na, int nr) {
@@ -632,188 +638,19 @@ __device__ __forceinline__ double fe_width_after(double mh, int it, int first, i
   }
   return mh;
 }
-__device__ __forceinline__ void fe_width_update(SimState& S, int it, int first, int na, int nr) {
-  S.it_a = na;
-  S.it_r = nr;
-  if ((it > first) && (na + nr > 0)) {
-    S.a_rate = (double)na / (double)(na + nr);
-    S.MH_std = S.MH_std * rd_exp(0.025 * (S.a_rate - 0.35));
-    if (S.MH_std > 0.1250)
-      S.MH_std = 0.1250;
-    else if (S.MH_std < 0.00005)
-      S.MH_std = 0.00005;
-  }
-}
-
-// What the accept step of one chain reads, loaded together ahead of the
-// field sums so that the loads overlap.
-struct AcceptIn {
-  int ok, pv;            // start found; proposal valid (tip)
-  double px, py, sup;    // proposal (chain coordinates), current log target
-  double lr;             // log-uniform of the jump
-  double x, y, z;        // proposal point
-};
-__device__ __forceinline__ AcceptIn accept_inputs(const Ent& e, const SimDesc& s,
-                                                  const Chains& ch, const double* lr,
-                                                  const double* ptx, const double* pty,
-                                                  const double* ptz, int k) {
-  AcceptIn in{};
-  if (k < 0) return in;
-  const int c = e.cbase + k, p = e.pbase + k;
-  in.ok = ch.ok[c];
-  in.pv = s.mode == RD_EMIT_TIP_FE ? ch.pv[c] : 1;
-  in.px = ch.px[c];
-  in.py = ch.py[c];
-  in.sup = ch.sup[c];
-  in.lr = lr[c];
-  in.x = ptx[p];
-  in.y = pty[p];
-  in.z = ptz[p];
-  return in;
-}
-
-// Accept/reject of jump `it` for chain k of entry e (k < 0: no chain), one
-// chain per lane of a block (a multiple of 64 lanes; ra, rr: LDS arrays of
-// blockDim.x / 64 entries for the batch acceptance counts; in: the chain's inputs;
-// (fxk, fyk, fzk): the field at the chain's proposal).  Planar FE: with
-// counts == nullptr the block holds every chain and updates the width
-// itself; otherwise it stores its (accepted, rejected) counts there (see
-// split_width).
-__device__ void mh_accept_block(const Ent& e, const SimDesc& s, SimState* st, const double* wf,
-                                const Chains& ch, int it, const AcceptIn& in, double fxk,
-                                double fyk, double fzk, int* ra, int* rr, int k, int* counts) {
-  const EmitConsts ec = emit_consts();
-  const int first = nint(s.ndim * 0.25);
-  const bool tip = s.mode == RD_EMIT_TIP_FE;
-  const bool counted = (s.mode == RD_EMIT_PLANAR_GTF) || (it > first);
-  int na = 0, nrj = 0;
-  const int c = e.cbase + k;
-  if (k >= 0 && in.ok == 1) {
-    bool acc = false;
-    bool rejected = false;
-    double F = 0.0;
-    if (tip && !in.pv) {
-      rejected = true;
-    } else {
-      F = tip ? field_normal(s.g, in.x, in.y, fxk, fyk, fzk) : fzk;
-      bool bad = (s.mode == RD_EMIT_PLANAR_GTF) ? (F > 0.0) : (F >= 0.0);
-      if (bad) {
-        rejected = true;
-      } else {
-        double sup_new = chain_target(s, wf, ec, F, in.px, in.py, in.x, in.y, in.z);
-        double alpha = sup_new - in.sup;
-        if (sup_new >= in.sup) {
-          acc = true;
-        } else {
-          acc = in.lr <= alpha;
-        }
-        if (acc) {
-          ch.cx[c] = in.px;
-          ch.cy[c] = in.py;
-          ch.sup[c] = sup_new;
-          ch.F[c] = F;
-          ch.ox[c] = in.x;
-          ch.oy[c] = in.y;
-          ch.oz[c] = in.z;
-        } else {
-          rejected = true;
-        }
-      }
-    }
-    if (acc) ++na;
-    if (rejected) ++nrj;
-    if (counted && !tip && s.mode == RD_EMIT_PLANAR_GTF) {
-      if (acc) ch.acc[c] += 1;
-      if (rejected) ch.rej[c] += 1;
-    }
-    if (tip && it > first) {
-      if (acc) ch.acc[c] += 1;
-      if (rejected) ch.rej[c] += 1;
-    }
-  }
-  if (s.mode != RD_EMIT_PLANAR_FE) return;  // per-chain schedules: no batch update
-  // batch counts: one chain per lane, so a ballot per wavefront, then the
-  // wavefront counts (integers: any order gives the same sums)
-  const unsigned long long ba = __ballot(na), br = __ballot(nrj);
-  if ((threadIdx.x & 63) == 0) {
-    ra[threadIdx.x >> 6] = __popcll(ba);
-    rr[threadIdx.x >> 6] = __popcll(br);
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int ta = 0, tr = 0;
-    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) {
-      ta += ra[w];
-      tr += rr[w];
-    }
-    if (counts) {
-      counts[0] = ta;
-      counts[1] = tr;
-    } else {
-      fe_width_update(st[e.slot], it, first, ta, tr);
-    }
-  }
-}
-
-// ------------------------------------------------------------------------
-// One Metropolis-Hastings jump in two launches.
-//
-// k_mh_field64 / k_mh_field32: every workgroup proposes the jump for its own
-// chains (the proposals are counter-based, so every workgroup of a chain
-// computes the same one; the first source segment's workgroup records it)
-// and writes the field partial sums of one source segment.  k_mh_settle: one
-// workgroup per kSettle chains of a simulation adds the partials in a fixed
-// order and runs the accept step for those chains (the planar FE width of
-// simulations whose chains take several workgroups: see split_width).
-// Kernel boundaries are the only synchronisation: no counters, no
-// device-wide fences.
-struct JumpArgs {
-  double *ptx, *pty, *ptz, *fx, *fy, *fz;
-  double* part;
-  const double *X, *Y, *Z, *Q;    // FP64 sources
-  const float4 *HI, *LO;          // packed sources (mixed)
-  const float4* SRF;              // (x, y, z, q z) high parts (mixed, cathode surface)
-  const double *ru1, *ru2, *rlr;  // per jump and chain: unit normals, log-uniform ([it-1][C])
-  int* counts;                    // [jump parity][accept workgroup][accepted, rejected]
-  int C;                          // chains in all
-  int nsettle;                    // accept workgroups of a jump
-};
-
-constexpr int kSettle = 256;  // lanes of a finish-and-accept workgroup
-
-// Workgroups of a simulation's finish-and-accept: one per kSettle chains.
-__host__ __device__ inline int settle_groups(int m) { return max(1, (m + kSettle - 1) / kSettle); }
-
-// Planar FE simulations whose accept step takes several workgroups ("split"):
-// the workgroups of jump j store their batch counts in counts[j & 1]; the
-// width after jump j, f(width after j - 1, counts of j), is formed by every
-// proposal of jump j + 1 from the stored width and those counts, and stored
-// into the state by the first accept workgroup of jump j + 1 (nothing else
-// reads the stored width during that launch, and nothing writes it during a
-// proposal launch).  The width after the last jump is stored by
-// k_mh_width_last.  No launch is added per jump.
-__device__ __forceinline__ bool split_width(const SimDesc& s, const Ent& e) {
-  return s.mode == RD_EMIT_PLANAR_FE && settle_groups(e.nch) > 1;
-}
-__device__ __forceinline__ void split_counts(const Ent& e, const int* counts, int nsettle, int j,
-                                             int& na, int& nr) {
-  const int* cn = counts + (size_t)(j & 1) * 2 * nsettle + 2 * (size_t)e.wg1;
-  na = 0;
-  nr = 0;
-  for (int g = 0; g < settle_groups(e.nch); ++g) {
-    na += cn[2 * g];
-    nr += cn[2 * g + 1];
-  }
-}
-
 // The random numbers of every jump of every chain, drawn before the jumps so
 // that none of them is on a jump's critical path: the unit normal pair of the
 // proposal and the log of the accept uniform, from the chain's (step, jump)
 // streams.
+// It also clears the jumps' acceptance counters.
 __global__ void k_mh_random(const Ent* tab, int ne, const SimDesc* desc, int C,
                             double* __restrict__ u1, double* __restrict__ u2,
-                            double* __restrict__ lr) {
+                            double* __restrict__ lr, unsigned long long* __restrict__ cnt,
+                            long long ncnt) {
   const int cg = blockIdx.x * blockDim.x + threadIdx.x;  // chain over all entries
+  const long long nth = (long long)gridDim.x * gridDim.y * blockDim.x;
+  for (long long k = (long long)blockIdx.y * gridDim.x * blockDim.x + cg; k < ncnt; k += nth)
+    cnt[k] = 0;
   if (cg >= C) return;
   int lo = 0, hi = ne - 1;  // entry holding chain cg (chains are laid out in entry order)
   while (lo < hi) {
@@ -838,516 +675,32 @@ __global__ void k_mh_random(const Ent* tab, int ne, const SimDesc* desc, int C,
       uniform(s.seed, s.stream, (uint64_t)e.step, tag(kTagAccept, (uint64_t)it), (uint64_t)k, 0));
 }
 
-__device__ __forceinline__ Proposal jump_proposal(const Ent& e, const SimDesc& s,
-                                                  const SimState* st, const Chains& ch, int it,
-                                                  int k, const JumpArgs& a) {
-  const size_t o = (size_t)(it - 1) * a.C + e.cbase + k;
-  double mh = st[e.slot].MH_std;
-  if (it >= 2 && split_width(s, e)) {
-    int na, nr;
-    split_counts(e, a.counts, a.nsettle, it - 1, na, nr);
-    mh = fe_width_after(mh, it - 1, nint(s.ndim * 0.25), na, nr);
-  }
-  return mh_proposal(e, s, mh, ch, it, k, a.ru1[o], a.ru2[o]);
-}
+}  // namespace rd
 
-// FP64: one lane per chain, 256 chains per workgroup, sources in 256-source
-// chunks (the canonical order of the field at points: partials per chunk,
-// bit-identical to the oracle).
-template <int KIND>
-__global__ __launch_bounds__(kBlock) void k_mh_field64(const Ent* tab, int ne,
-                                                       const SimDesc* desc, const SimState* st,
-                                                       Chains ch, int it, JumpArgs a) {
-  __shared__ double sx[kChunk], sy[kChunk], sz[kChunk], sq[kChunk];
-  const Ent e = tab[find_entry(tab, ne, blockIdx.x)];
-  const SimDesc& s = desc[e.slot];
-  if (s.g.kind != KIND || it > s.ndim) return;
-  const int m = e.nch;
-  const int gx = (m + kBlock - 1) / kBlock;
-  const int local = blockIdx.x - e.wg0;
-  const int bx = local % gx, by = local / gx;  // chain group, source segment
-  const DevGeom g = s.g;
-  const int n = st[e.slot].n;
-  const int nchunks = (n + kChunk - 1) / kChunk;
-  const int k = bx * kBlock + threadIdx.x;
-  const bool act = k < m;
-  Proposal P{};
-  if (act) {
-    P = jump_proposal(e, s, st, ch, it, k, a);
-    if (by == 0) mh_record(e, s, ch, k, P, a.ptx, a.pty, a.ptz);
-  }
-  const int c0 = by * e.cps;
-  const int c1 = min(nchunks, c0 + e.cps);
-  if (c0 < nchunks)
-    field_chunks64<KIND>(g, act, P.x, P.y, P.z, a.X + e.base, a.Y + e.base, a.Z + e.base,
-                         a.Q + e.base, n, c0, c1, sx, sy, sz, sq, a.part + e.part_off,
-                         (size_t)e.nchunks_ub * m, m, k);
-}
+#include "rd_jumps.h"
 
-// Mixed: 64 chains per workgroup, one per lane; the kJumpWaves wavefronts
-// take an equal slice of every 256-source chunk of the segment each (sources
-// staged in LDS and read as wavefront-wide broadcasts, or read through the
-// scalar cache), and their FP64 lane sums are added in wavefront order.  Many
-// short slices keep the per-wavefront dependency chain short: a lone jump is
-// latency-bound (4 wavefronts per workgroup measured slower in pools too).
-// A workgroup computes PPS consecutive segment partials (the set-up above the
-// source loop is paid once for all of them); the partials are the same for
-// every PPS.  At most 64 VGPRs (eight waves per SIMD: two workgroups per CU).
-constexpr int kJumpTargets = 64;
-constexpr int kJumpWaves = 16;
-constexpr int kJumpSlice = kChunk / kJumpWaves;
-
-// One mixed pair term (general series).
-__device__ __forceinline__ void mixed_pair(const float4 h1, const float4 l1, const float4 h2,
-                                           const float4 l2, int ic, int nic, float two_d,
-                                           double& fx, double& fy, double& fz) {
-  float dx = (h1.x - h2.x) + (l1.x - l2.x);
-  float dy = (h1.y - h2.y) + (l1.y - l2.y);
-  float dxy2 = __builtin_fmaf(dy, dy, dx * dx);
-  float dz = (h1.z - h2.z) + (l1.z - l2.z);
-  float r2 = fmaxf(__builtin_fmaf(dz, dz, dxy2), kR2Min);
-  float ri = rsq(r2);
-  float r3 = ri * ri * ri;
-  float cxy = r3, cz = dz * r3;
-  if (ic) {
-    float wxy, wz;
-    ic_planar32(h1.z + h2.z, l1.w + l2.w, dz, dxy2, nic, two_d, wxy, wz);
-    cxy += wxy;
-    cz += wz;
-  }
-  cxy *= h2.w;
-  cz *= h2.w;
-  fx += (double)(cxy * dx);
-  fy += (double)(cxy * dy);
-  fz += (double)cz;
-}
-
-// Layout of a simulation's chains in the mixed jump field, chosen from its
-// own chain count only: with few chains one wavefront per chain (its lanes
-// stride over the sources), otherwise one lane per chain (the wavefronts
-// take slices of every chunk).
-constexpr int kWaveChains = 32;  // at most this many chains: a wavefront per chain
-__host__ __device__ inline bool jump_by_wave(int m) { return m <= kWaveChains; }
-__host__ __device__ inline int jump_groups32(int m) {
-  return jump_by_wave(m) ? (m + kJumpWaves - 1) / kJumpWaves
-                         : (m + kJumpTargets - 1) / kJumpTargets;
-}
-
-template <int KIND, int PPS>
-__global__ __launch_bounds__(64 * kJumpWaves, 8) void k_mh_field32(const Ent* tab, int ne,
-                                                                const SimDesc* desc,
-                                                                const SimState* st, Chains ch,
-                                                                int it, JumpArgs a) {
-  __shared__ float4 shi[kChunk], slo[kChunk];
-  // the partials' sums alternate between two buffers: the barrier of partial
-  // q + 1 orders every read of partial q - 1's buffer before its reuse
-  __shared__ double red[PPS > 1 ? 2 : 1][3][kJumpWaves][kJumpTargets];
-  __shared__ float4 tgt[4][kJumpTargets];  // wavefront 0's packed targets
-  const Ent e = tab[find_entry(tab, ne, blockIdx.x)];
-  const SimDesc& s = desc[e.slot];
-  if (s.g.kind != KIND || it > s.ndim) return;
-  const int m = e.nch;
-  const bool by_wave = jump_by_wave(m);
-  const int gx = jump_groups32(m);
-  const int local = blockIdx.x - e.wg0;
-  const int bx = local % gx, by = local / gx;  // chain group, workgroup segment
-  const DevGeom& g = s.g;
-  const int n = st[e.slot].n;
-  const int nchunks = (n + kChunk - 1) / kChunk;
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  // the chain of this lane (uniform across a wavefront when by_wave)
-  const int k = by_wave ? bx * kJumpWaves + w : bx * kJumpTargets + lane;
-  const bool act = k < m;
-  float4 h1 = make_float4(0, 0, 0, 0), l1 = make_float4(0, 0, 0, 0);
-  float4 ih1 = make_float4(0, 0, 0, 1), il1 = make_float4(0, 0, 0, 0);
-  // One lane per chain: every wavefront holds the same kJumpTargets chains, so
-  // wavefront 0 forms and packs their proposals and the others read the packed
-  // targets from LDS (by_wave depends on m alone: uniform over the workgroup).
-  if (act && (by_wave || w == 0)) {
-    const Proposal P = jump_proposal(e, s, st, ch, it, k, a);
-    if (by == 0 && (!by_wave || lane == 0)) mh_record(e, s, ch, k, P, a.ptx, a.pty, a.ptz);
-    pack1(P.x, P.y, P.z, 0.0, g.d, h1, l1);
-    if (KIND == RD_GEOM_TIP) pack_image(P.x, P.y, P.z, g.z0, g.R, ih1, il1);
-  }
-  if (!by_wave) {
-    if (w == 0) {
-      tgt[0][lane] = h1;
-      tgt[1][lane] = l1;
-      tgt[2][lane] = ih1;
-      tgt[3][lane] = il1;
-    }
-    __syncthreads();
-    if (w != 0) {
-      h1 = tgt[0][lane];
-      l1 = tgt[1][lane];
-      ih1 = tgt[2][lane];
-      il1 = tgt[3][lane];
-    }
-  }
-  const float4* hi = a.HI + e.base;
-  const float4* lo = a.LO + e.base;
-  const float4* srf = a.SRF + e.base;
-  const int ic = g.ic, nic = g.nic;
-  const float two_d = (float)(2.0 * g.d * 1e9);
-  const float kt = g.ic ? (float)g.ktip : 0.0f;
-  const float Rn = (float)(g.R * 1e9);
-  const bool surf = KIND == RD_GEOM_PLANAR && wave_on_surface(ic, act, h1, l1);
-  // Planar chains on the cathode, one per lane: a wavefront's sources are
-  // the same for all its lanes, so they are read through the scalar cache
-  // into SGPRs (no LDS traffic) in the same order as the staged loop below.
-  // Every wavefront of the workgroup holds the same chains, so the branch is
-  // uniform over the workgroup.
-  const bool scalar_src = KIND == RD_GEOM_PLANAR && !by_wave &&
-                          __syncthreads_or(surf ? 1 : 0) && __syncthreads_and(surf ? 1 : 0);
-  double* part = a.part + e.part_off;
-  const size_t S = (size_t)e.segs * m;
-#pragma unroll
-  for (int q = 0; q < PPS; ++q) {
-    const int sg = by * PPS + q;  // the partial
-    if (sg >= e.segs) break;
-    const int c0 = sg * e.cps;
-    const int c1 = min(nchunks, c0 + e.cps);
-    double fx = 0.0, fy = 0.0, fz = 0.0;
-    if (scalar_src) {
-      const int wu = __builtin_amdgcn_readfirstlane(w);
-      const float dnm = 0.5f * two_d;
-      for (int c = c0; c < c1; ++c) {
-        const int jb = c * kChunk + wu * kJumpSlice;
-        const int je = min(n, jb + kJumpSlice);
-        if (act) {  // fz holds the sum without the factor -2 until the end
-          static_assert(kJumpSlice <= kSurfBlock, "a slice is one FP32 block");
-          auto sweep = [&](auto n0) {
-            constexpr bool N0 = decltype(n0)::value;
-            float acc = 0.f;  // N0: the slice's block sum
-            int j = jb;
-            for (; j + 4 <= je; j += 4) {  // four sources' loads in flight together
-              float4 hh[4], ll[4];
-#pragma unroll
-              for (int u = 0; u < 4; ++u) {
-                hh[u] = load_uniform(N0 ? srf : hi, j + u);
-                ll[u] = load_uniform(lo, j + u);
-              }
-#pragma unroll
-              for (int u = 0; u < 4; ++u) {
-                if (N0)
-                  acc = surface_accq32(h1, l1, hh[u], ll[u], acc);
-                else
-                  fz += (double)surface_term32<false>(h1, l1, hh[u], ll[u], nic, dnm);
-              }
-            }
-            for (; j < je; ++j) {
-              if (N0)
-                acc = surface_accq32(h1, l1, load_uniform(srf, j), load_uniform(lo, j), acc);
-              else
-                fz += (double)surface_term32<false>(h1, l1, load_uniform(hi, j),
-                                                    load_uniform(lo, j), nic, dnm);
-            }
-            if (N0) fz += (double)acc;
-          };
-          if (nic == 0)
-            sweep(std::true_type{});
-          else
-            sweep(std::false_type{});
-        }
-      }
-    }
-    for (int c = scalar_src ? c1 : c0; c < c1; ++c) {
-      const int jb = c * kChunk;
-      __syncthreads();
-      if (t < kChunk && jb + t < n) {
-        shi[t] = hi[jb + t];
-        slo[t] = lo[jb + t];
-      }
-      __syncthreads();
-      const int cnt = min(kChunk, n - jb);
-      // sources of this lane in the chunk: a slice per wavefront, or a stride
-      // of 64 over the chunk per lane
-      const int j0 = by_wave ? lane : w * kJumpSlice;
-      const int j1 = by_wave ? cnt : min(cnt, j0 + kJumpSlice);
-      const int dj = by_wave ? 64 : 1;
-      if (act) {
-        if (KIND == RD_GEOM_PLANAR) {
-          // one loop per form, so that no branch sits in the source loop
-          if (surf) {  // fz holds the sum without the factor -2 until the end
-            const float dnm = 0.5f * two_d;
-            if (nic == 0) {
-              // a lane's sources of the chunk: a slice of kJumpSlice, or at most
-              // kChunk / 64 by wavefront: one FP32 block either way
-              static_assert(kChunk / 64 <= kSurfBlock, "one FP32 block per chunk");
-              float acc = 0.f;
-              for (int jj = j0; jj < j1; jj += dj)
-                acc = surface_acc32(h1, l1, shi[jj], slo[jj], acc);
-              fz += (double)acc;
-            } else
-              for (int jj = j0; jj < j1; jj += dj)
-                fz += (double)surface_term32<false>(h1, l1, shi[jj], slo[jj], nic, dnm);
-          } else if (ic) {
-            for (int jj = j0; jj < j1; jj += dj)
-              mixed_pair(h1, l1, shi[jj], slo[jj], 1, nic, two_d, fx, fy, fz);
-          } else {
-            for (int jj = j0; jj < j1; jj += dj)
-              mixed_pair(h1, l1, shi[jj], slo[jj], 0, 0, two_d, fx, fy, fz);
-          }
-        } else {
-          for (int jj = j0; jj < j1; jj += dj) {
-            float cx, cy, cz;
-            tip_pair32_target(h1, l1, ih1, il1, shi[jj], slo[jj], kt, Rn, cx, cy, cz);
-            fx += (double)cx;
-            fy += (double)cy;
-            fz += (double)cz;
-          }
-        }
-      }
-    }
-    if (surf) fz = -2.0 * fz;
-    const int qb = q & 1;
-    red[qb][0][w][lane] = fx;
-    red[qb][1][w][lane] = fy;
-    red[qb][2][w][lane] = fz;
-    __syncthreads();
-    if (by_wave) {
-      // lane q of wavefront w adds component q over the 64 lanes, in lane order
-      if (lane < 3 && act) {
-        double v = red[qb][lane][w][0];
-        for (int u = 1; u < 64; ++u) v += red[qb][lane][w][u];
-        part[lane * S + (size_t)sg * m + k] = v;
-      }
-    } else if (w < 3 && act) {
-      // wavefront q adds component q over the wavefronts, in wavefront order
-      double v = red[qb][w][0][lane];
-      for (int u = 1; u < kJumpWaves; ++u) v += red[qb][w][u][lane];
-      part[w * S + (size_t)sg * m + k] = v;
-    }
-  }
-}
-
-// Finish and accept: one workgroup per kSettle chains of a simulation.  FP64
-// adds the chunk partials of every chain in chunk order (plus the vacuum
-// field); mixed adds the segment partials in segment order.
-template <int PREC>
-__global__ __launch_bounds__(kSettle) void k_mh_settle(const Ent* tab, int ne,
-                                                       const SimDesc* desc, SimState* st,
-                                                       const double* wf, Chains ch, int it,
-                                                       JumpArgs a) {
-  __shared__ int ra[kSettle / 64], rr[kSettle / 64];
-  const Ent e = tab[find_entry(tab, ne, blockIdx.x, true)];
-  const SimDesc& s = desc[e.slot];
-  if (it > s.ndim) return;
-  const int m = e.nch;
-  const int grp = blockIdx.x - e.wg1;
-  const int k0 = grp * kSettle, k1 = min(m, k0 + kSettle);
-  const int n = st[e.slot].n;
-  const int nchunks = (n + kChunk - 1) / kChunk;
-  const double* part = a.part + e.part_off;
-  // one chain per lane: k1 - k0 <= kSettle
-  const int k = k0 + (int)threadIdx.x < k1 ? k0 + (int)threadIdx.x : -1;
-  const AcceptIn in =
-      accept_inputs(e, s, ch, a.rlr + (size_t)(it - 1) * a.C, a.ptx, a.pty, a.ptz, k);
-  double fxk = 0.0, fyk = 0.0, fzk = 0.0;
-  if (k >= 0) {
-    const int p = e.pbase + k;
-    if (PREC == RD_PREC_FP64) {
-      field_finish64(s.g, part, (size_t)e.nchunks_ub * m, m, k, nchunks, in.x, in.y, in.z, fxk,
-                     fyk, fzk);
-    } else {
-      const int segs = nchunks == 0 ? 1 : min(e.segs, (nchunks + e.cps - 1) / e.cps);
-      if (s.g.kind == RD_GEOM_TIP)
-        field_finish32_tip(s.g, part, (size_t)e.segs * m, m, k, segs, in.x, in.y, in.z, fxk,
-                           fyk, fzk);
-      else
-        field_finish32(s.g, part, (size_t)e.segs * m, m, k, segs, fxk, fyk, fzk);
-    }
-    a.fx[p] = fxk;
-    a.fy[p] = fyk;
-    a.fz[p] = fzk;
-  }
-  const bool split = split_width(s, e);
-  if (split && grp == 0 && threadIdx.x == 0 && it >= 2) {
-    // store the width after the previous jump (its proposals formed it too)
-    int na, nr;
-    split_counts(e, a.counts, a.nsettle, it - 1, na, nr);
-    fe_width_update(st[e.slot], it - 1, nint(s.ndim * 0.25), na, nr);
-  }
-  mh_accept_block(e, s, st, wf, ch, it, in, fxk, fyk, fzk, ra, rr, k,
-                  split ? a.counts + (size_t)(it & 1) * 2 * a.nsettle + 2 * (size_t)blockIdx.x
-                        : nullptr);
-}
-
-// Split planar FE simulations (split_width): the width after their last jump.
-__global__ void k_mh_width_last(const Ent* tab, const SimDesc* desc, SimState* st,
-                                const int* __restrict__ counts, int nsettle) {
-  const Ent e = tab[blockIdx.x];
-  const SimDesc& s = desc[e.slot];
-  if (threadIdx.x != 0 || s.ndim < 1 || !split_width(s, e)) return;
-  int na, nr;
-  split_counts(e, counts, nsettle, s.ndim, na, nr);
-  fe_width_update(st[e.slot], s.ndim, nint(s.ndim * 0.25), na, nr);
-}
-
-// ------------------------------------------------------------------------
-// Every jump of a small planar simulation in one workgroup (mixed precision).
-//
-// A lone small simulation (a few chains over a few hundred electrons) spends
-// two launches per jump on a few microseconds of pair terms: the launches,
-// not the terms, set its step time.  Here one workgroup of kSoloThreads lanes
-// takes all jumps 1..ndim of one simulation, with barriers between the
-// phases of a jump:
-//   1. lane k < m proposes for chain k (jump_proposal: the same random
-//      numbers, width and reflection as the two-launch path), records the
-//      proposal and packs its point into LDS;
-//   2. the lanes form mp columns (mp: the power of two >= m) and
-//      kSoloThreads / mp rows, lane t taking chain t % mp and the sources
-//      j = row, row + rows, ... of each staged block, with the FP32 pair terms
-//      of the two-launch path added in FP64 (on the cathode with N_ic_max = 0,
-//      FP32 blocks of at most kSurfBlock of the lane's own terms); the rows'
-//      sums are then added pairwise in a fixed tree;
-//   3. lane k < m forms the field (field_from_sums32) and runs the accept
-//      step with the batch width update of mh_accept_block.
-// The sources do not move during the jumps: up to kSoloStage of them stay in
-// LDS for all jumps, more are staged per jump.  Which simulations run here
-// depends on the kind of context (a lone simulation) and on the simulation's
-// own chain count, electron count and image series (solo_jumps).  Tip
-// simulations start hundreds of chains or more and keep the two-launch path.
-constexpr int kSoloThreads = 1024;
-constexpr int kSoloStage = 2048;     // sources held in LDS
-constexpr double kSoloWork = 2.0e6;  // most estimated VALU work per jump, in lane-ops
-
-// Estimated lane-ops of one jump's pair terms: chains x electrons x the
-// instructions of one term (surface form with N_ic_max = 0: 12, each image
-// partner pair about 10 more; without images: 25).  At 64 lane-ops per cycle
-// on one CU, kSoloWork is about 13 us per jump, against about 15 us for the
-// two launches of a lone simulation.
-__host__ __device__ inline double solo_work(int ic, int nic, int m, int n) {
-  const double per = ic ? 12.0 + 10.0 * nic : 25.0;
-  return per * (double)m * (double)(n > 1 ? n : 1);
-}
-__host__ __device__ inline bool solo_jumps(int kind, int ic, int nic, int m, int n) {
-  return kind == RD_GEOM_PLANAR && m >= 1 && m <= kSettle && solo_work(ic, nic, m, n) <= kSoloWork;
-}
-
-__global__ __launch_bounds__(kSoloThreads) void k_mh_solo32(const Ent* tab, const SimDesc* desc,
-                                                            SimState* st, const double* wf,
-                                                            Chains ch, JumpArgs a) {
-  __shared__ float4 shi[kSoloStage], slo[kSoloStage];
-  __shared__ float4 tgt[2][kSettle];
-  __shared__ double red[3][kSoloThreads];
-  __shared__ int ra[kSoloThreads / 64], rr[kSoloThreads / 64];
-  const Ent e = tab[blockIdx.x];
-  const SimDesc& s = desc[e.slot];
-  const DevGeom& g = s.g;
-  const int m = e.nch;
-  const int n = st[e.slot].n;
-  const int t = threadIdx.x;
-  int lmp = 0;
-  while ((1 << lmp) < m) ++lmp;
-  const int mp = 1 << lmp, rows = kSoloThreads >> lmp;
-  const int col = t & (mp - 1), row = t >> lmp;
-  const bool act = col < m;
-  const float4* hi = a.HI + e.base;
-  const float4* lo = a.LO + e.base;
-  const int ic = g.ic, nic = g.nic;
-  const float two_d = (float)(2.0 * g.d * 1e9);
-  const float dnm = 0.5f * two_d;
-  const bool resident = n <= kSoloStage;
-  if (resident) {
-    for (int j = t; j < n; j += kSoloThreads) {
-      shi[j] = hi[j];
-      slo[j] = lo[j];
-    }
-  }
-  for (int it = 1; it <= s.ndim; ++it) {
-    // 1. proposals
-    AcceptIn in{};
-    if (t < m) {
-      const Proposal P = jump_proposal(e, s, st, ch, it, t, a);
-      mh_record(e, s, ch, t, P, a.ptx, a.pty, a.ptz);
-      float4 h1, l1;
-      pack1(P.x, P.y, P.z, 0.0, g.d, h1, l1);
-      tgt[0][t] = h1;
-      tgt[1][t] = l1;
-      in = accept_inputs(e, s, ch, a.rlr + (size_t)(it - 1) * a.C, a.ptx, a.pty, a.ptz, t);
-    }
-    __syncthreads();
-    // 2. pair terms
-    float4 h1 = make_float4(0, 0, 0, 0), l1 = make_float4(0, 0, 0, 0);
-    if (act) {
-      h1 = tgt[0][col];
-      l1 = tgt[1][col];
-    }
-    const bool surf = wave_on_surface(ic, act, h1, l1);
-    double fx = 0.0, fy = 0.0, fz = 0.0;
-    for (int jb = 0; jb < n; jb += kSoloStage) {
-      if (!resident) {
-        __syncthreads();
-        for (int j = t; j < kSoloStage && jb + j < n; j += kSoloThreads) {
-          shi[j] = hi[jb + j];
-          slo[j] = lo[jb + j];
-        }
-        __syncthreads();
-      }
-      const int cnt = min(kSoloStage, n - jb);
-      if (!act) continue;
-      if (surf) {  // fz holds the sum without the factor -2 until the end
-        if (nic == 0) {
-          for (int j0 = row; j0 < cnt; j0 += rows * kSurfBlock) {
-            const int je = min(cnt, j0 + rows * kSurfBlock);
-            float acc = 0.f;
-            for (int jj = j0; jj < je; jj += rows)
-              acc = surface_acc32(h1, l1, shi[jj], slo[jj], acc);
-            fz += (double)acc;
-          }
-        } else {
-          for (int jj = row; jj < cnt; jj += rows)
-            fz += (double)surface_term32<false>(h1, l1, shi[jj], slo[jj], nic, dnm);
-        }
-      } else if (ic) {
-        for (int jj = row; jj < cnt; jj += rows)
-          mixed_pair(h1, l1, shi[jj], slo[jj], 1, nic, two_d, fx, fy, fz);
-      } else {
-        for (int jj = row; jj < cnt; jj += rows)
-          mixed_pair(h1, l1, shi[jj], slo[jj], 0, 0, two_d, fx, fy, fz);
-      }
-    }
-    if (surf) fz = -2.0 * fz;
-    red[0][t] = fx;
-    red[1][t] = fy;
-    red[2][t] = fz;
-    // rows added pairwise: row r takes row r + h for h = rows/2, rows/4, ..., 1
-    for (int h = rows >> 1; h > 0; h >>= 1) {
-      __syncthreads();
-      if (row < h) {
-        const int u = t + (h << lmp);
-        red[0][t] += red[0][u];
-        red[1][t] += red[1][u];
-        red[2][t] += red[2][u];
-      }
-    }
-    __syncthreads();
-    // 3. field and accept (lane t < m holds chain t: row 0)
-    double fxk = 0.0, fyk = 0.0, fzk = 0.0;
-    if (t < m) {
-      field_from_sums32(g, red[0][t], red[1][t], red[2][t], fxk, fyk, fzk);
-      const int p = e.pbase + t;
-      a.fx[p] = fxk;
-      a.fy[p] = fyk;
-      a.fz[p] = fzk;
-    }
-    mh_accept_block(e, s, st, wf, ch, it, in, fxk, fyk, fzk, ra, rr, t < m ? t : -1, nullptr);
-    // the width and the chains' states are read by the next jump's proposals
-    __syncthreads();
-  }
-}
+namespace rd {
 
 // Per-chain width updates (thermal-field, tip) in chain order and the escape
 // quantity of every chain.
 __global__ __launch_bounds__(256) void k_mh_finish(const Ent* tab, const SimDesc* desc,
-                                                   SimState* st, const double* wf, Chains ch) {
+                                                   SimState* st, const double* wf, Chains ch,
+                                                   const double* __restrict__ width) {
   constexpr int kTile = 1024;
   __shared__ double fac[kTile], rate[kTile];
   const Ent e = tab[blockIdx.x];
   const SimDesc& s = desc[e.slot];
   const EmitConsts ec = emit_consts();
-  if (s.mode != RD_EMIT_PLANAR_FE) {
+  if (s.mode == RD_EMIT_PLANAR_FE) {
+    if (threadIdx.x == 0) {  // the width and counts after the last jump (JumpWidth::last)
+      const double* v = width + (size_t)kWidthSlots * e.acc_off;
+      SimState& S = st[e.slot];
+      S.MH_std = v[4];
+      S.a_rate = v[5];
+      S.it_a = (int)v[6];
+      S.it_r = (int)v[7];
+    }
+  } else {
     // The width factor of every chain depends on its own counts only, so the
     // exponentials are formed in parallel; the products and clamps, which
     // chain the chains together, follow in chain order in one lane.
@@ -2436,304 +1789,247 @@ static int reset_counters(rd_ctx* c, const std::vector<Ent>& ents) {
   return RD_OK;
 }
 
-// The Metropolis-Hastings jumps 1..maxndim of the chain entries `in` (C
-// chains in all: the stride of the point and field arrays): per jump, one
-// field launch per geometry present, then the finish-and-accept launch; after
-// the last jump, the width of split planar FE simulations (split_width).
-//
-// In a pool the simulations are dealt into up to kJumpStreams parts of about
-// equal work, each with its own launch table on its own stream.  Nothing of
-// one part depends on another during the jumps, so the latency-bound accept
-// step of one part overlaps the field launches of the others.  Every launch
-// still sees each simulation exactly as before, so results do not change.
+// Forms of the jump kernels: FP64; mixed, a lone simulation of few or many
+// particles, a pool (JumpForm).
+enum JumpKind { kJumpFp64, kJumpLone, kJumpMany, kJumpPool, kJumpKinds };
+static_assert(kJumpKinds == sizeof(rd_ctx::jump_room) / sizeof(int), "a room per form");
+
+// Instructions of one chain's pair terms per SIMD and jump over n particles.
+static double jump_work(const DevGeom& g, JumpKind kind, int n) {
+  const int waves = kind == kJumpMany ? 16 : 4;  // slices: the wavefronts a chain is spread over
+  const double rounds = std::max(1, (n + 64 * waves - 1) / (64 * waves)) * (waves / 4);
+  if (g.kind == RD_GEOM_TIP) return rounds * (kind == kJumpFp64 ? 160.0 : 50.0);
+  if (kind == kJumpFp64) return rounds * 40.0 * (g.ic ? 1 + 2 * g.nic : 1);
+  return rounds * (g.ic ? 12.0 + 20.0 * g.nic : 25.0);
+}
+
+// Chains a workgroup of the jump kernels takes for an entry of m chains: about
+// `target` instructions per SIMD and jump, in a number that the wavefronts can
+// share evenly, at least two where each particle is read from memory in every
+// jump, and at most max_groups workgroups.
+static int jump_chains(JumpKind kind, double work, int m, double target, int max_groups) {
+  static const int lone[] = {1, 2, 4, 8, 12, 16, 24, 32, 48, 64};
+  static const int pool[] = {2, 4, 8, 16, 24, 32, 48, 64};
+  static const int dbl[] = {4, 8, 12, 16, 24, 32, 48, 64};
+  const int* cand = kind == kJumpFp64 ? dbl : (kind == kJumpPool ? pool : lone);
+  const int nc = kind == kJumpLone || kind == kJumpMany ? 10 : 8;
+  int want = (int)(target / work);
+  if (kind == kJumpMany) want = std::max(want, 2);
+  const int least = (m + max_groups - 1) / max_groups;
+  int cw = cand[0];
+  for (int k = 0; k < nc; ++k)
+    if (cand[k] <= want || cw < least) cw = cand[k];
+  return cw;
+}
+
+// The Metropolis-Hastings jumps 1..maxndim of the chain entries `in` (C chains
+// in all) from the chain states V into R: one launch per geometry present
+// (rd_jumps.h).  *width receives the entries' final widths.
 static int run_jumps(rd_ctx* c, const std::vector<Ent>& in, int C, int precision,
-                     const Chains& V, int maxndim) {
+                     const Chains& V, const Chains& R, int maxndim, double** width) {
   const bool fp64 = precision == RD_PREC_FP64;
-  const int per = fp64 ? kBlock : kJumpTargets;  // chains per workgroup
-  std::vector<Ent> all;
-  for (const Ent& e : in)
-    if (e.nch > 0) all.push_back(e);
-  if (all.empty()) return RD_OK;
+  std::vector<Ent> ents = in;
   JumpArgs a;
   std::memset(&a, 0, sizeof(a));  // its bytes form part of the graph key
-  double* ptx = (double*)c->pts.p;
-  double* f = (double*)c->fld.p;
-  a.ptx = ptx;
-  a.pty = ptx + C;
-  a.ptz = ptx + 2 * (size_t)C;
-  a.fx = f;
-  a.fy = f + C;
-  a.fz = f + 2 * (size_t)C;
   a.X = c->x;
   a.Y = c->y;
   a.Z = c->z;
   a.Q = c->q;
   int r = RD_OK;
   if (!fp64) {
-    r = launch_pack(c, all, true);
+    r = launch_pack(c, ents, true);
     if (r) return r;
-  }
-  // A lone small simulation takes all its jumps in one workgroup
-  // (k_mh_solo32); the others, and every simulation of a pool, the two
-  // launches per jump below.  In a pool those launches serve every
-  // simulation at once, and a solo workgroup would hold a CU (and most of its
-  // LDS) for the whole jump phase: measured 7% fewer simulations per hour on
-  // the serving stream.
-  std::vector<Ent> ents, solo;
-  const bool lone = c->nslots_max == 1;
-  for (const Ent& e : all) {
-    const DevGeom& g = c->slots[e.slot].desc.g;
-    if (!fp64 && lone && c->solo_jumps && solo_jumps(g.kind, g.ic, g.nic, e.nch, e.n_ub))
-      solo.push_back(e);
-    else
-      ents.push_back(e);
   }
   a.HI = (const float4*)c->pack_hi.p;
   a.LO = (const float4*)c->pack_lo.p;
-  a.SRF = (const float4*)c->pack_srf.p;
-
-  // parts: consecutive runs of the table of about equal work
-  struct Half {
-    std::vector<Ent> ents;
-    int nwg = 0, nsettle = 0;
-    bool any_split = false, any_planar = false, any_tip = false;
-    Ent* dt = nullptr;
-    JumpArgs a;
-    hipStream_t stream = nullptr;
-  };
-  const int nparts = (c->nslots_max > 1 && !c->graphs)
-                         ? std::min<int>(kJumpStreams, (int)ents.size())
-                         : 1;
-  Half hv[kJumpStreams];
-  int nh = 0;
-  {
-    double total = 0.0, acc = 0.0;
-    for (const Ent& e : ents) total += (double)e.nch * std::max(e.n_ub, 1);
-    size_t k = 0;
-    for (int h = 0; h < nparts; ++h) {
-      // entries until this part reaches its share; leave one per later part
-      const size_t keep = (size_t)(nparts - 1 - h);
-      while (k < ents.size() - keep) {
-        hv[h].ents.push_back(ents[k]);
-        acc += (double)ents[k].nch * std::max(ents[k].n_ub, 1);
-        ++k;
-        if (h + 1 < nparts && acc >= total * (h + 1) / nparts) break;
-      }
-      if (!hv[h].ents.empty()) nh = h + 1;
+  a.SRX = (const double2*)c->pack_srx.p;
+  a.SRZ = (const float2*)c->pack_srz.p;
+  bool any_planar = false, any_tip = false;
+  for (const Ent& e : ents)
+    (c->slots[e.slot].desc.g.kind == RD_GEOM_TIP ? any_tip : any_planar) = true;
+  const JumpKind kind = fp64                  ? kJumpFp64
+                        : c->nslots_max > 1   ? kJumpPool
+                        : ents[0].n_ub < kJumpLarge ? kJumpLone
+                                                    : kJumpMany;
+  using Kernel = void (*)(const Ent*, int, const SimDesc*, const SimState*, const double*, Chains,
+                          Chains, JumpArgs);
+  static const struct {
+    Kernel planar, tip;
+    int threads;
+  } forms[kJumpKinds] = {
+      {k_mh_jumps64<RD_GEOM_PLANAR>, k_mh_jumps64<RD_GEOM_TIP>, kJump64Threads},
+      {k_mh_jumps32<RD_GEOM_PLANAR, LoneForm>, k_mh_jumps32<RD_GEOM_TIP, LoneForm>,
+       64 * LoneForm::kWaves},
+      {k_mh_jumps32<RD_GEOM_PLANAR, LargeForm>, k_mh_jumps32<RD_GEOM_TIP, LargeForm>,
+       64 * LargeForm::kWaves},
+      {k_mh_jumps32<RD_GEOM_PLANAR, PoolForm>, k_mh_jumps32<RD_GEOM_TIP, PoolForm>,
+       64 * PoolForm::kWaves}};
+  const auto& form = forms[kind];
+  // workgroups that can be resident at once
+  int& room = c->jump_room[kind];
+  if (room == 0) {
+    int cus = 0, p = 0, q = 0;
+    RD_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device));
+    RD_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&p, form.planar, form.threads, 0));
+    RD_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&q, form.tip, form.threads, 0));
+    room = std::max(1, cus * std::min(p, q));
+  }
+  // The largest first, so that their workgroups start together and the small
+  // simulations fill up behind them.
+  std::stable_sort(ents.begin(), ents.end(), [](const Ent& x, const Ent& y) {
+    return (double)x.nch * std::max(x.n_ub, 1) > (double)y.nch * std::max(y.n_ub, 1);
+  });
+  // Chains per workgroup: from the smallest target that lets every workgroup be
+  // resident at once.
+  bool spin = true;
+  int nwg = 0;
+  long long words = 0;
+  double target = kJumpTarget;
+  for (int pass = 0; pass < 24; ++pass) {
+    nwg = 0;
+    words = 0;
+    spin = c->solo_jumps;
+    for (Ent& e : ents) {
+      const SimDesc& d = c->slots[e.slot].desc;
+      const bool fe = d.mode == RD_EMIT_PLANAR_FE;
+      const int most = fe ? std::max(1, room - room / 4) : room;
+      const double work = jump_work(d.g, kind, e.n_ub);
+      e.cps = jump_chains(kind, work, e.nch, target, most);
+      e.segs = (e.nch + e.cps - 1) / e.cps;
+      if (fe && e.segs > most) spin = false;  // too many chains to be resident together
+      e.wg0 = nwg;
+      nwg += e.segs;
+      e.pslots = jump_words(e.segs);
+      e.part_off = words;
+      words += (long long)e.pslots * d.ndim;
+    }
+    if (nwg <= room) break;
+    target *= 1.2;
+  }
+  if (!spin) {
+    // a launch per jump: nothing has to be resident, so small workgroups, which
+    // even out over the CUs
+    nwg = 0;
+    words = 0;
+    for (Ent& e : ents) {
+      e.cps = std::min(e.cps, kJumpApart);
+      e.segs = (e.nch + e.cps - 1) / e.cps;
+      e.wg0 = nwg;
+      nwg += e.segs;
+      e.pslots = jump_words(e.segs);
+      e.part_off = words;
+      words += (long long)e.pslots * c->slots[e.slot].desc.ndim;
     }
   }
-  // A context made for one simulation spreads each jump's sums over up to
-  // kWantJump workgroups (latency); in a pool, whose launches serve many
-  // simulations, every mixed partial covers at least kPoolJumpChunks chunks
-  // of sources (throughput; the FP64 kernel, bound by its arithmetic, keeps
-  // the finer split).  Either way the split depends on the simulation's own
-  // size and the kind of context only.
-  const int min_cps = (c->nslots_max > 1 && !fp64) ? kPoolJumpChunks : 1;
-  long long off = 0;
-  int nsettle_all = 0;
-  for (int h = 0; h < nh; ++h) {
-    Half& H = hv[h];
-    for (Ent& e : H.ents) {
-      if (c->slots[e.slot].desc.g.kind == RD_GEOM_TIP)
-        H.any_tip = true;
-      else
-        H.any_planar = true;
-      e.wg1 = H.nsettle;
-      H.nsettle += settle_groups(e.nch);
-      if (settle_groups(e.nch) > 1 && c->slots[e.slot].desc.mode == RD_EMIT_PLANAR_FE)
-        H.any_split = true;
-      const int nch = (e.n_ub + kChunk - 1) / kChunk;
-      const int gx = fp64 ? (e.nch + per - 1) / per : jump_groups32(e.nch);
-      e.nchunks_ub = nch;
-      segment(nch, seg_limit(gx, kWantJump), e.segs, e.cps);
-      if (e.cps < min_cps) {
-        e.cps = std::min(min_cps, std::max(nch, 1));
-        e.segs = (std::max(nch, 1) + e.cps - 1) / e.cps;
-      }
-      e.part_off = off;
-      off += 3LL * (fp64 ? std::max(nch, 1) : e.segs) * e.nch;
-    }
-    nsettle_all += H.nsettle;
-  }
-  // Partials per mixed workgroup: one, or kJumpPairs when the launches are
-  // large enough to keep every CU busy with that many times fewer workgroups
-  // (each then pays the proposal and set-up once for all its sources).  The
-  // partials themselves keep their size, so the sums do not depend on this
-  // choice.
-  int pps = 1;
-  if (!fp64 && c->nslots_max > 1) {
-    long long wg_all = 0;
-    for (int h = 0; h < nh; ++h)
-      for (const Ent& e : hv[h].ents) wg_all += (long long)jump_groups32(e.nch) * e.segs;
-    if (wg_all >= c->jump_pair_wgs) pps = kJumpPairs;
-  }
-  for (int h = 0; h < nh; ++h) {
-    Half& H = hv[h];
-    for (Ent& e : H.ents) {
-      const int gx = fp64 ? (e.nch + per - 1) / per : jump_groups32(e.nch);
-      e.wg0 = H.nwg;
-      H.nwg += gx * ((e.segs + pps - 1) / pps);
-    }
-  }
-  r = ensure(c, c->part, sizeof(double) * (size_t)std::max(off, 1LL));
-  if (r) return r;
+  a.C = C;
+  a.fits = nwg <= room;
   const size_t nr = (size_t)maxndim * C;
   r = ensure(c, c->rnd, sizeof(double) * 3 * nr);
   if (r) return r;
-  r = ensure(c, c->cnt, sizeof(int) * 4 * (size_t)std::max(nsettle_all, 1));
+  const size_t wbytes = sizeof(double) * kWidthSlots * ents.size();
+  r = ensure(c, c->cnt, sizeof(unsigned long long) * (size_t)(words + 1) + wbytes);
   if (r) return r;
-  if (nh > 1 && !c->jstream[0]) {
-    for (int h = 0; h < kJumpStreams - 1; ++h) {
-      RD_HIP(hipStreamCreateWithFlags(&c->jstream[h], hipStreamNonBlocking));
-      RD_HIP(hipEventCreateWithFlags(&c->ev_join[h], hipEventDisableTiming));
-    }
-  }
-  // the solo launch overlaps the two-launch jumps on a stream of its own
-  // (one stream when the loop is captured)
-  const bool solo_own = !solo.empty() && nh > 0 && !c->graphs;
-  if (solo_own && !c->sstream) {
-    RD_HIP(hipStreamCreateWithFlags(&c->sstream, hipStreamNonBlocking));
-    RD_HIP(hipEventCreateWithFlags(&c->ev_solo, hipEventDisableTiming));
-  }
-  if ((nh > 1 || solo_own) && !c->ev_fork)
-    RD_HIP(hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming));
   double* rb = (double*)c->rnd.p;
   a.ru1 = rb;
   a.ru2 = rb + nr;
   a.rlr = rb + 2 * nr;
-  a.C = C;
-  a.part = (double*)c->part.p;
-  Ent* dall = nullptr;  // every entry, for the random numbers of all chains
-  Ent* dsolo = nullptr;
-  if (nh > 1 || !solo.empty()) {
-    r = upload_tab(c, all, &dall);
-    if (r) return r;
-  }
-  if (!solo.empty()) {
-    r = upload_tab(c, solo, &dsolo);
-    if (r) return r;
-  }
-  int cnt_off = 0;
-  for (int h = 0; h < nh; ++h) {
-    Half& H = hv[h];
-    r = upload_tab(c, H.ents, &H.dt);
-    if (r) return r;
-    H.a = a;
-    H.a.counts = (int*)c->cnt.p + cnt_off;
-    H.a.nsettle = H.nsettle;
-    cnt_off += 4 * H.nsettle;
-    H.stream = h == 0 ? c->stream : c->jstream[h - 1];
-  }
-  if (nh == 1 && solo.empty()) dall = hv[0].dt;
-  const int ne_all = (int)all.size();
-  // Everything the launches below depend on besides device data.  With graphs
-  // on, an unchanged key replays the captured loop (the kernels read the
-  // launch table and the chains from device memory, so new contents under
-  // the same pointers are picked up).  Graphs use one stream (nh == 1).
-  const Half& G = hv[0];
-  std::vector<unsigned char> key;
-  auto put = [&key](const void* v, size_t bytes) {
-    const unsigned char* b = (const unsigned char*)v;
-    key.insert(key.end(), b, b + bytes);
+  a.cnt = (unsigned long long*)c->cnt.p;
+  a.stop = (int*)(a.cnt + words);
+  a.width = (double*)(a.cnt + words + 1);
+  *width = a.width;
+  Ent *dall = nullptr, *dt = nullptr;
+  r = upload_tab(c, in, &dall);
+  if (!r) r = upload_tab(c, ents, &dt);
+  if (r) return r;
+  const int ne = (int)ents.size();
+  auto random = [&]() {
+    k_mh_random<<<dim3((C + 255) / 256, maxndim), 256, 0, c->stream>>>(
+        dall, ne, c->d_desc, C, rb, rb + nr, rb + 2 * nr, a.cnt, words + 1);
   };
-  const int ints[] = {(int)G.ents.size(), G.nwg, G.nsettle, (int)G.any_split,
-                      (int)G.any_planar, (int)G.any_tip, (int)fp64, maxndim, C,
-                      (int)solo.size(), nh};
-  const void* ptrs[] = {G.dt, dall, dsolo, c->d_desc, c->d_state, c->d_wf};
-  put(ints, sizeof(ints));
-  put(ptrs, sizeof(ptrs));
-  put(&G.a, sizeof(G.a));
-  put(&V, sizeof(V));
-  if (c->graphs && c->jump_exec && key == c->jump_key) {
-    RD_HIP(hipGraphLaunch(c->jump_exec, c->stream));
+  auto jumps = [&](const Chains& from, int it0, int it1, bool sp) {
+    a.it0 = it0;
+    a.it1 = it1;
+    a.spin = sp;
+    if (any_planar)
+      form.planar<<<nwg, form.threads, 0, c->stream>>>(dt, ne, c->d_desc, c->d_state, c->d_wf,
+                                                       from, R, a);
+    if (any_tip)
+      form.tip<<<nwg, form.threads, 0, c->stream>>>(dt, ne, c->d_desc, c->d_state, c->d_wf, from,
+                                                    R, a);
+  };
+  auto one_by_one = [&]() {
+    for (int it = 1; it <= maxndim + 1; ++it) jumps(it == 1 ? V : R, it, it + 1, false);
+  };
+  if (!spin) {
+    random();
+    one_by_one();
+    RD_HIP(hipGetLastError());
     return RD_OK;
   }
   if (c->graphs) {
-    // the stream was synchronised after the previous launch of the old graph
-    if (c->jump_exec) RD_HIP(hipGraphExecDestroy(c->jump_exec));
-    c->jump_exec = nullptr;
-    c->jump_key.clear();
-    RD_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-  }
-  k_mh_random<<<dim3((C + 255) / 256, maxndim), 256, 0, c->stream>>>(dall, ne_all, c->d_desc, C,
-                                                                       rb, rb + nr, rb + 2 * nr);
-  if (nh > 1 || solo_own) {
-    RD_HIP(hipEventRecord(c->ev_fork, c->stream));
-    for (int h = 1; h < nh; ++h) RD_HIP(hipStreamWaitEvent(hv[h].stream, c->ev_fork, 0));
-    if (solo_own) RD_HIP(hipStreamWaitEvent(c->sstream, c->ev_fork, 0));
-  }
-  if (!solo.empty()) {
-    hipStream_t ss = solo_own ? c->sstream : c->stream;
-    k_mh_solo32<<<(int)solo.size(), kSoloThreads, 0, ss>>>(dsolo, c->d_desc, c->d_state,
-                                                          c->d_wf, V, a);
-    if (solo_own) RD_HIP(hipEventRecord(c->ev_solo, c->sstream));
-  }
-  for (int it = 1; it <= maxndim; ++it) {
-    for (int h = 0; h < nh; ++h) {
-      const Half& H = hv[h];
-      const int ne = (int)H.ents.size();
-      if (fp64) {
-        if (H.any_planar)
-          k_mh_field64<RD_GEOM_PLANAR><<<H.nwg, kBlock, 0, H.stream>>>(
-              H.dt, ne, c->d_desc, c->d_state, V, it, H.a);
-        if (H.any_tip)
-          k_mh_field64<RD_GEOM_TIP><<<H.nwg, kBlock, 0, H.stream>>>(H.dt, ne, c->d_desc,
-                                                                     c->d_state, V, it, H.a);
-        k_mh_settle<RD_PREC_FP64><<<H.nsettle, kSettle, 0, H.stream>>>(
-            H.dt, ne, c->d_desc, c->d_state, c->d_wf, V, it, H.a);
-      } else {
-        if (H.any_planar) {
-          if (pps == kJumpPairs)
-            k_mh_field32<RD_GEOM_PLANAR, kJumpPairs><<<H.nwg, 64 * kJumpWaves, 0, H.stream>>>(
-                H.dt, ne, c->d_desc, c->d_state, V, it, H.a);
-          else
-            k_mh_field32<RD_GEOM_PLANAR, 1><<<H.nwg, 64 * kJumpWaves, 0, H.stream>>>(
-                H.dt, ne, c->d_desc, c->d_state, V, it, H.a);
-        }
-        if (H.any_tip) {
-          if (pps == kJumpPairs)
-            k_mh_field32<RD_GEOM_TIP, kJumpPairs><<<H.nwg, 64 * kJumpWaves, 0, H.stream>>>(
-                H.dt, ne, c->d_desc, c->d_state, V, it, H.a);
-          else
-            k_mh_field32<RD_GEOM_TIP, 1><<<H.nwg, 64 * kJumpWaves, 0, H.stream>>>(
-                H.dt, ne, c->d_desc, c->d_state, V, it, H.a);
-        }
-        k_mh_settle<RD_PREC_MIXED><<<H.nsettle, kSettle, 0, H.stream>>>(
-            H.dt, ne, c->d_desc, c->d_state, c->d_wf, V, it, H.a);
-      }
-    }
-  }
-  for (int h = 0; h < nh; ++h) {
-    const Half& H = hv[h];
-    if (H.any_split)
-      k_mh_width_last<<<(int)H.ents.size(), 64, 0, H.stream>>>(H.dt, c->d_desc, c->d_state,
-                                                               H.a.counts, H.nsettle);
-  }
-  for (int h = 1; h < nh; ++h) {
-    RD_HIP(hipEventRecord(c->ev_join[h - 1], hv[h].stream));
-    RD_HIP(hipStreamWaitEvent(c->stream, c->ev_join[h - 1], 0));
-  }
-  if (solo_own) RD_HIP(hipStreamWaitEvent(c->stream, c->ev_solo, 0));
-  if (c->graphs) {
-    hipGraph_t g = nullptr;
-    const hipError_t le = hipGetLastError();
-    const hipError_t ce = hipStreamEndCapture(c->stream, &g);
-    if (le != hipSuccess) {
-      if (g) (void)hipGraphDestroy(g);
-      return hip_fail(le, "jump loop launch (capture)");
-    }
-    RD_HIP(ce);
-    const hipError_t ie = hipGraphInstantiate(&c->jump_exec, g, nullptr, nullptr, 0);
-    (void)hipGraphDestroy(g);
-    if (ie != hipSuccess) {
+    // Everything the launches depend on besides device data.  An unchanged key
+    // replays the captured launches (the kernels read the launch table and
+    // the chains from device memory, so new contents under the same pointers
+    // are picked up).
+    std::vector<unsigned char> key;
+    auto put = [&key](const void* v, size_t bytes) {
+      const unsigned char* b = (const unsigned char*)v;
+      key.insert(key.end(), b, b + bytes);
+    };
+    const int ints[] = {ne, nwg, (int)any_planar, (int)any_tip, (int)fp64, maxndim, C};
+    const void* ptrs[] = {dt, dall, c->d_desc, c->d_state, c->d_wf};
+    a.it0 = 1;
+    a.it1 = maxndim + 1;
+    a.spin = 1;
+    put(ints, sizeof(ints));
+    put(ptrs, sizeof(ptrs));
+    put(&words, sizeof(words));
+    put(&a, sizeof(a));
+    put(&V, sizeof(V));
+    put(&R, sizeof(R));
+    if (!(c->jump_exec && key == c->jump_key)) {
+      // the stream was synchronised after the previous launch of the old graph
+      if (c->jump_exec) RD_HIP(hipGraphExecDestroy(c->jump_exec));
       c->jump_exec = nullptr;
-      return hip_fail(ie, "hipGraphInstantiate (jump loop)");
+      c->jump_key.clear();
+      RD_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
+      random();
+      jumps(V, 1, maxndim + 1, true);
+      hipGraph_t g = nullptr;
+      const hipError_t le = hipGetLastError();
+      const hipError_t ce = hipStreamEndCapture(c->stream, &g);
+      if (le != hipSuccess) {
+        if (g) (void)hipGraphDestroy(g);
+        return hip_fail(le, "jump loop launch (capture)");
+      }
+      RD_HIP(ce);
+      const hipError_t ie = hipGraphInstantiate(&c->jump_exec, g, nullptr, nullptr, 0);
+      (void)hipGraphDestroy(g);
+      if (ie != hipSuccess) {
+        c->jump_exec = nullptr;
+        return hip_fail(ie, "hipGraphInstantiate (jump loop)");
+      }
+      c->jump_key = key;
     }
-    c->jump_key = key;
     RD_HIP(hipGraphLaunch(c->jump_exec, c->stream));
-    return RD_OK;
+  } else {
+    random();
+    jumps(V, 1, maxndim + 1, true);
   }
   RD_HIP(hipGetLastError());
+  bool waits = false;  // simulations of several workgroups that wait for each other
+  for (const Ent& e : ents)
+    waits |= e.segs > 1 && c->slots[e.slot].desc.mode == RD_EMIT_PLANAR_FE;
+  if (!waits) return RD_OK;
+  // a wait that gave up: its workgroups were never resident together (another
+  // context's work held the device); the chain states V are untouched
+  RD_HIP(hipMemcpyAsync(c->h_stop, a.stop, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+  RD_HIP(hipStreamSynchronize(c->stream));
+  if (*c->h_stop) {
+    random();
+    one_by_one();
+    RD_HIP(hipGetLastError());
+  }
   return RD_OK;
 }
 
@@ -2822,13 +2118,14 @@ static int engine_emission(rd_ctx* c, const std::vector<Ent>& all, int precision
     e.nch = nr;
     e.pbase = C;
     e.m = nr;
+    e.acc_off = (long long)ch.size();  // its place among the widths of the jumps
     C += nr;
     maxc = std::max(maxc, nr);
     maxndim = std::max(maxndim, c->slots[e.slot].desc.ndim);
     ch.push_back(e);
   }
   if (C == 0) return RD_OK;
-  r = ensure(c, c->chains, chain_bytes(C));
+  r = ensure(c, c->chains, 2 * chain_bytes(C));  // before and after the jumps
   if (!r) r = ensure(c, c->pts, sizeof(double) * 3 * (size_t)C);
   if (!r) r = ensure(c, c->fld, sizeof(double) * 3 * (size_t)C);
   if (r) return r;
@@ -2836,7 +2133,10 @@ static int engine_emission(rd_ctx* c, const std::vector<Ent>& all, int precision
   double* f = (double*)c->fld.p;
   double *pty = ptx + C, *ptz = ptx + 2 * (size_t)C;
   double *fx = f, *fy = f + C, *fz = f + 2 * (size_t)C;
-  Chains V = chain_view(c, C);
+  const Chains V = chain_view(c, C, 0);
+  Chains R = chain_view(c, C, 1);
+  R.ok = V.ok;
+  double* width = nullptr;
   Ent* dc;
   r = upload_tab(c, ch, &dc);
   if (r) return r;
@@ -2857,12 +2157,12 @@ static int engine_emission(rd_ctx* c, const std::vector<Ent>& all, int precision
     for (const Ent& e : ch) pend += c->h_state[e.slot].pending;
     if (pend == 0 || last) break;
   }
-  r = run_jumps(c, ch, C, precision, V, maxndim);
+  r = run_jumps(c, ch, C, precision, V, R, maxndim, &width);
   if (r) return r;
   r = upload_tab(c, ch, &dc);
   if (r) return r;
-  k_mh_finish<<<ch.size(), 256, 0, c->stream>>>(dc, c->d_desc, c->d_state, c->d_wf, V);
-  k_emit<<<ch.size(), 256, 0, c->stream>>>(dc, c->d_desc, c->d_state, c->d_wf, V, RD_ARRAYS,
+  k_mh_finish<<<ch.size(), 256, 0, c->stream>>>(dc, c->d_desc, c->d_state, c->d_wf, R, width);
+  k_emit<<<ch.size(), 256, 0, c->stream>>>(dc, c->d_desc, c->d_state, c->d_wf, R, RD_ARRAYS,
                                             c->logs ? (rd_emit_record*)c->elog.p : nullptr);
   RD_HIP(hipGetLastError());
   return RD_OK;

@@ -84,6 +84,12 @@ __device__ __forceinline__ void pack1(double xm, double ym, double zm, double qv
                    (float)(d * s - zn));
 }
 
+// The two parts of one coordinate.
+__device__ __forceinline__ void split(double xn, float& hi, float& lo) {
+  hi = (float)xn;
+  lo = (float)(xn - (double)hi);
+}
+
 __device__ __forceinline__ float rsq(float v) { return __builtin_amdgcn_rsqf(v); }
 
 // Guard for squared distances that can be exactly zero (a pair with itself
@@ -305,17 +311,6 @@ __device__ __forceinline__ float surface_acc32(const float4 h1, const float4 l1,
   const float dxy2 = __builtin_fmaf(dy, dy, dx * dx);
   const float ri = rsq(fmaxf(__builtin_fmaf(h2.z, h2.z, dxy2), kR2Min));
   return __builtin_fmaf(h2.w, h2.z * (ri * ri * ri), acc);
-}
-
-// surface_acc32 for a source s2 = (x, y, z, q_j/q_0 z) of high parts
-// (k_pack_particles' srf) and its low parts l2.
-__device__ __forceinline__ float surface_accq32(const float4 h1, const float4 l1, const float4 s2,
-                                                const float4 l2, float acc) {
-  const float dx = (h1.x - s2.x) + (l1.x - l2.x);
-  const float dy = (h1.y - s2.y) + (l1.y - l2.y);
-  const float dxy2 = __builtin_fmaf(dy, dy, dx * dx);
-  const float ri = rsq(fmaxf(__builtin_fmaf(s2.z, s2.z, dxy2), kR2Min));
-  return __builtin_fmaf(s2.w, ri * ri * ri, acc);
 }
 
 // True when every active target of the wavefront lies on the plane z = 0 and
@@ -652,8 +647,8 @@ __device__ __forceinline__ void field_finish32_tip(const DevGeom& g, const doubl
 // ------------------------------------------------------------------------
 // Mixed precision, hyperboloid tip.  The sphere image of a point (FP64,
 // tip_image_point64) is packed like a position: ihi = (x_im, y_im, z_im in nm
-// as float, distance of the point from the sphere centre in nm), ilo = the
-// low parts of the coordinates.  Pair terms are FP32 in nm; the image term
+// as float, sphere radius R / distance D of the point from the sphere centre),
+// ilo = the low parts of the coordinates.  Pair terms are FP32 in nm; the image term
 // keeps the reference's factor k_tip (acc_tip_ic_force.inc:17-22), so a
 // pair adds  q_j/q_0 * [ d/r^3 + k_tip (d/r^3 + R e/(D t^3)) ]  (nm^-2,
 // scaled by 1e18 * dfc * q_i * q_0 at the end), with d = target - source,
@@ -665,7 +660,7 @@ __device__ __forceinline__ void pack_image(double xm, double ym, double zm, doub
   const double s = 1.0e9;
   double xn = xi * s, yn = yi * s, zn = zi * s;
   float xh = (float)xn, yh = (float)yn, zh = (float)zn;
-  ihi = make_float4(xh, yh, zh, (float)(da * s));
+  ihi = make_float4(xh, yh, zh, (float)(R / da));
   ilo = make_float4((float)(xn - (double)xh), (float)(yn - (double)yh), (float)(zn - (double)zh),
                     0.0f);
 }
@@ -675,7 +670,7 @@ __device__ __forceinline__ void pack_image(double xm, double ym, double zm, doub
 __device__ __forceinline__ void tip_pair32_target(const float4 h1, const float4 l1,
                                                   const float4 ih1, const float4 il1,
                                                   const float4 h2, const float4 l2, float kt,
-                                                  float Rn, float& cx, float& cy, float& cz) {
+                                                  float& cx, float& cy, float& cz) {
   const float dx = (h1.x - h2.x) + (l1.x - l2.x);
   const float dy = (h1.y - h2.y) + (l1.y - l2.y);
   const float dz = (h1.z - h2.z) + (l1.z - l2.z);
@@ -694,11 +689,11 @@ __device__ __forceinline__ void tip_pair32_target(const float4 h1, const float4 
   const float ez = (h2.z - ih1.z) + (l2.z - il1.z);
   const float t2 = fmaxf(__builtin_fmaf(ez, ez, __builtin_fmaf(ey, ey, ex * ex)), kR2Min);
   const float ti = rsq(t2);
-  const float w = Rn * (ti * ti * ti) / ih1.w;
-  const float a = 1.0f + kt;
-  cx = h2.w * (dx * r3 * a + kt * (w * ex));
-  cy = h2.w * (dy * r3 * a + kt * (w * ey));
-  cz = h2.w * (dz * r3 * a + kt * (w * ez));
+  const float p = h2.w * (r3 * (1.0f + kt));
+  const float w = (h2.w * kt) * (ih1.w * (ti * ti * ti));
+  cx = __builtin_fmaf(dx, p, w * ex);
+  cy = __builtin_fmaf(dy, p, w * ey);
+  cz = __builtin_fmaf(dz, p, w * ez);
 }
 
 // Source-image pair (accelerations with j < i): the image is the source's;
@@ -707,7 +702,7 @@ __device__ __forceinline__ void tip_pair32_target(const float4 h1, const float4 
 __device__ __forceinline__ void tip_pair32_source(const float4 h1, const float4 l1,
                                                   const float4 h2, const float4 l2,
                                                   const float4 ih2, const float4 il2, float kt,
-                                                  float Rn, float& cx, float& cy, float& cz) {
+                                                  float& cx, float& cy, float& cz) {
   const float dx = (h1.x - h2.x) + (l1.x - l2.x);
   const float dy = (h1.y - h2.y) + (l1.y - l2.y);
   const float dz = (h1.z - h2.z) + (l1.z - l2.z);
@@ -725,11 +720,12 @@ __device__ __forceinline__ void tip_pair32_source(const float4 h1, const float4 
   const float fz = (h1.z - ih2.z) + (l1.z - il2.z);
   const float t2 = fmaxf(__builtin_fmaf(fz, fz, __builtin_fmaf(fy, fy, fx * fx)), kR2Min);
   const float ti = rsq(t2);
-  const float w = Rn * (ti * ti * ti) / ih2.w;
   // x, y: d/r^3 + k_tip (d/r^3 - R f/(D t^3));  z: d/r^3 + k_tip (-d/r^3 + R f/(D t^3))
-  cx = h2.w * (dx * r3 * (1.0f + kt) - kt * (w * fx));
-  cy = h2.w * (dy * r3 * (1.0f + kt) - kt * (w * fy));
-  cz = h2.w * (dz * r3 * (1.0f - kt) + kt * (w * fz));
+  const float w = (h2.w * kt) * (ih2.w * (ti * ti * ti));
+  const float p = h2.w * (r3 * (1.0f + kt));
+  cx = __builtin_fmaf(dx, p, -(w * fx));
+  cy = __builtin_fmaf(dy, p, -(w * fy));
+  cz = __builtin_fmaf(dz, h2.w * (r3 * (1.0f - kt)), w * fz);
 }
 
 // Mixed (tip): FP64 sums of the packed sources of chunks [c0, c1) at the
@@ -741,7 +737,6 @@ __device__ __forceinline__ void field_seg32_tip(const DevGeom& g, bool act, floa
                                                 int c1, float4* shi, float4* slo, double& fx,
                                                 double& fy, double& fz) {
   const float kt = g.ic ? (float)g.ktip : 0.0f;
-  const float Rn = (float)(g.R * 1e9);
   const int t = threadIdx.x;
   fx = 0.0;
   fy = 0.0;
@@ -758,7 +753,7 @@ __device__ __forceinline__ void field_seg32_tip(const DevGeom& g, bool act, floa
     if (act) {
       for (int jj = 0; jj < cnt; ++jj) {
         float cx, cy, cz;
-        tip_pair32_target(h1, l1, ih1, il1, shi[jj], slo[jj], kt, Rn, cx, cy, cz);
+        tip_pair32_target(h1, l1, ih1, il1, shi[jj], slo[jj], kt, cx, cy, cz);
         fx += (double)cx;
         fy += (double)cy;
         fz += (double)cz;

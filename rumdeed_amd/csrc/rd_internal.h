@@ -156,7 +156,6 @@ __device__ __forceinline__ int find_entry(const Ent* tab, int ne, int b, bool se
 }
 
 constexpr int kChunk = 256;  // canonical FP64 summation chunk
-constexpr int kJumpStreams = 2;  // streams of a pool's jump loop (3: the same makespan; 4: slower)
 constexpr int kBlock = 256;
 constexpr int kMaxSlots = 4096;
 constexpr int kLife = 1000;  // MAX_LIFE_TIME
@@ -178,13 +177,13 @@ struct Slot {
 
 }  // namespace rd
 
-// Jump workgroups (one partial each) from which a pool's mixed jump launches
-// give every workgroup kJumpPairs partials, paying the proposal and set-up
-// once for all of them (measured on the 256-request serving stream: 66.2 s
-// with 3 chunks per workgroup, 57.6 s with 6, 54.5 s with 12; below this size
-// the pool is latency-bound and more, smaller workgroups are faster).
-constexpr int kJumpPairWgs = 2048;
-constexpr int kJumpPairs = 4;
+// Instructions of pair terms per SIMD and jump a jump workgroup aims at, at
+// least (jump_chains).
+constexpr double kJumpTarget = 400.0;
+// Most chains per workgroup with a launch per jump: fewer read the particles
+// more often, more leave CUs idle (85k electrons, 150k chains, ms per step: 8
+// chains 171.9, 16 156.5, 32 150.6, 64 193.4).
+constexpr int kJumpApart = 32;
 
 // Partial sums of one pair launch are bounded by this many bytes (512 MiB);
 // larger launches run in bands whose partials are folded, in order, into
@@ -219,9 +218,9 @@ struct rd_ctx {
   // work buffers (grown on demand, never shrunk)
   rd::Buf part, pack_hi, pack_lo, pts, fld, pts_hi, pts_lo, stage, img64, tab, red, chains;
   rd::Buf pack_far;  // far-partner series of the particles (surface_far_coeffs)
-  rd::Buf pack_srf;  // (x, y, z, q z) high parts of the particles: cathode-surface sums
+  rd::Buf pack_srx, pack_srz;  // cathode-surface sums of the jumps: (x, y) FP64, (z^2, q z) FP32, nm
   rd::Buf rnd;  // random numbers of the Metropolis-Hastings jumps of a step
-  rd::Buf cnt;  // accept / reject counts per accept workgroup of a jump
+  rd::Buf cnt;  // acceptance counters and widths of a step's jumps (rd_jumps.h)
   rd::Buf img_hi, img_lo;  // packed sphere images of the particles (mixed, tip)
   // far image partners as an expansion (rd_tail.hip): the plan of the last
   // (d, N_ic_max), work arrays, lateral boxes; force options (rd_set_force_options)
@@ -252,18 +251,10 @@ struct rd_ctx {
   // while they are unchanged.
   int graphs = 0;
   hipGraphExec_t jump_exec = nullptr;
-  // Jump workgroups from which a pool's mixed jump launches give each
-  // workgroup kJumpPairs partials (rd_set_jump_pairing; kJumpPairWgs by default).
-  long long jump_pair_wgs = kJumpPairWgs;
+  int jump_room[4] = {};       // resident jump workgroups per form; 0: not asked yet
+  bool solo_jumps = true;      // all jumps of a step in one launch (rd_set_solo_jumps)
+  int* h_stop = nullptr;       // pinned: a jump workgroup's wait gave up
   std::vector<unsigned char> jump_key;
-
-  // further streams of the pool jump loop (default priority) and the events
-  // that fork them from and join them to `stream`
-  hipStream_t jstream[rd::kJumpStreams - 1] = {};
-  hipEvent_t ev_fork = nullptr, ev_join[rd::kJumpStreams - 1] = {};
-  bool solo_jumps = true;          // small simulations' jumps in one workgroup (mixed)
-  hipStream_t sstream = nullptr;  // one-workgroup jump loops of small simulations
-  hipEvent_t ev_solo = nullptr;
 };
 
 namespace rd {
@@ -318,8 +309,8 @@ inline int quad_lmax(int g0, int levels) {
   while (l > 0 && (g0 << l) > 1024) --l;
   return l;
 }
-// Packed mixed-precision copies (c->pack_hi / pack_lo, and c->pack_srf when
-// `surface`) of every entry's particles.
+// Packed mixed-precision copies (c->pack_hi / pack_lo, and c->pack_srx /
+// pack_srz when `surface`) of every entry's particles.
 int launch_pack(rd_ctx* c, const std::vector<Ent>& ents, bool surface = false);
 // Split nchunks source chunks into `segs` (at most max_segs) segments of
 // `cps` chunks each.
@@ -331,8 +322,6 @@ inline int seg_limit(int target_blocks, int want) {
   return (want + tb - 1) / tb;
 }
 constexpr int kWantPair = 8192;  // accelerations, field at points
-constexpr int kWantJump = 512;   // fields of the Metropolis-Hastings chains
-constexpr int kPoolJumpChunks = 3;  // least source chunks per jump partial in a pool
 int launch_grid_points(rd_ctx* c, double x0, double y0, double lx, double ly, int nx, int ny,
                        double zz);
 

@@ -18,6 +18,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "rd_ops64.h"
+
 #define RD_HD __host__ __device__ __forceinline__
 
 namespace rd {
@@ -30,7 +32,46 @@ static constexpr double kLn2Lo = 0x1.fdf473de6af28p-22;
 static constexpr double kInvLn2 = 0x1.71547652b82fep+0;
 static constexpr double kSqrtHalf = 0.70710678118654752440;
 
+// log(m 2^k) for m in [sqrt(1/2), sqrt(2)) given as f = m - 1 and
+// s = f / (2 + f).
+RD_HD double log_series(double f, double s, int k) {
+  double z = s * s;
+  double R = 2.0 / 23.0;
+  R = 2.0 / 21.0 + z * R;
+  R = 2.0 / 19.0 + z * R;
+  R = 2.0 / 17.0 + z * R;
+  R = 2.0 / 15.0 + z * R;
+  R = 2.0 / 13.0 + z * R;
+  R = 2.0 / 11.0 + z * R;
+  R = 2.0 / 9.0 + z * R;
+  R = 2.0 / 7.0 + z * R;
+  R = 2.0 / 5.0 + z * R;
+  R = 2.0 / 3.0 + z * R;
+  R = z * R;
+  double lm = f - s * (f - R);
+  double dk = (double)k;
+  return dk * kLn2Hi + (lm + dk * kLn2Lo);
+}
+
+// On the device the special cases are selected at the end instead of branched
+// around, and the quotient, whose operands are ordinary, takes the short
+// sequence: an accept step is a serial chain of logarithms in one wavefront.
 RD_HD double rd_log(double x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const bool sub = (dbits(x) >> 52) == 0;  // +0 or subnormal
+  const uint64_t u = dbits(sub ? x * 0x1p54 : x);
+  int k = (int)((u >> 52) & 0x7ff) - (sub ? 1023 + 54 : 1023);
+  double mm = bitsd((u & 0x000fffffffffffffULL) | 0x3ff0000000000000ULL);
+  const bool big = mm > 2.0 * kSqrtHalf;
+  mm = big ? mm * 0.5 : mm;
+  k += big;
+  const double f = mm - 1.0;
+  double r = log_series(f, Fast64::Div(2.0 + f)(f), k);
+  r = x == __builtin_inf() ? x : r;
+  r = x == 0.0 ? -__builtin_inf() : r;
+  r = x < 0.0 ? __builtin_nan("") : r;
+  return x != x ? x : r;
+#else
   if (x != x) return x;
   if (x < 0.0) return __builtin_nan("");
   if (x == 0.0) return -__builtin_inf();
@@ -49,23 +90,8 @@ RD_HD double rd_log(double x) {
     k += 1;
   }
   double f = mm - 1.0;
-  double s = f / (2.0 + f);
-  double z = s * s;
-  double R = 2.0 / 23.0;
-  R = 2.0 / 21.0 + z * R;
-  R = 2.0 / 19.0 + z * R;
-  R = 2.0 / 17.0 + z * R;
-  R = 2.0 / 15.0 + z * R;
-  R = 2.0 / 13.0 + z * R;
-  R = 2.0 / 11.0 + z * R;
-  R = 2.0 / 9.0 + z * R;
-  R = 2.0 / 7.0 + z * R;
-  R = 2.0 / 5.0 + z * R;
-  R = 2.0 / 3.0 + z * R;
-  R = z * R;
-  double lm = f - s * (f - R);
-  double dk = (double)k;
-  return dk * kLn2Hi + (lm + dk * kLn2Lo);
+  return log_series(f, f / (2.0 + f), k);
+#endif
 }
 
 RD_HD double rd_exp(double x) {

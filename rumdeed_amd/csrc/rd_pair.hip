@@ -399,7 +399,7 @@ __global__ void k_pack_particles(const Ent* tab, const SimDesc* desc, const SimS
                                  const double* __restrict__ X, const double* __restrict__ Y,
                                  const double* __restrict__ Z, const double* __restrict__ Q,
                                  float4* __restrict__ hi, float4* __restrict__ lo,
-                                 float4* __restrict__ srf) {
+                                 double2* __restrict__ srx, float2* __restrict__ srz) {
   const Ent e = tab[blockIdx.z];
   const int n = st[e.slot].n;
   int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -409,7 +409,10 @@ __global__ void k_pack_particles(const Ent* tab, const SimDesc* desc, const SimS
   pack1(X[gi], Y[gi], Z[gi], Q[gi], desc[e.slot].g.d, h, l);
   hi[gi] = h;
   lo[gi] = l;
-  if (srf) srf[gi] = make_float4(h.x, h.y, h.z, h.w * h.z);
+  if (srx) {
+    srx[gi] = make_double2(X[gi] * 1.0e9, Y[gi] * 1.0e9);
+    srz[gi] = make_float2(fmaxf(h.z * h.z, kR2Min), h.w * h.z);
+  }
 }
 
 // Far-partner coefficients (surface_far_coeffs) of the particles of every
@@ -889,7 +892,6 @@ __global__ __launch_bounds__(kBlock) void k_accel_tip32(const Ent* tab, int ne, 
   const DevGeom& gg = desc[e.slot].g;
   if (gg.kind != RD_GEOM_TIP) return;
   const float kt = gg.ic ? (float)gg.ktip : 0.0f;
-  const float Rn = (float)(gg.R * 1e9);
   const float4* hi = HI + e.base;
   const float4* lo = LO + e.base;
   const float4* ih = IHI + e.base;
@@ -923,9 +925,9 @@ __global__ __launch_bounds__(kBlock) void k_accel_tip32(const Ent* tab, int ne, 
         if (j == i) h2.w = 0.0f;
         float cx, cy, cz;
         if (j > i)
-          tip_pair32_target(h1, l1, ih1, il1, h2, slo[jj], kt, Rn, cx, cy, cz);
+          tip_pair32_target(h1, l1, ih1, il1, h2, slo[jj], kt, cx, cy, cz);
         else
-          tip_pair32_source(h1, l1, h2, slo[jj], sih[jj], sil[jj], kt, Rn, cx, cy, cz);
+          tip_pair32_source(h1, l1, h2, slo[jj], sih[jj], sil[jj], kt, cx, cy, cz);
         fx += (double)cx;
         fy += (double)cy;
         fz += (double)cz;
@@ -1342,7 +1344,7 @@ int launch_accel(rd_ctx* c, const std::vector<Ent>& in, int precision, hipEvent_
   if (r) return r;
   k_pack_particles<<<fin, 256, 0, c->stream>>>(dt, c->d_desc, c->d_state, c->x, c->y, c->z,
                                                 c->q, (float4*)c->pack_hi.p,
-                                                (float4*)c->pack_lo.p, nullptr);
+                                                (float4*)c->pack_lo.p, nullptr, nullptr);
   if (any_tip) {
     r = ensure(c, c->img_hi, sizeof(float4) * (size_t)c->cap);
     if (!r) r = ensure(c, c->img_lo, sizeof(float4) * (size_t)c->cap);
@@ -1540,7 +1542,7 @@ int launch_field(rd_ctx* c, const std::vector<Ent>& in, int mtot, int precision,
   k_pack_points<<<fin, 256, 0, c->stream>>>(dt, c->d_desc, ptx, pty, ptz, phi, plo);
   if (maxn > 0)
     k_pack_particles<<<dim3((maxn + 255) / 256, 1, ne), 256, 0, c->stream>>>(
-        dt, c->d_desc, c->d_state, c->x, c->y, c->z, c->q, ahi, alo, nullptr);
+        dt, c->d_desc, c->d_state, c->x, c->y, c->z, c->q, ahi, alo, nullptr, nullptr);
   if (any_far && maxn > 0)
     k_pack_far<<<dim3((maxn + 255) / 256, 1, ne), 256, 0, c->stream>>>(dt, c->d_desc, c->d_state,
                                                                          c->z, afar);
@@ -1564,14 +1566,16 @@ int launch_pack(rd_ctx* c, const std::vector<Ent>& ents, bool surface) {
   if (ents.empty() || maxn == 0) return RD_OK;
   int r = ensure(c, c->pack_hi, sizeof(float4) * (size_t)c->cap);
   if (!r) r = ensure(c, c->pack_lo, sizeof(float4) * (size_t)c->cap);
-  if (!r && surface) r = ensure(c, c->pack_srf, sizeof(float4) * (size_t)c->cap);
+  if (!r && surface) r = ensure(c, c->pack_srx, sizeof(double2) * (size_t)c->cap);
+  if (!r && surface) r = ensure(c, c->pack_srz, sizeof(float2) * (size_t)c->cap);
   if (r) return r;
   Ent* dt = nullptr;
   r = upload_tab(c, ents, &dt);
   if (r) return r;
   k_pack_particles<<<dim3((maxn + 255) / 256, 1, ents.size()), 256, 0, c->stream>>>(
       dt, c->d_desc, c->d_state, c->x, c->y, c->z, c->q, (float4*)c->pack_hi.p,
-      (float4*)c->pack_lo.p, surface ? (float4*)c->pack_srf.p : nullptr);
+      (float4*)c->pack_lo.p, surface ? (double2*)c->pack_srx.p : nullptr,
+      surface ? (float2*)c->pack_srz.p : nullptr);
   RD_HIP(hipGetLastError());
   return RD_OK;
 }

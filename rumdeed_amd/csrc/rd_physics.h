@@ -88,31 +88,48 @@ RD_HD EmitConsts emit_consts() {
   return e;
 }
 
+// The functions of the field and the work function take their quotients and
+// roots from M: Fast64 where F and w are ordinary numbers (f64_ordinary),
+// Ieee64 in general; the results are the same.
 // l = y^2 of the Forbes-Deane approximation, clamped to 1.
-RD_HD double fn_l(double l_const, double F, double w) { return l_const * (-1.0 * F) / (w * w); }
-RD_HD double fn_v(int ic, double l_const, double F, double w) {
+template <class M = Ieee64>
+__device__ __forceinline__ double fn_l(double l_const, double F, double w) {
+  return typename M::Div(w * w)(l_const * (-1.0 * F));
+}
+template <class M = Ieee64>
+__device__ __forceinline__ double fn_v(int ic, double l_const, double F, double w) {
   if (!ic) return 1.0;
-  double l = fn_l(l_const, F, w);
+  double l = fn_l<M>(l_const, F, w);
   if (l > 1.0) l = 1.0;
   return 1.0 - l + 1.0 / 6.0 * l * rd_log(l);
 }
-RD_HD double fn_t(int ic, double l_const, double F, double w) {
+template <class M = Ieee64>
+__device__ __forceinline__ double fn_t(int ic, double l_const, double F, double w) {
   if (!ic) return 1.0;
-  double l = fn_l(l_const, F, w);
+  double l = fn_l<M>(l_const, F, w);
   if (l > 1.0) l = 1.0;
   return 1.0 + l * (1.0 / 9.0 - 1.0 / 18.0 * rd_log(l));
 }
 // Escape_Prob_log: b_FN w^(3/2) v_y / (-F)
-RD_HD double fn_escape_log(const EmitConsts& e, int ic, double F, double w) {
+__device__ __forceinline__ double fn_escape_log(const EmitConsts& e, int ic, double F, double w) {
   double sw = __builtin_sqrt(w);
   return e.b_FN * (sw * sw * sw) * fn_v(ic, e.l_const, F, w) / (-1.0 * F);
 }
-// Elec_Supply_log: 2 log(-F) - 2 log(t_y) - log(w)
-RD_HD double fn_supply_log(const EmitConsts& e, int ic, double F, double w) {
-  return 2.0 * rd_log(-1.0 * F) - 2.0 * rd_log(fn_t(ic, e.l_const, F, w)) - rd_log(w);
+// Elec_Supply_log: 2 log(-F) - 2 log(t_y) - log(w), with log(w) given; the
+// logarithms of F and l side by side, so that their dependent chains overlap
+template <class M = Ieee64>
+__device__ __forceinline__ double fn_supply_log(const EmitConsts& e, int ic, double F, double w,
+                                                double log_w) {
+  if (!ic) return 2.0 * rd_log(-1.0 * F) - 2.0 * rd_log(1.0) - log_w;
+  double l = fn_l<M>(e.l_const, F, w);
+  l = l > 1.0 ? 1.0 : l;
+  const double log_l = rd_log(l), log_f = rd_log(-1.0 * F);
+  const double t = 1.0 + l * (1.0 / 9.0 - 1.0 / 18.0 * log_l);
+  return 2.0 * log_f - 2.0 * rd_log(t) - log_w;
 }
 // Elec_Supply_V2: (dt/q0) a_FN / (t_y^2 w) F^2
-RD_HD double fn_supply(const EmitConsts& e, int ic, double dt_q0, double F, double w) {
+__device__ __forceinline__ double fn_supply(const EmitConsts& e, int ic, double dt_q0, double F,
+                                            double w) {
   double t = fn_t(ic, e.l_const, F, w);
   return dt_q0 * e.a_FN / (t * t * w) * (F * F);
 }
@@ -137,68 +154,99 @@ RD_HD GtfConsts gtf_consts() {
   return k;
 }
 
-RD_HD double gtf_Nns(double n, double s) {
+template <class M>
+__device__ __forceinline__ double gtf_Nns(double n, double s) {
   if (n == 1.0) return (s + 1.0) * rd_exp(-s);
   double x = n * n;
-  double y = 1.0 / x;
+  double y = M::rcp(x);
   double z = (n - 1.0) * s;
+  const double es = rd_exp(-s), ens = rd_exp(-n * s);
   double sng;
   if (__builtin_fabs(z) > 1.0e-5)
-    sng = (x + 1.0) * (x * rd_exp(-s) - rd_exp(-n * s)) / (x - 1.0);
+    sng = typename M::Div(x - 1.0)((x + 1.0) * (x * es - ens));
   else
-    sng = (0.5 * (x + 1.0) * rd_exp(-s) / (n + 1.0)) *
+    sng = typename M::Div(n + 1.0)(0.5 * (x + 1.0) * es) *
           ((1.0 - n) * (s * s) + 2.0 * (1.0 + n) + 2.0 * s);
   double sn = -x * (0.10593434 * x + 0.35506593);
   double sd = -y * (0.10593434 * y + 0.35506593);
-  double sfn = x * rd_exp(-s);
-  double v = sng + sn * rd_exp(-n * s) + x * sd * rd_exp(-s);
+  double sfn = x * es;
+  double v = sng + sn * ens + x * sd * es;
   return v > sfn ? v : sfn;
 }
 
-// Get_Kevin_Jgtf_v2: current density (A/m^2) for field F (V/m), T (K), phi (eV).
-RD_HD double gtf_current(double F, double To, double Phi) {
+// Get_Kevin_Jgtf_v2 with the roots and quotients of M; `ok` turns false where
+// a quotient's operand may be outside M's range.
+template <class M>
+__device__ __forceinline__ double gtf_current_by(double F, double To, double Phi, bool& ok) {
   const GtfConsts k = gtf_consts();
   double Fo = __builtin_fabs(F) * 1.0e-9;
   if (Fo < 1.0e-9) return 0.0;
   const double chem = 7.0;
-  double s4 = __builtin_sqrt(4.0 * k.Qo * Fo);
-  double yo = s4 / Phi;
+  double s4 = M::sqrt(4.0 * k.Qo * Fo);
+  double yo = typename M::Div(Phi)(s4);
   double phix = Phi - s4;
   double ly = rd_log(yo);
-  double ty = 1.0 + (yo * yo) * (1.0 - ly) / 9.0;
-  double vy = 1.0 - (yo * yo) * (3.0 - ly) / 3.0;
-  double Tmin = (k.hbar * Fo / (4.0 * k.kb * ty)) * __builtin_sqrt(2.0 / (k.mo * Phi));
-  double Tmax = k.hbar * Fo / (k.kb * k.pi * __builtin_sqrt(k.mo * Phi * yo));
-  double betaT = 1.0 / (k.kb * To);
-  double betau = (2.0 / (k.hbar * Fo)) * __builtin_sqrt(2.0 * k.mo * Phi) * ty;
-  double betap = (k.pi / (k.hbar * Fo)) * __builtin_sqrt(k.mo * Phi * yo);
-  double theto = (4.0 * __builtin_sqrt(2.0 * k.mo * (Phi * Phi * Phi)) / (3.0 * k.hbar * Fo)) * vy;
+  double ty = 1.0 + typename M::Div(9.0)((yo * yo) * (1.0 - ly));
+  double vy = 1.0 - typename M::Div(3.0)((yo * yo) * (3.0 - ly));
+  const double rphi = M::sqrt(2.0 * k.mo * Phi), rpy = M::sqrt(k.mo * Phi * yo);
+  const typename M::Div by_hf(k.hbar * Fo);
+  double Tmin = typename M::Div(4.0 * k.kb * ty)(k.hbar * Fo) *
+                M::sqrt(typename M::Div(k.mo * Phi)(2.0));
+  double Tmax = typename M::Div(k.kb * k.pi * rpy)(k.hbar * Fo);
+  double betaT = M::rcp(k.kb * To);
+  double betau = by_hf(2.0) * rphi * ty;
+  double betap = by_hf(k.pi) * rpy;
+  double theto = typename M::Div(3.0 * k.hbar * Fo)(4.0 * M::sqrt(2.0 * k.mo * (Phi * Phi * Phi))) *
+                 vy;
+  ok = ok && ty != 0.0;
   double nft, sft;
   if (To < Tmin) {
-    nft = betaT / betau;
+    ok = ok && f64_ordinary(betau) && betau != 0.0;
+    nft = typename M::Div(betau)(betaT);
     sft = theto;
   } else if (To > Tmax) {
-    nft = betaT / betap;
+    nft = typename M::Div(betap)(betaT);
     sft = betap * phix;
   } else {
-    double Ap = 3.0 * (betap + betau) - 6.0 * theto / phix;
-    double Bp = -2.0 * (betap + 2.0 * betau) + 6.0 * theto / phix;
+    const typename M::Div by_phix(phix);
+    const double q6 = by_phix(6.0 * theto);
+    double Ap = 3.0 * (betap + betau) - q6;
+    double Bp = -2.0 * (betap + 2.0 * betau) + q6;
     double Cp = betau - betaT;
-    double po = (-Bp - __builtin_sqrt(Bp * Bp - 4.0 * Ap * Cp)) / (2.0 * Ap);
+    const double disc = Bp * Bp - 4.0 * Ap * Cp;
+    ok = ok && f64_ordinary(phix) && phix != 0.0 && f64_ordinary(Ap) && Ap != 0.0 && disc != 0.0;
+    double po = typename M::Div(2.0 * Ap)(-Bp - M::sqrt(disc));
     double Em = chem + po * phix;
     double theta = ((1.0 - po) * (1.0 - po)) * (2.0 * po + 1.0) * theto -
                    phix * po * (1.0 - po) * ((1.0 - po) * betau - po * betap);
     nft = 1.0;
     sft = theta + betaT * (Em - chem);
   }
-  double J = k.Arld * gtf_Nns(nft, sft) * (To * To);
+  ok = ok && f64_ordinary(nft) && nft != 0.0;
+  double J = k.Arld * gtf_Nns<M>(nft, sft) * (To * To);
   return J * 1.0e4;
+}
+
+// Get_Kevin_Jgtf_v2: current density (A/m^2) for field F (V/m), T (K), phi (eV).
+__device__ __forceinline__ double gtf_current(double F, double To, double Phi) {
+  const double aF = __builtin_fabs(F);
+  bool ok = aF >= 1.0e-3 && aF <= 1.0e15 && To >= 1.0e-3 && To <= 1.0e9 && Phi >= 1.0e-3 &&
+            Phi <= 1.0e3;
+  if (ok) {
+    const double J = gtf_current_by<Fast64>(F, To, Phi, ok);
+    if (ok) return J;
+  }
+  return gtf_current_by<Ieee64>(F, To, Phi, ok);
 }
 
 // ---- checkerboard work function (w_theta_checkerboard).  table: ny rows as
 // read from the file (first row = top), nx columns.  Returns w, sets sec.
 RD_HD double work_checker(const double* table, int nx, int ny, double ex0, double ey0,
                           double elx, double ely, double x, double y, int& sec) {
+  if (nx == 1 && ny == 1) {  // one section: no quotients
+    sec = 1;
+    return table[0];
+  }
   double xs = (x - ex0) / elx;
   double ys = (y - ey0) / ely;
   double x_len = 1.0 / nx, y_len = 1.0 / ny;

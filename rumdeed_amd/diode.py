@@ -113,7 +113,7 @@ class Diode:
         return rec
 
     def set_graphs(self, on: bool = True):
-        """Launch each step's Metropolis-Hastings jump loop as one HIP graph."""
+        """Launch each step's random numbers and Metropolis-Hastings jumps as one HIP graph."""
         check(self._lib.rd_set_graphs(self._h, int(bool(on))))
 
     def set_force_options(self, no_symmetric: bool = False, no_far_expansion: bool = False):
@@ -135,13 +135,12 @@ class Diode:
         return v.value
 
     def set_jump_pairing(self, min_workgroups: int):
-        """Pool launches of at least min_workgroups jump workgroups give each
-        workgroup four of their partial sums (results unchanged; 0: always)."""
+        """Checked, no effect: a step's jumps take one launch (rd_set_jump_pairing)."""
         check(self._lib.rd_set_jump_pairing(self._h, int(min_workgroups)))
 
     def set_solo_jumps(self, on: bool):
-        """Mixed precision: small simulations run all their jumps in one
-        workgroup (default on; rd_set_solo_jumps)."""
+        """All jumps of a step in one launch (default) or a launch per jump; the
+        results are identical (rd_set_solo_jumps)."""
         check(self._lib.rd_set_solo_jumps(self._h, int(bool(on))))
 
     def set_seed(self, seed: int, stream: int = 0):
