@@ -24,19 +24,18 @@ __device__ __forceinline__ double inv_r3_64(double r2, double es) {
   return M::rcp(r * r * r);
 }
 
-// Direct and planar image terms of one pair (acc_ic_planar_series.inc:19-63):
-// weights with the charge product pre.  za, zb: the heights of the pair's
-// first and second particle; (dx, dy, dz): target - source.
+// Direct and planar image factors of one pair (acc_ic_planar_series.inc:19-63):
+// i0 = 1 / r^3 of the direct term, (ix, iy, iz) the image series (g.ic).  za, zb:
+// the heights of the pair's first and second particle; (dx, dy, dz): target -
+// source.  For the source as the target, i0 and iz are the same and ix, iy
+// change sign.
 template <class M>
-__device__ __forceinline__ void planar_pair64(const DevGeom& g, double pre, double dx, double dy,
-                                              double dz, double za, double zb, double& ax,
-                                              double& ay, double& az) {
+__device__ __forceinline__ void planar_series64(const DevGeom& g, double dx, double dy, double dz,
+                                                double za, double zb, double& i0, double& ix,
+                                                double& iy, double& iz) {
   const double dxy2 = M::lift(dx * dx + dy * dy);
-  const double i0 = inv_r3_64<M>(dxy2 + dz * dz, g.es);
-  const double p0 = pre * i0;
-  ax = p0 * dx;
-  ay = p0 * dy;
-  az = p0 * dz;
+  i0 = inv_r3_64<M>(dxy2 + dz * dz, g.es);
+  ix = iy = iz = 0.0;
   if (!g.ic) return;
   auto partner = [&](double z_ic, double& diff) {
     diff = za - z_ic;
@@ -44,7 +43,9 @@ __device__ __forceinline__ void planar_pair64(const DevGeom& g, double pre, doub
   };
   double diff;
   double inv = partner(-1.0 * zb, diff);
-  double ix = -dx * inv, iy = -dy * inv, iz = -diff * inv;
+  ix = -dx * inv;
+  iy = -dy * inv;
+  iz = -diff * inv;
   for (int n = 1; n <= g.nic; ++n) {
     const double tnd = 2.0 * n * g.d;
     inv = partner(tnd - zb, diff);
@@ -64,6 +65,20 @@ __device__ __forceinline__ void planar_pair64(const DevGeom& g, double pre, doub
     iy = iy + dy * inv;
     iz = iz + diff * inv;
   }
+}
+
+// Direct and image terms of one pair with the charge product pre.
+template <class M>
+__device__ __forceinline__ void planar_pair64(const DevGeom& g, double pre, double dx, double dy,
+                                              double dz, double za, double zb, double& ax,
+                                              double& ay, double& az) {
+  double i0, ix, iy, iz;
+  planar_series64<M>(g, dx, dy, dz, za, zb, i0, ix, iy, iz);
+  const double p0 = pre * i0;
+  ax = p0 * dx;
+  ay = p0 * dy;
+  az = p0 * dz;
+  if (!g.ic) return;
   ax = ax + pre * ix;
   ay = ay + pre * iy;
   az = az + pre * iz;

@@ -28,6 +28,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <type_traits>
 
 #include "rd_field.h"
 #include "rd_internal.h"
@@ -39,16 +40,16 @@ namespace rd {
 // Workgroup of a compact pair launch: the launch-table entry it belongs to
 // (workgroups [wg0, next wg0) of the 1-D grid), its target block bx and its
 // source segment by.  The host lays the entry out as gx target blocks by
-// segs segments with gx = max(1, ceil(targets / kBlock)).
+// segs segments with gx = max(1, ceil(targets / per)).
 struct Tile {
   Ent e;
   int bx, by;
 };
-__device__ __forceinline__ Tile tile_of(const Ent* tab, int ne, bool points) {
+__device__ __forceinline__ Tile tile_of(const Ent* tab, int ne, bool points, int per = kBlock) {
   Tile t;
   t.e = tab[find_entry(tab, ne, blockIdx.x)];
   const int targets = points ? t.e.m : t.e.n_ub;
-  const int gx = max(1, (targets + kBlock - 1) / kBlock);
+  const int gx = max(1, (targets + per - 1) / per);
   const int local = blockIdx.x - t.e.wg0;
   t.bx = local % gx;
   t.by = local / gx;
@@ -104,6 +105,12 @@ __device__ __forceinline__ bool tts_pair(const TtsRole& r, int i, int j, int sp2
   if (r.sp1 != sp2) first = r.sp1 == RD_SPECIES_ELEC;
   return !(r.ion_only_e && sp2 == RD_SPECIES_ION);
 }
+
+}  // namespace rd
+
+#include "rd_terms64.h"
+
+namespace rd {
 
 // FP64 accelerations.  part layout per entry: [3][nchunks_ub][n_ub].
 template <int KIND>
@@ -1158,43 +1165,85 @@ static int launch_fp64_bands(rd_ctx* c, std::vector<Ent>& ents, bool points, hip
   const int ne = (int)ents.size();
   dim3 fin((maxt + 255) / 256, 1, ne);
   double* ptx = (double*)c->pts.p;
+  // Each pair evaluated once (k_accel64sym): unbanded, without the two-time-step
+  // roles, with image terms (without, the sums through LDS cost what the halved
+  // terms save: 16 384 electrons 0.48 ms, against 0.58), and from kSymRound pairs of
+  // chunks, a workgroup per CU: 4096 electrons, ten image terms, 120 pairs: 0.94
+  // ms, a lane per target 0.95, k_rows64 0.83; 6000, 276 pairs: 1.10, 2.26, 1.69.
+  auto sym_entry = [&](const Ent& e) {
+    return !points && B == 1 && e.tts == 0 && c->slots[e.slot].desc.g.ic && e.nchunks_ub > 1;
+  };
+  long long nsym = 0, waves = 0;
+  for (const Ent& e : ents)
+    if (sym_entry(e)) nsym += sym_pairs(e.nchunks_ub);
+  const bool sym = nsym >= kSymRound;
+  // Lanes on the terms (k_rows64) while a lane per target would leave SIMDs
+  // without a wavefront (1024 of them), or, where the image series makes a
+  // term dearer than its part in the sum, without a second one.  us a call, a
+  // lane per target / k_rows64: no series, 853 electrons (56 wavefronts) 122 /
+  // 54, 4096 (1024) 127 / 120, 6000 (2256) 200 / 202; two image terms, 2861 (540)
+  // 303 / 190, 6000 621 / 505, 8192 (4096) 789 / 820.
+  for (const Ent& e : ents)
+    if (!(sym && sym_entry(e))) {
+      const DevGeom& g = c->slots[e.slot].desc.g;
+      const bool series = g.kind == RD_GEOM_PLANAR && g.ic && g.nic > 0;
+      waves += (series ? 1LL : 2LL) * ((targets(e) + 63) / 64) * std::max(1, e.nchunks_ub);
+    }
+  const bool rows = waves <= 2048;
+  const int per = rows ? kRowT : kBlock;
   if (k0) RD_HIP(hipEventRecord(k0, c->stream));
   for (int b = 0; b < B; ++b) {
-    int nwg = 0;
+    int nwg = 0, nsw = 0;
     for (Ent& e : ents) {
       const int nch = std::max(e.nchunks_ub, 1);
       e.band0 = std::min(nch, b * e.pslots);
       e.band1 = std::min(nch, (b + 1) * e.pslots);
       e.wg0 = nwg;
       e.segs = 0;
-      if (e.band1 > e.band0 && targets(e) > 0) {
-        const int gx = std::max(1, (targets(e) + kBlock - 1) / kBlock);
+      e.wg1 = nsw;
+      if (sym && sym_entry(e)) {
+        const int p = sym_pairs(e.nchunks_ub), left = p % kSymRound;
+        e.segs = left < kSymRound / 3 && p > kSymRound ? p - left : p;
+        nsw += sym_groups(e.nchunks_ub, e.segs);
+      } else if (e.band1 > e.band0 && targets(e) > 0) {
+        const int gx = std::max(1, (targets(e) + per - 1) / per);
         segment(e.band1 - e.band0, seg_limit(gx, kWantPair), e.segs, e.cps);
         nwg += gx * e.segs;
       }
     }
     r = upload_tab(c, ents, dlast);
     if (r) return r;
-    if (nwg > 0) {
-      if (points) {
-        if (any_planar)
-          k_field64<RD_GEOM_PLANAR><<<nwg, kBlock, 0, c->stream>>>(
-              *dlast, ne, c->d_desc, c->d_state, ptx, ptx + mtot, ptx + 2 * (size_t)mtot, c->x,
-              c->y, c->z, c->q, part);
-        if (any_tip)
-          k_field64<RD_GEOM_TIP><<<nwg, kBlock, 0, c->stream>>>(
-              *dlast, ne, c->d_desc, c->d_state, ptx, ptx + mtot, ptx + 2 * (size_t)mtot, c->x,
-              c->y, c->z, c->q, part);
-      } else {
-        if (any_planar)
-          k_accel64<RD_GEOM_PLANAR><<<nwg, kBlock, 0, c->stream>>>(
-              *dlast, ne, c->d_desc, c->d_state, c->x, c->y, c->z, c->q, c->species,
-              (const double*)c->img64.p, part);
-        if (any_tip)
-          k_accel64<RD_GEOM_TIP><<<nwg, kBlock, 0, c->stream>>>(
-              *dlast, ne, c->d_desc, c->d_state, c->x, c->y, c->z, c->q, c->species,
-              (const double*)c->img64.p, part);
-      }
+    const double* img = (const double*)c->img64.p;
+    auto field = [&](auto kind) {
+      constexpr int K = decltype(kind)::value;
+      if (rows)
+        k_rows64<K, true><<<nwg, kBlock, 0, c->stream>>>(
+            *dlast, ne, c->d_desc, c->d_state, ptx, ptx + mtot, ptx + 2 * (size_t)mtot, c->x, c->y,
+            c->z, c->q, c->species, img, part);
+      else
+        k_field64<K><<<nwg, kBlock, 0, c->stream>>>(*dlast, ne, c->d_desc, c->d_state, ptx,
+                                                    ptx + mtot, ptx + 2 * (size_t)mtot, c->x, c->y,
+                                                    c->z, c->q, part);
+    };
+    auto accel = [&](auto kind) {
+      constexpr int K = decltype(kind)::value;
+      if (nsw > 0)
+        k_accel64sym<K><<<nsw, kBlock, 0, c->stream>>>(*dlast, ne, c->d_desc, c->d_state, c->x,
+                                                       c->y, c->z, c->q, img, part);
+      if (nwg > 0 && rows)
+        k_rows64<K, false><<<nwg, kBlock, 0, c->stream>>>(*dlast, ne, c->d_desc, c->d_state, c->x,
+                                                          c->y, c->z, c->x, c->y, c->z, c->q,
+                                                          c->species, img, part);
+      else if (nwg > 0)
+        k_accel64<K><<<nwg, kBlock, 0, c->stream>>>(*dlast, ne, c->d_desc, c->d_state, c->x, c->y,
+                                                    c->z, c->q, c->species, img, part);
+    };
+    if (points && nwg > 0) {
+      if (any_planar) field(std::integral_constant<int, RD_GEOM_PLANAR>{});
+      if (any_tip) field(std::integral_constant<int, RD_GEOM_TIP>{});
+    } else if (!points) {
+      if (any_planar) accel(std::integral_constant<int, RD_GEOM_PLANAR>{});
+      if (any_tip) accel(std::integral_constant<int, RD_GEOM_TIP>{});
     }
     if (B > 1) k_fold64<<<fin, 256, 0, c->stream>>>(*dlast, c->d_state, part, (double*)c->acc.p, points);
   }
