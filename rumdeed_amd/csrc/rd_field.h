@@ -236,9 +236,10 @@ __device__ __forceinline__ float surface_sum32(float zb, float wb, float dxy2, i
 constexpr int kFarTerms = 8;
 constexpr float kFarS = 0.1f;
 
-// a_0 .. a_7 of one source: zb = z_b, wb = d - z_b, dnm = d (nm).
-__device__ __forceinline__ void surface_far_coeffs(double zb, double wb, double dnm, int nic,
-                                                   float4& c0, float4& c1) {
+// q a_0 .. q a_7 of one source: q its charge over q_0, zb = z_b, wb = d - z_b,
+// dnm = d (nm).
+__device__ __forceinline__ void surface_far_coeffs(double q, double zb, double wb, double dnm,
+                                                   int nic, float4& c0, float4& c1) {
   double S[kFarTerms];
   for (int m = 0; m < kFarTerms; ++m) S[m] = 0.0;
   for (int k = 1; k <= nic; ++k) {
@@ -253,7 +254,7 @@ __device__ __forceinline__ void surface_far_coeffs(double zb, double wb, double 
     }
   }
   float c[kFarTerms];
-  double b = 1.0;  // binom(-3/2, m)
+  double b = q;  // q binom(-3/2, m)
   double d2m = 1.0;  // d^(2m)
   for (int m = 0; m < kFarTerms; ++m) {
     c[m] = (float)(b * S[m] * d2m);
@@ -264,53 +265,44 @@ __device__ __forceinline__ void surface_far_coeffs(double zb, double wb, double 
   c1 = make_float4(c[4], c[5], c[6], c[7]);
 }
 
-// sum_m a_m t^m, t = s / d^2.
-__device__ __forceinline__ float surface_far_eval(float t, float4 c0, float4 c1) {
+// acc + q sum_{m >= 1} a_m t^m, t = s / d^2 (a_0 is the same for every target).
+__device__ __forceinline__ float surface_far_acc(float t, float4 c0, float4 c1, float acc) {
   float v = __builtin_fmaf(c1.w, t, c1.z);
   v = __builtin_fmaf(v, t, c1.y);
   v = __builtin_fmaf(v, t, c1.x);
   v = __builtin_fmaf(v, t, c0.w);
   v = __builtin_fmaf(v, t, c0.z);
   v = __builtin_fmaf(v, t, c0.y);
-  return __builtin_fmaf(v, t, c0.x);
+  return __builtin_fmaf(v, t, acc);
 }
 
 // q_j/q_0 times surface_sum32 for the packed target (h1, l1) on the cathode
-// and the packed source (h2, l2); N0: the series stops at n = 0 (nic = 0).
-// The source height is its high part alone (the float sum of both parts
-// rounds to it but for ties).
-template <bool N0>
+// and the packed source (h2, l2).  The source height is its high part alone
+// (the float sum of both parts rounds to it but for ties).
 __device__ __forceinline__ float surface_term32(const float4 h1, const float4 l1, const float4 h2,
                                                 const float4 l2, int nic, float dnm) {
   const float dx = (h1.x - h2.x) + (l1.x - l2.x);
   const float dy = (h1.y - h2.y) + (l1.y - l2.y);
   const float dxy2 = __builtin_fmaf(dy, dy, dx * dx);
-  if (N0) {
-    const float ri = rsq(fmaxf(__builtin_fmaf(h2.z, h2.z, dxy2), kR2Min));
-    return h2.w * (h2.z * (ri * ri * ri));
-  }
   return h2.w * surface_sum32(h2.z, l2.w, dxy2, nic, dnm);
 }
 
-// With N_ic_max = 0: acc + q_j/q_0 z_b / r^3 for one source, in FP32.  The
-// callers add blocks of at most kSurfBlock such terms in FP32 and each block
-// sum to their FP64 total.  Every term of a block has the sign of the
-// charges (z_b >= 0, one species), so a block's FP32 sum is within
-// (kSurfBlock - 1) u = 15 * 2^-24 (< 1e-6) of its exact value; per source it
-// saves the conversion and the FP64 add.  The same holds for the paired-image
-// sum with N_ic_max > 0: sum_{k=-nic..nic} u_k / (rho^2 + u_k^2)^(3/2),
-// u_k = z_b + 2kd, is positive for every z_b in (0, d), rho and N_ic_max
-// (the terms n and -n-1 pair off towards (2 nic + 1) z_b / rho^3 at large
-// rho; checked on a grid of z_b and rho for N_ic_max up to 20), so the
-// cathode field's far-series loop adds its terms in the same blocks.
+// The sums over the sources of a target on the cathode: terms in FP32, in blocks
+// of at most kSurfBlock, block sums in FP64.  Every term q z_b / r^3 of a block has
+// the sign of the charges (z_b >= 0, one species), so a block's FP32 sum is within
+// (kSurfBlock - 1) u = 15 * 2^-24 (< 1e-6) of its exact value; so have the far
+// series' terms beyond a_0: their sum over k != 0, negative, rises towards 0 with
+// s.  Per source a block saves the conversion and the FP64 add.
 constexpr int kSurfBlock = 16;
-__device__ __forceinline__ float surface_acc32(const float4 h1, const float4 l1, const float4 h2,
-                                               const float4 l2, float acc) {
-  const float dx = (h1.x - h2.x) + (l1.x - l2.x);
-  const float dy = (h1.y - h2.y) + (l1.y - l2.y);
-  const float dxy2 = __builtin_fmaf(dy, dy, dx * dx);
-  const float ri = rsq(fmaxf(__builtin_fmaf(h2.z, h2.z, dxy2), kR2Min));
-  return __builtin_fmaf(h2.w, h2.z * (ri * ri * ri), acc);
+
+// acc + q z_b / r^3 of one source at the target t = (x, y, x_lo, y_lo): xy = (x, y,
+// x_lo, y_lo), zq = (z^2, q z); s receives the squared lateral distance.
+__device__ __forceinline__ float surface_acc32(float4 t, float4 xy, float2 zq, float& s,
+                                               float acc) {
+  const float dx = (t.x - xy.x) + (t.z - xy.z), dy = (t.y - xy.y) + (t.w - xy.w);
+  s = __builtin_fmaf(dy, dy, dx * dx);
+  const float ri = rsq(s + zq.x);
+  return __builtin_fmaf(zq.y, ri * ri * ri, acc);
 }
 
 // True when every active target of the wavefront lies on the plane z = 0 and
@@ -467,14 +459,45 @@ __device__ __forceinline__ void wave_min4(float v[4]) {
     for (int q = 0; q < 4; ++q) v[q] = fminf(v[q], __shfl_xor(v[q], o));
 }
 
+// Sum over the staged sources [0, cnt) of one chunk at a target on the cathode
+// (without the factor -2).  FAR: with the far series, every pair within its range;
+// far points at the chunk's coefficients.
+template <bool FAR>
+__device__ __forceinline__ double surface_chunk32(float4 t1, const float4* sxy, const float2* szq,
+                                                  const float4* far, int cnt, float inv_d2) {
+  double f = 0.0;
+  for (int jb = 0; jb < cnt; jb += kSurfBlock) {
+    const int je = min(cnt, jb + kSurfBlock);
+    float acc = 0.f, s;
+#pragma unroll 4
+    for (int jj = jb; jj < je; ++jj) {
+      acc = surface_acc32(t1, sxy[jj], szq[jj], s, acc);
+      // the coefficients through the scalar cache, beside the LDS reads
+      if (FAR)
+        acc = surface_far_acc(s * inv_d2, load_uniform(far, 2 * jj), load_uniform(far, 2 * jj + 1),
+                              acc);
+    }
+    f += (double)acc;
+  }
+  return f;
+}
+
 // Mixed (planar): FP64 sums, in nm^-2 per unit charge, of the packed sources
 // of chunks [c0, c1) at the packed target (h1, l1).
+//
+// On the cathode the pair terms are bound by VALU issue (the far series 21
+// instructions a pair, without 11; two or four targets per lane, which halve and
+// quarter the LDS and scalar reads, measured the same).  65 536 electrons at 256
+// x 256 points: 2.02 -> 1.81 ms with the far series, 1.37 -> 1.12 without, by terms
+// without a product or an addition of their own (charge and a_0 taken out of the
+// series, z^2 and q z formed at staging).
 __device__ __forceinline__ void field_seg32(const DevGeom& g, bool act, float4 h1, float4 l1,
                                             const float4* __restrict__ hi,
                                             const float4* __restrict__ lo,
                                             const float4* __restrict__ far, int n, int c0,
                                             int c1, float4* shi, float4* slo, float4* sfar,
-                                            double& fx, double& fy, double& fz) {
+                                            float4* sxy, float2* szq, double& fx, double& fy,
+                                            double& fz) {
   const int ic = g.ic, nic = g.nic;
   const float two_d = (float)(2.0 * g.d * 1e9);
   const float dnm = (float)(g.d * 1e9);
@@ -484,13 +507,14 @@ __device__ __forceinline__ void field_seg32(const DevGeom& g, bool act, float4 h
   const int t = threadIdx.x;
   // Lateral box of the wavefront's targets and of each chunk's sources (high
   // parts): when every pair of a chunk lies within the far series' range,
-  // the wavefront takes the chunk without the per-pair test (the same choice
-  // the test makes for each pair, so the same result).
+  // the wavefront takes the chunk without the per-pair test.
   const bool boxes = far && nic > 0;
+  const float4 t1 = make_float4(h1.x, h1.y, l1.x, l1.y);
   float tb[4] = {act ? h1.x : 3e38f, act ? -h1.x : 3e38f, act ? h1.y : 3e38f,
                  act ? -h1.y : 3e38f};  // min x, -max x, min y, -max y
   if (boxes) wave_min4(tb);
   __shared__ float sbox[4][kBlock / 64];
+  __shared__ double sa0[kBlock / 64];  // far series: the chunk's sum of q a_0
   fx = 0.0;
   fy = 0.0;
   fz = 0.0;
@@ -498,13 +522,18 @@ __device__ __forceinline__ void field_seg32(const DevGeom& g, bool act, float4 h
     const int jb = c * kChunk;
     __syncthreads();
     float sb[4] = {3e38f, 3e38f, 3e38f, 3e38f};
+    double a0 = 0.0;
     if (jb + t < n) {
-      const float4 hv = hi[jb + t];
+      const float4 hv = hi[jb + t], lv = lo[jb + t];
       shi[t] = hv;
-      slo[t] = lo[jb + t];
-      if (far) {
-        sfar[2 * t] = far[2 * (jb + t)];
+      slo[t] = lv;
+      sxy[t] = make_float4(hv.x, hv.y, lv.x, lv.y);
+      szq[t] = make_float2(fmaxf(hv.z * hv.z, kR2Min), hv.w * hv.z);
+      if (boxes) {
+        const float4 cv = far[2 * (jb + t)];
+        sfar[2 * t] = cv;
         sfar[2 * t + 1] = far[2 * (jb + t) + 1];
+        a0 = (double)cv.x;
       }
       sb[0] = hv.x;
       sb[1] = -hv.x;
@@ -513,74 +542,47 @@ __device__ __forceinline__ void field_seg32(const DevGeom& g, bool act, float4 h
     }
     if (boxes) {
       wave_min4(sb);
-      if ((t & 63) == 0)
+      for (int o = 32; o > 0; o >>= 1) a0 += __shfl_xor(a0, o);
+      if ((t & 63) == 0) {
         for (int q = 0; q < 4; ++q) sbox[q][t >> 6] = sb[q];
+        sa0[t >> 6] = a0;
+      }
     }
     __syncthreads();
     const int cnt = min(kChunk, n - jb);
     bool inside = false;
     if (boxes) {
+      a0 = 0.0;
+      for (int u = 0; u < kBlock / 64; ++u) a0 += sa0[u];
       for (int q = 0; q < 4; ++q) {
         sb[q] = sbox[q][0];
-        for (int u = 1; u < (int)(blockDim.x >> 6); ++u) sb[q] = fminf(sb[q], sbox[q][u]);
+        for (int u = 1; u < kBlock / 64; ++u) sb[q] = fminf(sb[q], sbox[q][u]);
       }
       // largest |dx|, |dy| over the chunk's pairs, with a margin of 1e-3 nm for
       // the low parts and the rounding of the differences
       const float ex = fmaxf(-tb[1] - sb[0], -sb[1] - tb[0]) + 1e-3f;
       const float ey = fmaxf(-tb[3] - sb[2], -sb[3] - tb[2]) + 1e-3f;
-      inside = fmaxf(ex, 0.f) * fmaxf(ex, 0.f) + fmaxf(ey, 0.f) * fmaxf(ey, 0.f) <=
-               0.999f * slim;
+      inside = __all(fmaxf(ex, 0.f) * fmaxf(ex, 0.f) + fmaxf(ey, 0.f) * fmaxf(ey, 0.f) <=
+                     0.999f * slim);
     }
-    if (act && surf) {  // fz holds the sum without the factor -2 until the end
-      if (nic > 0 && far && inside)
-        for (int jb2 = 0; jb2 < cnt; jb2 += kSurfBlock) {
-          const int je2 = min(cnt, jb2 + kSurfBlock);
-          float acc = 0.f;
-#pragma unroll 4
-          for (int jj = jb2; jj < je2; ++jj) {
-            const float4 h2 = shi[jj], l2 = slo[jj];
-            const float dx = (h1.x - h2.x) + (l1.x - l2.x);
-            const float dy = (h1.y - h2.y) + (l1.y - l2.y);
-            const float s = __builtin_fmaf(dy, dy, dx * dx);
-            const float ri = rsq(fmaxf(__builtin_fmaf(h2.z, h2.z, s), kR2Min));
-            float w = h2.z * (ri * ri * ri);
-            // the series coefficients through the scalar cache: the LDS
-            // reads of the sources are the kernel's limit
-            w += surface_far_eval(s * inv_d2, load_uniform(far, 2 * (jb + jj)),
-                                  load_uniform(far, 2 * (jb + jj) + 1));
-            acc = __builtin_fmaf(h2.w, w, acc);
-          }
-          fz += (double)acc;
+    if (surf && !boxes) {  // N_ic_max = 0; fz: without the factor -2 until the end
+      fz += surface_chunk32<false>(t1, sxy, szq, nullptr, cnt, inv_d2);
+    } else if (surf && inside) {
+      fz += a0 + surface_chunk32<true>(t1, sxy, szq, far + 2 * jb, cnt, inv_d2);
+    } else if (surf) {
+      for (int jb2 = 0; jb2 < cnt; jb2 += kSurfBlock) {
+        const int je2 = min(cnt, jb2 + kSurfBlock);
+        float acc = 0.f, s;
+        for (int jj = jb2; jj < je2; ++jj) {
+          acc = surface_acc32(t1, sxy[jj], szq[jj], s, acc);
+          if (s <= slim)
+            acc += surface_far_acc(s * inv_d2, sfar[2 * jj], sfar[2 * jj + 1], sfar[2 * jj].x);
+          else
+            acc = __builtin_fmaf(shi[jj].w, surface_far32(shi[jj].z, slo[jj].w, s, nic, dnm, 0.f),
+                                 acc);
         }
-      else if (nic > 0 && far)
-        for (int jb2 = 0; jb2 < cnt; jb2 += kSurfBlock) {
-          const int je2 = min(cnt, jb2 + kSurfBlock);
-          float acc = 0.f;
-          for (int jj = jb2; jj < je2; ++jj) {
-            const float4 h2 = shi[jj], l2 = slo[jj];
-            const float dx = (h1.x - h2.x) + (l1.x - l2.x);
-            const float dy = (h1.y - h2.y) + (l1.y - l2.y);
-            const float s = __builtin_fmaf(dy, dy, dx * dx);
-            const float ri = rsq(fmaxf(__builtin_fmaf(h2.z, h2.z, s), kR2Min));
-            float w = h2.z * (ri * ri * ri);
-            if (s <= slim)
-              w += surface_far_eval(s * inv_d2, sfar[2 * jj], sfar[2 * jj + 1]);
-            else
-              w = surface_far32(h2.z, l2.w, s, nic, dnm, w);
-            acc = __builtin_fmaf(h2.w, w, acc);
-          }
-          fz += (double)acc;
-        }
-      else if (nic == 0)
-        for (int jb2 = 0; jb2 < cnt; jb2 += kSurfBlock) {
-          const int je2 = min(cnt, jb2 + kSurfBlock);
-          float acc = 0.f;
-          for (int jj = jb2; jj < je2; ++jj) acc = surface_acc32(h1, l1, shi[jj], slo[jj], acc);
-          fz += (double)acc;
-        }
-      else
-        for (int jj = 0; jj < cnt; ++jj)
-          fz += (double)surface_term32<false>(h1, l1, shi[jj], slo[jj], nic, dnm);
+        fz += (double)acc;
+      }
     } else if (act) {
       for (int jj = 0; jj < cnt; ++jj) {
         const float4 h2 = shi[jj], l2 = slo[jj];

@@ -545,7 +545,7 @@ __device__ __forceinline__ void jump_planar(int ic, int nic, float dnm, const fl
 #pragma unroll
     for (int u = 0; u < T; ++u) {
       if (ic) {
-        d[u] += (double)surface_term32<false>(h1[u], l1[u], h2, l2, nic, dnm);
+        d[u] += (double)surface_term32(h1[u], l1[u], h2, l2, nic, dnm);
       } else {
         const float dx = (h1[u].x - h2.x) + (l1[u].x - l2.x);
         const float dy = (h1[u].y - h2.y) + (l1[u].y - l2.y);

@@ -425,7 +425,8 @@ __global__ void k_pack_particles(const Ent* tab, const SimDesc* desc, const SimS
 // Far-partner coefficients (surface_far_coeffs) of the particles of every
 // planar entry with image partners beyond n = 0: far[2 i], far[2 i + 1].
 __global__ void k_pack_far(const Ent* tab, const SimDesc* desc, const SimState* st,
-                           const double* __restrict__ Z, float4* __restrict__ far) {
+                           const double* __restrict__ Z, const double* __restrict__ Q,
+                           float4* __restrict__ far) {
   const Ent e = tab[blockIdx.z];
   const DevGeom& g = desc[e.slot].g;
   if (g.kind != RD_GEOM_PLANAR || !g.ic || g.nic < 1) return;
@@ -435,7 +436,7 @@ __global__ void k_pack_far(const Ent* tab, const SimDesc* desc, const SimState* 
   const size_t gi = (size_t)e.base + i;
   const double zn = Z[gi] * 1.0e9, dnm = g.d * 1.0e9;
   float4 c0, c1;
-  surface_far_coeffs(zn, dnm - zn, dnm, g.nic, c0, c1);
+  surface_far_coeffs(Q[gi] / Consts::q_0, zn, dnm - zn, dnm, g.nic, c0, c1);
   far[2 * gi] = c0;
   far[2 * gi + 1] = c1;
 }
@@ -1000,7 +1001,8 @@ __global__ __launch_bounds__(kBlock) void k_field_planar32(const Ent* tab, int n
                                                            const float4* __restrict__ LO,
                                                            const float4* __restrict__ FAR,
                                                            double* __restrict__ part) {
-  __shared__ float4 shi[kChunk], slo[kChunk], sfar[2 * kChunk];
+  __shared__ float4 shi[kChunk], slo[kChunk], sfar[2 * kChunk], sxy[kChunk];
+  __shared__ float2 szq[kChunk];
   const Tile tl = tile_of(tab, ne, true);
   const Ent& e = tl.e;
   const int m = e.m;
@@ -1021,7 +1023,7 @@ __global__ __launch_bounds__(kBlock) void k_field_planar32(const Ent* tab, int n
   }
   double fx, fy, fz;
   field_seg32(g, act, h1, l1, HI + e.base, LO + e.base, FAR ? FAR + 2 * (size_t)e.base : nullptr,
-              n, c0, c1, shi, slo, sfar, fx, fy, fz);
+              n, c0, c1, shi, slo, sfar, sxy, szq, fx, fy, fz);
   if (act) {
     double* P = part + e.part_off;
     const size_t S = (size_t)e.segs * m;
@@ -1594,7 +1596,7 @@ int launch_field(rd_ctx* c, const std::vector<Ent>& in, int mtot, int precision,
         dt, c->d_desc, c->d_state, c->x, c->y, c->z, c->q, ahi, alo, nullptr, nullptr);
   if (any_far && maxn > 0)
     k_pack_far<<<dim3((maxn + 255) / 256, 1, ne), 256, 0, c->stream>>>(dt, c->d_desc, c->d_state,
-                                                                         c->z, afar);
+                                                                         c->z, c->q, afar);
   if (k0) RD_HIP(hipEventRecord(k0, c->stream));
   if (any_planar)
     k_field_planar32<<<grid, kBlock, 0, c->stream>>>(dt, ne, c->d_desc, c->d_state, phi, plo,
