@@ -98,6 +98,12 @@ __device__ __forceinline__ float rsq(float v) { return __builtin_amdgcn_rsqf(v);
 // contribution for zero offsets.
 constexpr float kR2Min = 1.0e-20f;
 
+// Squared lateral distance with the guard in it: below a pair distance of 1e-7
+// nm it is no longer FP32's rounding, far below the reference's softening there.
+__device__ __forceinline__ float lateral2(float dx, float dy) {
+  return __builtin_fmaf(dy, dy, __builtin_fmaf(dx, dx, kR2Min));
+}
+
 // One image partner of a series at dz = DZ: add 1/r^3 to the suffix sum S.
 #define RD_PARTNER_SUM(DZ, S)                   \
   {                                             \
@@ -123,61 +129,49 @@ constexpr float kR2Min = 1.0e-20f;
 // particles near the anode.
 // NEAR: the caller guarantees nic <= 1 (no partners n >= 2), so the
 // suffix-sum loop is compiled out.
+//
+// dxy2 carries the guard (lateral2), so no partner needs one of its own.
 template <bool NEAR = false>
 __device__ __forceinline__ void ic_planar32(float zsum, float wsum, float dzab, float dxy2,
                                             int nic, float two_d, float& wxy, float& wz) {
-  float wo, wzo;
-  {
-    float r2 = fmaxf(__builtin_fmaf(zsum, zsum, dxy2), kR2Min);
-    float ri = rsq(r2);
-    wo = ri * ri * ri;
-    wzo = zsum * wo;
-  }
+  auto r3 = [dxy2](float dz) {
+    const float ri = rsq(__builtin_fmaf(dz, dz, dxy2));
+    return ri * ri * ri;
+  };
+  float wo = r3(zsum);
   if (nic < 1) {
     wxy = -wo;
-    wz = -wzo;
+    wz = -(zsum * wo);
     return;
   }
-  {
-    float dz1 = -wsum;
-    float r2 = fmaxf(__builtin_fmaf(dz1, dz1, dxy2), kR2Min);
-    float ri = rsq(r2);
-    float r3 = ri * ri * ri;
-    wo += r3;
-    wzo = __builtin_fmaf(dz1, r3, wzo);
+  const float ww = r3(wsum);
+  const float wzo = __builtin_fmaf(-wsum, ww, zsum * wo);
+  wo += ww;
+  if (NEAR || nic == 1) {  // each partner's own offset
+    const float zp = zsum + two_d, dp = dzab + two_d, dm = dzab - two_d;
+    const float po = r3(zp), ps = r3(dp), ms = r3(dm);
+    wxy = (ps + ms) - (wo + po);
+    wz = __builtin_fmaf(dp, ps, dm * ms) - __builtin_fmaf(zp, po, wzo);
+    return;
   }
   // suffix sums of 1/r^3: p (a + t_n) and m (a - t_n), o(pposite) and s(ame)
   float po = 0.f, mo = 0.f, ps = 0.f, ms = 0.f, ro = 0.f, rs = 0.f;
-  if (NEAR) {
-    // n = 1 alone: the sums start at its terms (the same values as adding
-    // them to zero, without the additions: every term is positive)
-    auto r3 = [dxy2](float dz) {
-      const float ri = rsq(__builtin_fmaf(dz, dz, dxy2));
-      return ri * ri * ri;
-    };
-    po = r3(zsum + two_d);
-    ps = r3(dzab + two_d);
-    ms = r3(dzab - two_d);
-    ro = po;
-    rs = ps - ms;
-  } else {
-    float tn = (float)nic * two_d;
-    for (int n = nic; n >= 2; --n) {
-      RD_PARTNER_SUM(zsum + tn, po);
-      RD_PARTNER_SUM(zsum - tn, mo);
-      RD_PARTNER_SUM(dzab + tn, ps);
-      RD_PARTNER_SUM(dzab - tn, ms);
-      ro = (ro + po) - mo;
-      rs = (rs + ps) - ms;
-      tn -= two_d;
-    }
-    RD_PARTNER_SUM(zsum + two_d, po);
-    RD_PARTNER_SUM(dzab + two_d, ps);
-    RD_PARTNER_SUM(dzab - two_d, ms);
+  float tn = (float)nic * two_d;
+  for (int n = nic; n >= 2; --n) {
+    RD_PARTNER_SUM(zsum + tn, po);
+    RD_PARTNER_SUM(zsum - tn, mo);
+    RD_PARTNER_SUM(dzab + tn, ps);
+    RD_PARTNER_SUM(dzab - tn, ms);
     ro = (ro + po) - mo;
     rs = (rs + ps) - ms;
+    tn -= two_d;
   }
-  const float so = NEAR ? po : po + mo, ss = ps + ms;
+  RD_PARTNER_SUM(zsum + two_d, po);
+  RD_PARTNER_SUM(dzab + two_d, ps);
+  RD_PARTNER_SUM(dzab - two_d, ms);
+  ro = (ro + po) - mo;
+  rs = (rs + ps) - ms;
+  const float so = po + mo, ss = ps + ms;
   wxy = ss - (wo + so);
   wz = __builtin_fmaf(dzab, ss, two_d * rs) - (__builtin_fmaf(zsum, so, wzo) + two_d * ro);
 }
@@ -459,9 +453,17 @@ __device__ __forceinline__ void wave_min4(float v[4]) {
     for (int q = 0; q < 4; ++q) v[q] = fminf(v[q], __shfl_xor(v[q], o));
 }
 
-// Sum over the staged sources [0, cnt) of one chunk at a target on the cathode
+// A wavefront's part of the staged sources [0, cnt) of a chunk: all of them, or
+// its quarter (split).
+struct ChunkPart {
+  int j0, j1;
+  __device__ __forceinline__ ChunkPart(bool split, int wv, int cnt)
+      : j0(split ? wv * 64 : 0), j1(split ? min(cnt, wv * 64 + 64) : cnt) {}
+};
+
+// Sum over cnt staged sources of one chunk at a target on the cathode
 // (without the factor -2).  FAR: with the far series, every pair within its range;
-// far points at the chunk's coefficients.
+// far points at their coefficients.  (Counted from 0, so that the addresses step.)
 template <bool FAR>
 __device__ __forceinline__ double surface_chunk32(float4 t1, const float4* sxy, const float2* szq,
                                                   const float4* far, int cnt, float inv_d2) {
@@ -482,8 +484,30 @@ __device__ __forceinline__ double surface_chunk32(float4 t1, const float4* sxy, 
   return f;
 }
 
+// The sums of a workgroup's wavefronts over their quarters of the chunks, added in
+// order into wavefront 0's.  lds: kQuarters doubles that the sums no longer read.
+constexpr int kQuarters = 3 * 3 * 64;
+__device__ __forceinline__ void add_quarters(void* lds, double& fx, double& fy, double& fz) {
+  double (*red)[3][64] = static_cast<double (*)[3][64]>(lds);
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  __syncthreads();
+  if (wv > 0) {
+    red[wv - 1][0][lane] = fx;
+    red[wv - 1][1][lane] = fy;
+    red[wv - 1][2][lane] = fz;
+  }
+  __syncthreads();
+  if (wv == 0)
+    for (int u = 0; u < 3; ++u) {
+      fx += red[u][0][lane];
+      fy += red[u][1][lane];
+      fz += red[u][2][lane];
+    }
+}
+
 // Mixed (planar): FP64 sums, in nm^-2 per unit charge, of the packed sources
-// of chunks [c0, c1) at the packed target (h1, l1).
+// of chunks [c0, c1) at the packed target (h1, l1); split: of this wavefront's
+// quarters of them.
 //
 // On the cathode the pair terms are bound by VALU issue (the far series 21
 // instructions a pair, without 11; two or four targets per lane, which halve and
@@ -491,7 +515,8 @@ __device__ __forceinline__ double surface_chunk32(float4 t1, const float4* sxy, 
 // x 256 points: 2.02 -> 1.81 ms with the far series, 1.37 -> 1.12 without, by terms
 // without a product or an addition of their own (charge and a_0 taken out of the
 // series, z^2 and q z formed at staging).
-__device__ __forceinline__ void field_seg32(const DevGeom& g, bool act, float4 h1, float4 l1,
+__device__ __forceinline__ void field_seg32(const DevGeom& g, bool split, bool act, float4 h1,
+                                            float4 l1,
                                             const float4* __restrict__ hi,
                                             const float4* __restrict__ lo,
                                             const float4* __restrict__ far, int n, int c0,
@@ -505,6 +530,7 @@ __device__ __forceinline__ void field_seg32(const DevGeom& g, bool act, float4 h
   const float inv_d2 = (float)(1.0 / ((g.d * 1e9) * (g.d * 1e9)));
   const bool surf = wave_on_surface(ic, act, h1, l1);
   const int t = threadIdx.x;
+  const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
   // Lateral box of the wavefront's targets and of each chunk's sources (high
   // parts): when every pair of a chunk lies within the far series' range,
   // the wavefront takes the chunk without the per-pair test.
@@ -549,7 +575,8 @@ __device__ __forceinline__ void field_seg32(const DevGeom& g, bool act, float4 h
       }
     }
     __syncthreads();
-    const int cnt = min(kChunk, n - jb);
+    const ChunkPart part(split, wv, min(kChunk, n - jb));
+    const int pc = part.j1 - part.j0;
     bool inside = false;
     if (boxes) {
       a0 = 0.0;
@@ -566,12 +593,14 @@ __device__ __forceinline__ void field_seg32(const DevGeom& g, bool act, float4 h
                      0.999f * slim);
     }
     if (surf && !boxes) {  // N_ic_max = 0; fz: without the factor -2 until the end
-      fz += surface_chunk32<false>(t1, sxy, szq, nullptr, cnt, inv_d2);
+      fz += surface_chunk32<false>(t1, sxy + part.j0, szq + part.j0, nullptr, pc, inv_d2);
     } else if (surf && inside) {
-      fz += a0 + surface_chunk32<true>(t1, sxy, szq, far + 2 * jb, cnt, inv_d2);
+      if (split && wv > 0) a0 = 0.0;  // the chunk's, once
+      fz += a0 + surface_chunk32<true>(t1, sxy + part.j0, szq + part.j0, far + 2 * (jb + part.j0), pc,
+                                       inv_d2);
     } else if (surf) {
-      for (int jb2 = 0; jb2 < cnt; jb2 += kSurfBlock) {
-        const int je2 = min(cnt, jb2 + kSurfBlock);
+      for (int jb2 = part.j0; jb2 < part.j1; jb2 += kSurfBlock) {
+        const int je2 = min(part.j1, jb2 + kSurfBlock);
         float acc = 0.f, s;
         for (int jj = jb2; jj < je2; ++jj) {
           acc = surface_acc32(t1, sxy[jj], szq[jj], s, acc);
@@ -584,28 +613,40 @@ __device__ __forceinline__ void field_seg32(const DevGeom& g, bool act, float4 h
         fz += (double)acc;
       }
     } else if (act) {
-      for (int jj = 0; jj < cnt; ++jj) {
-        const float4 h2 = shi[jj], l2 = slo[jj];
-        float dx = (h1.x - h2.x) + (l1.x - l2.x);
-        float dy = (h1.y - h2.y) + (l1.y - l2.y);
-        float dz = (h1.z - h2.z) + (l1.z - l2.z);
-        float dxy2 = __builtin_fmaf(dy, dy, dx * dx);
-        float r2 = fmaxf(__builtin_fmaf(dz, dz, dxy2), kR2Min);
-        float ri = rsq(r2);
-        float r3 = ri * ri * ri;
-        float cxy = r3, cz = dz * r3;
-        if (ic) {
-          float wxy, wz;
-          ic_planar32(h1.z + h2.z, l1.w + l2.w, dz, dxy2, nic, two_d, wxy, wz);
-          cxy += wxy;
-          cz += wz;
+      // the image series' switches are constants of each copy of the loop
+      auto sweep = [&](auto ic_t, auto near_t, auto n1_t) {
+        constexpr bool IC = decltype(ic_t)::value, NEAR = decltype(near_t)::value;
+        const int nicv = NEAR ? (decltype(n1_t)::value ? 1 : 0) : nic;
+#pragma unroll 2
+        for (int jj = part.j0; jj < part.j1; ++jj) {
+          const float4 h2 = shi[jj], l2 = slo[jj];
+          float dx = (h1.x - h2.x) + (l1.x - l2.x);
+          float dy = (h1.y - h2.y) + (l1.y - l2.y);
+          float dz = (h1.z - h2.z) + (l1.z - l2.z);
+          float dxy2 = lateral2(dx, dy);
+          float ri = rsq(__builtin_fmaf(dz, dz, dxy2));
+          float cxy = ri * ri * ri, cz = dz * cxy;
+          if (IC) {
+            float wxy, wz;
+            ic_planar32<NEAR>(h1.z + h2.z, l1.w + l2.w, dz, dxy2, nicv, two_d, wxy, wz);
+            cz = __builtin_fmaf(dz, cxy, wz);
+            cxy += wxy;
+          }
+          cxy *= h2.w;
+          cz *= h2.w;
+          fx += (double)(cxy * dx);
+          fy += (double)(cxy * dy);
+          fz += (double)cz;
         }
-        cxy *= h2.w;
-        cz *= h2.w;
-        fx += (double)(cxy * dx);
-        fy += (double)(cxy * dy);
-        fz += (double)cz;
-      }
+      };
+      if (!ic)
+        sweep(std::false_type{}, std::true_type{}, std::false_type{});
+      else if (nic == 0)
+        sweep(std::true_type{}, std::true_type{}, std::false_type{});
+      else if (nic == 1)
+        sweep(std::true_type{}, std::true_type{}, std::true_type{});
+      else
+        sweep(std::true_type{}, std::false_type{}, std::false_type{});
     }
   }
   if (surf) fz = -2.0 * fz;
@@ -730,8 +771,8 @@ __device__ __forceinline__ void tip_pair32_source(const float4 h1, const float4 
   cz = __builtin_fmaf(dz, h2.w * (r3 * (1.0f - kt)), w * fz);
 }
 
-// Mixed (tip): FP64 sums of the packed sources of chunks [c0, c1) at the
-// packed target (h1, l1) with its packed image (ih1, il1).
+// Mixed (tip): FP64 sums of this wavefront's quarters of the packed sources of
+// chunks [c0, c1) at the packed target (h1, l1) with its packed image (ih1, il1).
 __device__ __forceinline__ void field_seg32_tip(const DevGeom& g, bool act, float4 h1, float4 l1,
                                                 float4 ih1, float4 il1,
                                                 const float4* __restrict__ hi,
@@ -740,6 +781,7 @@ __device__ __forceinline__ void field_seg32_tip(const DevGeom& g, bool act, floa
                                                 double& fy, double& fz) {
   const float kt = g.ic ? (float)g.ktip : 0.0f;
   const int t = threadIdx.x;
+  const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
   fx = 0.0;
   fy = 0.0;
   fz = 0.0;
@@ -751,9 +793,10 @@ __device__ __forceinline__ void field_seg32_tip(const DevGeom& g, bool act, floa
       slo[t] = lo[jb + t];
     }
     __syncthreads();
-    const int cnt = min(kChunk, n - jb);
+    const ChunkPart part(true, wv, min(kChunk, n - jb));
     if (act) {
-      for (int jj = 0; jj < cnt; ++jj) {
+#pragma unroll 2
+      for (int jj = part.j0; jj < part.j1; ++jj) {
         float cx, cy, cz;
         tip_pair32_target(h1, l1, ih1, il1, shi[jj], slo[jj], kt, cx, cy, cz);
         fx += (double)cx;

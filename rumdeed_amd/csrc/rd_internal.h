@@ -108,6 +108,8 @@ struct Ent {
   int wg0, wg1;   // first workgroup of the entry in a compact launch (two layouts)
   int nic_pair;   // image partners n <= nic_pair in the mixed pair kernels (the
                   // rest, when fewer than N_ic_max, come from rd_tail.hip)
+  int split;      // mixed pair kernels: 4: a workgroup's wavefronts share 64 targets,
+                  // a quarter of every source chunk each; else 256 targets
   int lev;        // refinement level of the supply points (quad << lev per side)
   int tts;        // accelerations of the two-time-step update: atom_time_interval;
                   // 0: the standard accelerations (Calculate_Acceleration_Particles)

@@ -5,9 +5,9 @@
 // series (src/acc_ic_planar_series.inc:19-63) and the hyperboloid tip
 // (src/acc_tip_field_E.inc, src/acc_tip_image_point.inc, src/acc_tip_ic_force.inc).
 //
-// Shape: one lane per target (particle or field point), 256-lane workgroups;
-// sources are staged through LDS 256 at a time and read as wavefront-uniform
-// broadcasts.  blockIdx.z selects a simulation (launch-table entry), so one
+// Shape: one lane per target (particle or field point), 256-lane workgroups, or
+// four lanes per target (mixed, Targets32); sources are staged through LDS 256 at
+// a time and read as wavefront-uniform broadcasts.  blockIdx.z selects a simulation (launch-table entry), so one
 // launch serves every simulation of a pool; the source range of a simulation
 // is split over gridDim.y segments so that a launch has enough workgroups to
 // fill 256 CUs.  Every (segment, target) writes FP64 partial sums and a
@@ -49,12 +49,36 @@ __device__ __forceinline__ Tile tile_of(const Ent* tab, int ne, bool points, int
   Tile t;
   t.e = tab[find_entry(tab, ne, blockIdx.x)];
   const int targets = points ? t.e.m : t.e.n_ub;
+  if (t.e.split == 4) per = 64;
   const int gx = max(1, (targets + per - 1) / per);
   const int local = blockIdx.x - t.e.wg0;
   t.bx = local % gx;
   t.by = local / gx;
   return t;
 }
+
+// The targets of a mixed pair workgroup (Ent::split): 64 shared by its four
+// wavefronts, which take a quarter of every source chunk each, or, where there
+// are wavefronts enough, one per lane.  Sharing makes a lane's chain of sums a
+// quarter as long and gives a call on few targets four times the wavefronts.
+// us a call, one target per lane / shared: accelerations of 850 electrons, one
+// image term 88 / 55, 2861 of the tip 113 / 70, 11 000 174 / 157; the field at 777
+// points over 2861, tip 99 / 67, ten image terms 296 / 114; 5000 over 8000 161 /
+// 146.  On the cathode, where a pair takes 11 to 21 instructions, the staging of
+// the sources shows from 8000 wavefronts on: kernel 1.81 / 2.39 ms at 256 x 256
+// points over 65 536, equal at 40 x 40 over 37 409 (3675 wavefronts).
+constexpr int kSplitWaves = 4096;  // most wavefronts of a planar field that shares
+struct Targets32 {
+  bool split;
+  int wv, first, mine;  // the wavefront, the workgroup's first target, the lane's
+  bool writes;
+  __device__ __forceinline__ explicit Targets32(const Tile& tl, bool s = true)
+      : split(s), wv(__builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6)),
+        first(tl.bx * (s ? 64 : kBlock)),
+        mine(first + (s ? (int)threadIdx.x & 63 : (int)threadIdx.x)), writes(!s || wv == 0) {}
+};
+
+static_assert(2 * kChunk * sizeof(float4) >= kQuarters * sizeof(double), "add_quarters: staging LDS");
 
 // Image points of every particle (they depend on the particle alone).
 __global__ void k_tip_images64(const Ent* tab, const SimDesc* desc, const SimState* st,
@@ -464,13 +488,15 @@ __global__ __launch_bounds__(kBlock) void k_accel_planar32(const Ent* tab, int n
                                                            const float4* __restrict__ HI,
                                                            const float4* __restrict__ LO,
                                                            const int32_t* __restrict__ SP,
-                                                           double* __restrict__ part) {
-  __shared__ float4 shi[kChunk], slo[kChunk];
+                                                           double* __restrict__ out) {
+  __shared__ float4 shl[2 * kChunk];
+  float4 *shi = shl, *slo = shl + kChunk;
   __shared__ int ssp[TTS ? kChunk : 1];
   const Tile tl = tile_of(tab, ne, false);
   const Ent& e = tl.e;
   const int n = st[e.slot].n;
-  if (tl.bx * kBlock >= n) return;
+  const Targets32 tg(tl);
+  if (tg.first >= n) return;
   const int nchunks = (n + kChunk - 1) / kChunk;
   const int c0 = tl.by * e.cps;
   if (c0 >= nchunks) return;
@@ -482,7 +508,7 @@ __global__ __launch_bounds__(kBlock) void k_accel_planar32(const Ent* tab, int n
   const float4* hi = HI + e.base;
   const float4* lo = LO + e.base;
   const int t = threadIdx.x;
-  const int i = tl.bx * kBlock + t;
+  const int i = tg.mine;
   const bool act = i < n;
   float4 h1 = make_float4(0, 0, 0, 0), l1 = make_float4(0, 0, 0, 0);
   if (act) {
@@ -501,28 +527,36 @@ __global__ __launch_bounds__(kBlock) void k_accel_planar32(const Ent* tab, int n
       if (TTS) ssp[t] = e.tts > 0 ? SP[e.base + jb + t] : 0;
     }
     __syncthreads();
-    const int cnt = min(kChunk, n - jb);
-    if (act) {
-      for (int jj = 0; jj < cnt; ++jj) {
+    const ChunkPart part(true, tg.wv, min(kChunk, n - jb));
+    // The image series' switches and, away from the diagonal, the pair's roles are
+    // constants of each copy of the loop (a workgroup's targets lie in one chunk).
+    auto sweep = [&](auto ic_t, auto n1_t, auto role_t) {
+      constexpr bool IC = decltype(ic_t)::value;
+      constexpr bool N1 = decltype(n1_t)::value;      // NEAR: nic_pair == 1
+      constexpr int ROLE = decltype(role_t)::value;   // 0: by the indices, 1: first, 2: second
+      const int nicv = NEAR ? (N1 ? 1 : 0) : nic;
+      for (int jj = part.j0; jj < part.j1; ++jj) {
         const int j = jb + jj;
         const float4 h2 = shi[jj], l2 = slo[jj];
         float dx = (h1.x - h2.x) + (l1.x - l2.x);
         float dy = (h1.y - h2.y) + (l1.y - l2.y);
         float dz = (h1.z - h2.z) + (l1.z - l2.z);
-        float qj = (j == i) ? 0.0f : h2.w;
-        bool first = j > i;  // the target takes the first role of the pair
-        if (TTS && e.tts > 0 && !tts_pair(role, i, j, ssp[jj], first)) qj = 0.0f;
-        float dxy2 = __builtin_fmaf(dy, dy, dx * dx);
-        float r2 = fmaxf(__builtin_fmaf(dz, dz, dxy2), kR2Min);
-        float ri = rsq(r2);
-        float r3 = ri * ri * ri;
-        float cxy = r3, cz = dz * r3;
-        if (ic) {
+        float qj = h2.w;
+        bool first = ROLE == 1;  // the target takes the first role of the pair
+        if (ROLE == 0) {
+          first = j > i;
+          if (j == i) qj = 0.0f;
+          if (TTS && e.tts > 0 && !tts_pair(role, i, j, ssp[jj], first)) qj = 0.0f;
+        }
+        float dxy2 = lateral2(dx, dy);
+        float ri = rsq(__builtin_fmaf(dz, dz, dxy2));
+        float cxy = ri * ri * ri, cz = dz * cxy;
+        if (IC) {
           float wxy, wz;
           float dzab = first ? dz : -dz;
-          ic_planar32<NEAR>(h1.z + h2.z, l1.w + l2.w, dzab, dxy2, nic, two_d, wxy, wz);
+          ic_planar32<NEAR>(h1.z + h2.z, l1.w + l2.w, dzab, dxy2, nicv, two_d, wxy, wz);
+          cz = __builtin_fmaf(dz, cxy, wz);
           cxy += wxy;
-          cz += wz;
         }
         cxy *= qj;
         cz *= qj;
@@ -530,10 +564,28 @@ __global__ __launch_bounds__(kBlock) void k_accel_planar32(const Ent* tab, int n
         fy += (double)(cxy * dy);
         fz += (double)cz;
       }
+    };
+    auto by_series = [&](auto role_t) {
+      if (!ic)
+        sweep(std::false_type{}, std::false_type{}, role_t);
+      else if (NEAR && nic >= 1)
+        sweep(std::true_type{}, std::true_type{}, role_t);
+      else
+        sweep(std::true_type{}, std::false_type{}, role_t);
+    };
+    if (act) {
+      const int own = tg.first / kChunk;
+      if (TTS || c == own)
+        by_series(std::integral_constant<int, 0>{});
+      else if (c > own)
+        by_series(std::integral_constant<int, 1>{});
+      else
+        by_series(std::integral_constant<int, 2>{});
     }
   }
-  if (act) {
-    double* P = part + e.part_off;
+  add_quarters(shl, fx, fy, fz);
+  if (act && tg.writes) {
+    double* P = out + e.part_off;
     const size_t S = (size_t)e.segs * e.n_ub;
     P[0 * S + (size_t)tl.by * e.n_ub + i] = fx;
     P[1 * S + (size_t)tl.by * e.n_ub + i] = fy;
@@ -548,11 +600,11 @@ __global__ __launch_bounds__(kBlock) void k_accel_planar32(const Ent* tab, int n
 // evaluates every unordered pair once: the image series of the pair (i < j)
 // at z_i from j's partners, +F on i, and on j the Coulomb part reversed and
 // the image part with x and y reversed and z kept.  This kernel does the
-// same on the GPU.  Particles form blocks of kSymBlock; workgroup (X, Y),
+// same on the GPU.  Particles form blocks (kSymBlock); workgroup (X, Y),
 // X <= Y, takes the block pair.
-//   X < Y: wavefront w holds 64 targets of block X (one per lane) and, in
-//     phase p, the 64 sources of tile (w + p) mod kSymWaves of block Y.  Over
-//     64 steps lane l pairs its target with every source of the tile; the
+//   X < Y: wavefront w holds 64 T targets of block X (T per lane) and, in
+//     phase p, the 64 sources of tile (T w + p) mod kTiles of block Y.  Over
+//     64 steps lane l pairs its targets with every source of the tile; the
 //     sources' FP64 reaction sums ride along the wavefront (rotated one lane
 //     per step), so every source's sum is added in a fixed order without
 //     atomics.  Each tile belongs to one wavefront per phase, and the phases
@@ -567,9 +619,23 @@ __global__ __launch_bounds__(kBlock) void k_accel_planar32(const Ent* tab, int n
 // reaction sums) at part_off, [3][pslots][n_ub] from slot band0; the slots
 // Y >= X of the rows' own particles at d_off, [3][segs][d_ld] from particle
 // band0 * kSymBlock; k_fold_sym adds them to the running sums in slot order.
-constexpr int kSymWaves = 16;
-constexpr int kSymBlock = 64 * kSymWaves;
-constexpr int kSymMin = 16384;
+//
+// The pair terms are bound by VALU issue.  Forms, by a simulation's own particle
+// bound and series: `heavy` (nic_pair >= 1) or light, each from `min`
+// particles (below, the gather form finishes sooner: 8192 electrons 0.143 against
+// 0.123 ms heavy, 0.083 against 0.113 light), in blocks of kSymSmall below
+// `large` particles, so that the block pairs fill and even out the CUs, of
+// kSymLarge above, which halves the partials.  ms a call, blocks of 1024 (the
+// form before) / 512 / 256: heavy 16 384: 0.525 / 0.36 / 0.276, 37 409: 1.41 /
+// 1.20 / 1.16, 65 536: 3.94 / 3.45 / 3.42.  Light: two targets per lane, which halve
+// the rotations and LDS reads, 37 409: 0.95 (1024, one target) / 0.84 (512, one) /
+// 0.67 (512, two), 65 536: 2.55 / 2.22 / 1.86; heavy is slower with two (3.56
+// against 3.45), which leaves it five wavefronts per SIMD instead of eight.
+constexpr int kSymSmall = 256, kSymLarge = 512;
+struct SymRule {
+  int min, large;
+};
+constexpr SymRule kSymLight = {12288, 28672}, kSymHeavy = {5120, 49152};
 
 // One lane to the next: lane l takes lane l + 1's value (wave_rol:1).  Every
 // lane receives a value, so the old-value operand is v itself: the move can
@@ -584,12 +650,14 @@ __device__ __forceinline__ double wave_rotate(double v) {
   return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
 }
 
-template <bool NEAR>
-__global__ __launch_bounds__(kSymBlock) void k_accel_sym32(const Ent* tab, int ne,
-                                                           const SimDesc* desc, const SimState* st,
-                                                           const float4* __restrict__ HI,
-                                                           const float4* __restrict__ LO,
-                                                           double* __restrict__ part) {
+template <bool NEAR, int kSymBlock, int T>
+__global__ __launch_bounds__(kSymBlock / T) void k_accel_sym32(const Ent* tab, int ne,
+                                                             const SimDesc* desc,
+                                                             const SimState* st,
+                                                             const float4* __restrict__ HI,
+                                                             const float4* __restrict__ LO,
+                                                             double* __restrict__ part) {
+  constexpr int kThreads = kSymBlock / T, kTiles = kSymBlock / 64;
   __shared__ float4 shi[kSymBlock], slo[kSymBlock];
   __shared__ double jsum[3][kSymBlock];
   const Ent e = tab[find_entry(tab, ne, blockIdx.x, true)];
@@ -612,25 +680,32 @@ __global__ __launch_bounds__(kSymBlock) void k_accel_sym32(const Ent* tab, int n
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
   // padding (beyond n): charge 0 at the origin, so every term it enters is 0
   const float4 h0 = make_float4(0, 0, 0, 0), l0 = make_float4(0, 0, 0, dnm);
-  const int i = X * kSymBlock + t;
+  const int ib = X * kSymBlock + t, jb = Y * kSymBlock + t;  // the first of T
+  // Electrons only: every q/q_0 of both blocks exactly -1
+  bool electrons = true;
   // (values, not a select of addresses: selecting between a global element
   // and a local would put the local in scratch memory)
-  float4 h1 = h0, l1 = l0;
-  if (i < n) {
-    h1 = hi[i];
-    l1 = lo[i];
+  float4 h1[T], l1[T];
+#pragma unroll
+  for (int u = 0; u < T; ++u) {
+    h1[u] = h0;
+    l1[u] = l0;
+    if (ib + u * kThreads < n) {
+      h1[u] = hi[ib + u * kThreads];
+      l1[u] = lo[ib + u * kThreads];
+    }
+    float4 hs = h0, ls = l0;
+    if (jb + u * kThreads < n) {
+      hs = hi[jb + u * kThreads];
+      ls = lo[jb + u * kThreads];
+    }
+    electrons = electrons && h1[u].w == -1.0f && hs.w == -1.0f;
+    shi[t + u * kThreads] = hs;
+    slo[t + u * kThreads] = ls;
+    jsum[0][t + u * kThreads] = 0.0;
+    jsum[1][t + u * kThreads] = 0.0;
+    jsum[2][t + u * kThreads] = 0.0;
   }
-  const int js = Y * kSymBlock + t;
-  float4 hs = h0, ls = l0;
-  if (js < n) {
-    hs = hi[js];
-    ls = lo[js];
-  }
-  shi[t] = hs;
-  slo[t] = ls;
-  jsum[0][t] = 0.0;
-  jsum[1][t] = 0.0;
-  jsum[2][t] = 0.0;
   __syncthreads();
   // direct sums of the row's particles: D[c][slot][i - i0]; reaction sums of
   // the column's particles: R[c][X - band0][js]
@@ -639,92 +714,99 @@ __global__ __launch_bounds__(kSymBlock) void k_accel_sym32(const Ent* tab, int n
   const int i0 = e.banded ? e.band0 * kSymBlock : 0;
   double* R = part + e.part_off;
   const size_t RS = (size_t)e.pslots * e.n_ub;
-  double fx = 0.0, fy = 0.0, fz = 0.0;
+  double fx[T], fy[T], fz[T];
+#pragma unroll
+  for (int u = 0; u < T; ++u) fx[u] = fy[u] = fz[u] = 0.0;
   if (X == Y) {
     const int cnt = min(kSymBlock, n - Y * kSymBlock);
     for (int jj = 0; jj < cnt; ++jj) {
       const int j = Y * kSymBlock + jj;
       const float4 h2 = shi[jj], l2 = slo[jj];
-      float dx = (h1.x - h2.x) + (l1.x - l2.x);
-      float dy = (h1.y - h2.y) + (l1.y - l2.y);
-      float dz = (h1.z - h2.z) + (l1.z - l2.z);
-      float qj = (j == i) ? 0.0f : h2.w;
-      float dxy2 = __builtin_fmaf(dy, dy, dx * dx);
-      float r2 = fmaxf(__builtin_fmaf(dz, dz, dxy2), kR2Min);
-      float ri = rsq(r2);
-      float r3 = ri * ri * ri;
-      float cxy = r3, cz = dz * r3;
-      if (ic) {
-        float wxy, wz;
-        float dzab = (j > i) ? dz : -dz;
-        ic_planar32<NEAR>(h1.z + h2.z, l1.w + l2.w, dzab, dxy2, nic, two_d, wxy, wz);
-        cxy += wxy;
-        cz += wz;
+#pragma unroll
+      for (int u = 0; u < T; ++u) {
+        const int i = ib + u * kThreads;
+        float dx = (h1[u].x - h2.x) + (l1[u].x - l2.x);
+        float dy = (h1[u].y - h2.y) + (l1[u].y - l2.y);
+        float dz = (h1[u].z - h2.z) + (l1[u].z - l2.z);
+        float qj = (j == i) ? 0.0f : h2.w;
+        float dxy2 = lateral2(dx, dy);
+        float ri = rsq(__builtin_fmaf(dz, dz, dxy2));
+        float cxy = ri * ri * ri, cz = dz * cxy;
+        if (ic) {
+          float wxy, wz;
+          float dzab = (j > i) ? dz : -dz;
+          ic_planar32<NEAR>(h1[u].z + h2.z, l1[u].w + l2.w, dzab, dxy2, nic, two_d, wxy, wz);
+          cz = __builtin_fmaf(dz, cxy, wz);
+          cxy += wxy;
+        }
+        cxy *= qj;
+        cz *= qj;
+        fx[u] += (double)(cxy * dx);
+        fy[u] += (double)(cxy * dy);
+        fz[u] += (double)cz;
       }
-      cxy *= qj;
-      cz *= qj;
-      fx += (double)(cxy * dx);
-      fy += (double)(cxy * dy);
-      fz += (double)cz;
     }
-    if (i < n) {
-      const size_t o = (size_t)X * e.d_ld + (i - i0);
-      D[0 * DS + o] = fx;
-      D[1 * DS + o] = fy;
-      D[2 * DS + o] = fz;
-    }
+#pragma unroll
+    for (int u = 0; u < T; ++u)
+      if (ib + u * kThreads < n) {
+        const size_t o = (size_t)X * e.d_ld + (ib + u * kThreads - i0);
+        D[0 * DS + o] = fx[u];
+        D[1 * DS + o] = fy[u];
+        D[2 * DS + o] = fz[u];
+      }
     return;
   }
-  // Electrons only (every q/q_0 of both blocks exactly -1, uniform over the
-  // workgroup): a product with -1 is a sign, so each term is formed once for
-  // the pair and added to the target's sum and subtracted from the source's
-  // (or the reverse) -- the same roundings as multiplying by the charges.
-  // The image series' switches (ic; with NEAR, nic_pair in {0, 1}) are
-  // compile-time constants of each copy of the loop, so the loop holds no
-  // branch.
-  const bool uni = __syncthreads_and(h1.w == -1.0f && hs.w == -1.0f);
+  // Electrons only (uniform over the workgroup): a product with -1 is a sign, so
+  // each term is formed once for the pair and added to the target's sum and
+  // subtracted from the source's (or the reverse) -- the same roundings as
+  // multiplying by the charges.  The image series' switches (ic; with NEAR,
+  // nic_pair in {0, 1}) are compile-time constants of each copy of the loop, so
+  // the loop holds no branch.
+  const bool uni = __syncthreads_and(electrons);
   auto tiles = [&](auto uni_t, auto ic_t, auto n1_t) {
     constexpr bool UNI = decltype(uni_t)::value;
     constexpr bool IC = decltype(ic_t)::value;
     constexpr bool N1 = decltype(n1_t)::value;  // NEAR: nic_pair == 1
     const int nicv = NEAR ? (N1 ? 1 : 0) : nic;
-    for (int ph = 0; ph < kSymWaves; ++ph) {
-      const int tb = ((w + ph) & (kSymWaves - 1)) * 64;  // the tile of this wavefront
+    for (int ph = 0; ph < kTiles; ++ph) {
+      const int tb = ((w * T + ph) & (kTiles - 1)) * 64;  // the tile of this wavefront
       int jl = lane;  // the source whose reaction sum this lane holds
       double gx = jsum[0][tb + lane], gy = jsum[1][tb + lane], gz = jsum[2][tb + lane];
       for (int step = 0; step < 64; ++step) {
         const float4 h2 = shi[tb + jl], l2 = slo[tb + jl];
-        float dx = (h1.x - h2.x) + (l1.x - l2.x);
-        float dy = (h1.y - h2.y) + (l1.y - l2.y);
-        float dz = (h1.z - h2.z) + (l1.z - l2.z);
-        float dxy2 = __builtin_fmaf(dy, dy, dx * dx);
-        float r2 = fmaxf(__builtin_fmaf(dz, dz, dxy2), kR2Min);
-        float ri = rsq(r2);
-        float r3 = ri * ri * ri;
-        float cxy = r3, czi = dz * r3, czj = -czi;
-        if (IC) {
-          float wxy, wz;
-          ic_planar32<NEAR>(h1.z + h2.z, l1.w + l2.w, dz, dxy2, nicv, two_d, wxy, wz);
-          cxy += wxy;
-          czi += wz;
-          czj += wz;
-        }
-        if (UNI) {
-          const double tx = (double)(cxy * dx), ty = (double)(cxy * dy);
-          fx -= tx;
-          fy -= ty;
-          fz -= (double)czi;
-          gx += tx;
-          gy += ty;
-          gz -= (double)czj;
-        } else {
-          const float ci = cxy * h2.w, cj = cxy * h1.w;
-          fx += (double)(ci * dx);
-          fy += (double)(ci * dy);
-          fz += (double)(czi * h2.w);
-          gx -= (double)(cj * dx);
-          gy -= (double)(cj * dy);
-          gz += (double)(czj * h1.w);
+#pragma unroll
+        for (int u = 0; u < T; ++u) {
+          float dx = (h1[u].x - h2.x) + (l1[u].x - l2.x);
+          float dy = (h1[u].y - h2.y) + (l1[u].y - l2.y);
+          float dz = (h1[u].z - h2.z) + (l1[u].z - l2.z);
+          float dxy2 = lateral2(dx, dy);
+          float ri = rsq(__builtin_fmaf(dz, dz, dxy2));
+          float cxy = ri * ri * ri;
+          float czi = dz * cxy, czj = -czi;
+          if (IC) {
+            float wxy, wz;
+            ic_planar32<NEAR>(h1[u].z + h2.z, l1[u].w + l2.w, dz, dxy2, nicv, two_d, wxy, wz);
+            czi = __builtin_fmaf(dz, cxy, wz);
+            czj = __builtin_fmaf(-dz, cxy, wz);
+            cxy += wxy;
+          }
+          if (UNI) {
+            const double tx = (double)(cxy * dx), ty = (double)(cxy * dy);
+            fx[u] -= tx;
+            fy[u] -= ty;
+            fz[u] -= (double)czi;
+            gx += tx;
+            gy += ty;
+            gz -= (double)czj;
+          } else {
+            const float ci = cxy * h2.w, cj = cxy * h1[u].w;
+            fx[u] += (double)(ci * dx);
+            fy[u] += (double)(ci * dy);
+            fz[u] += (double)(czi * h2.w);
+            gx -= (double)(cj * dx);
+            gy -= (double)(cj * dy);
+            gz += (double)(czj * h1[u].w);
+          }
         }
         gx = wave_rotate(gx);
         gy = wave_rotate(gy);
@@ -741,7 +823,7 @@ __global__ __launch_bounds__(kSymBlock) void k_accel_sym32(const Ent* tab, int n
   auto by_series = [&](auto uni_t) {
     if (!ic)
       tiles(uni_t, std::false_type{}, std::false_type{});
-    else if (NEAR && nic >= 1)
+    else if (NEAR && T == 1 && nic >= 1)  // T = 2: nic_pair = 0
       tiles(uni_t, std::true_type{}, std::true_type{});
     else
       tiles(uni_t, std::true_type{}, std::false_type{});
@@ -750,17 +832,21 @@ __global__ __launch_bounds__(kSymBlock) void k_accel_sym32(const Ent* tab, int n
     by_series(std::true_type{});
   else
     by_series(std::false_type{});
-  if (i < n) {
-    const size_t o = (size_t)Y * e.d_ld + (i - i0);
-    D[0 * DS + o] = fx;
-    D[1 * DS + o] = fy;
-    D[2 * DS + o] = fz;
-  }
-  if (js < n) {
-    const size_t o = (size_t)(X - e.band0) * e.n_ub + js;
-    R[0 * RS + o] = jsum[0][t];
-    R[1 * RS + o] = jsum[1][t];
-    R[2 * RS + o] = jsum[2][t];
+#pragma unroll
+  for (int u = 0; u < T; ++u) {
+    const int i = ib + u * kThreads, j = jb + u * kThreads;
+    if (i < n) {
+      const size_t o = (size_t)Y * e.d_ld + (i - i0);
+      D[0 * DS + o] = fx[u];
+      D[1 * DS + o] = fy[u];
+      D[2 * DS + o] = fz[u];
+    }
+    if (j < n) {
+      const size_t o = (size_t)(X - e.band0) * e.n_ub + j;
+      R[0 * RS + o] = jsum[0][t + u * kThreads];
+      R[1 * RS + o] = jsum[1][t + u * kThreads];
+      R[2 * RS + o] = jsum[2][t + u * kThreads];
+    }
   }
 }
 
@@ -776,14 +862,14 @@ __global__ void k_fold_sym(const Ent* tab, const SimState* st, const double* __r
   const int n = st[e.slot].n;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const int B = i / kSymBlock;
+  const int block = e.cps * kChunk, B = i / block;
   const int x0 = e.band0, x1 = e.band1;
   if (B < x0) return;
-  const int nbk = min(e.segs, (n + kSymBlock - 1) / kSymBlock);
+  const int nbk = min(e.segs, (n + block - 1) / block);
   const int last = B >= x1 ? x1 : nbk;
   const double* R = part + e.part_off + i;
   const size_t RS = (size_t)e.pslots * e.n_ub;
-  const double* D = part + e.d_off + (i - x0 * kSymBlock);
+  const double* D = part + e.d_off + (i - x0 * block);
   const size_t DS = (size_t)e.segs * e.d_ld;
   double* A = acc + e.acc_off;
   double sx = 0.0, sy = 0.0, sz = 0.0;
@@ -887,12 +973,14 @@ __global__ __launch_bounds__(kBlock) void k_accel_tip32(const Ent* tab, int ne, 
                                                         const float4* __restrict__ LO,
                                                         const float4* __restrict__ IHI,
                                                         const float4* __restrict__ ILO,
-                                                        double* __restrict__ part) {
-  __shared__ float4 shi[kChunk], slo[kChunk], sih[kChunk], sil[kChunk];
+                                                        double* __restrict__ out) {
+  __shared__ float4 shl[4 * kChunk];
+  float4 *shi = shl, *slo = shl + kChunk, *sih = shl + 2 * kChunk, *sil = shl + 3 * kChunk;
   const Tile tl = tile_of(tab, ne, false);
   const Ent& e = tl.e;
   const int n = st[e.slot].n;
-  if (tl.bx * kBlock >= n) return;
+  const Targets32 tg(tl);
+  if (tg.first >= n) return;
   const int nchunks = (n + kChunk - 1) / kChunk;
   const int c0 = tl.by * e.cps;
   if (c0 >= nchunks) return;
@@ -905,7 +993,7 @@ __global__ __launch_bounds__(kBlock) void k_accel_tip32(const Ent* tab, int ne, 
   const float4* ih = IHI + e.base;
   const float4* il = ILO + e.base;
   const int t = threadIdx.x;
-  const int i = tl.bx * kBlock + t;
+  const int i = tg.mine;
   const bool act = i < n;
   float4 h1 = make_float4(0, 0, 0, 0), l1 = h1, ih1 = make_float4(0, 0, 0, 1), il1 = h1;
   if (act) {
@@ -925,9 +1013,9 @@ __global__ __launch_bounds__(kBlock) void k_accel_tip32(const Ent* tab, int ne, 
       sil[t] = il[jb + t];
     }
     __syncthreads();
-    const int cnt = min(kChunk, n - jb);
+    const ChunkPart part(true, tg.wv, min(kChunk, n - jb));
     if (act) {
-      for (int jj = 0; jj < cnt; ++jj) {
+      for (int jj = part.j0; jj < part.j1; ++jj) {
         const int j = jb + jj;
         float4 h2 = shi[jj];
         if (j == i) h2.w = 0.0f;
@@ -942,8 +1030,9 @@ __global__ __launch_bounds__(kBlock) void k_accel_tip32(const Ent* tab, int ne, 
       }
     }
   }
-  if (act) {
-    double* P = part + e.part_off;
+  add_quarters(shl, fx, fy, fz);
+  if (act && tg.writes) {
+    double* P = out + e.part_off;
     const size_t S = (size_t)e.segs * e.n_ub;
     P[0 * S + (size_t)tl.by * e.n_ub + i] = fx;
     P[1 * S + (size_t)tl.by * e.n_ub + i] = fy;
@@ -960,11 +1049,13 @@ __global__ __launch_bounds__(kBlock) void k_field_tip32(const Ent* tab, int ne, 
                                                         const float4* __restrict__ HI,
                                                         const float4* __restrict__ LO,
                                                         double* __restrict__ part) {
-  __shared__ float4 shi[kChunk], slo[kChunk];
+  __shared__ float4 shl[2 * kChunk];
+  float4 *shi = shl, *slo = shl + kChunk;
   const Tile tl = tile_of(tab, ne, true);
   const Ent& e = tl.e;
   const int m = e.m;
-  if (tl.bx * kBlock >= m) return;
+  const Targets32 tg(tl);
+  if (tg.first >= m) return;
   const int n = st[e.slot].n;
   const int nchunks = (n + kChunk - 1) / kChunk;
   const int c0 = tl.by * e.cps;
@@ -972,7 +1063,7 @@ __global__ __launch_bounds__(kBlock) void k_field_tip32(const Ent* tab, int ne, 
   const int c1 = min(nchunks, c0 + e.cps);
   const DevGeom& g = desc[e.slot].g;
   if (g.kind != RD_GEOM_TIP) return;
-  const int p = tl.bx * kBlock + threadIdx.x;
+  const int p = tg.mine;
   const bool act = p < m;
   float4 h1 = make_float4(0, 0, 0, 0), l1 = h1, ih1 = make_float4(0, 0, 0, 1), il1 = h1;
   if (act) {
@@ -983,7 +1074,8 @@ __global__ __launch_bounds__(kBlock) void k_field_tip32(const Ent* tab, int ne, 
   double fx, fy, fz;
   field_seg32_tip(g, act, h1, l1, ih1, il1, HI + e.base, LO + e.base, n, c0, c1, shi, slo, fx,
                   fy, fz);
-  if (act) {
+  add_quarters(shl, fx, fy, fz);
+  if (act && tg.writes) {
     double* P = part + e.part_off;
     const size_t S = (size_t)e.segs * m;
     P[0 * S + (size_t)tl.by * m + p] = fx;
@@ -993,7 +1085,7 @@ __global__ __launch_bounds__(kBlock) void k_field_tip32(const Ent* tab, int ne, 
 }
 
 // Mixed field at points (planar).
-__global__ __launch_bounds__(kBlock) void k_field_planar32(const Ent* tab, int ne, const SimDesc* desc,
+__global__ __launch_bounds__(kBlock, 6) void k_field_planar32(const Ent* tab, int ne, const SimDesc* desc,
                                                            const SimState* st,
                                                            const float4* __restrict__ PHI,
                                                            const float4* __restrict__ PLO,
@@ -1001,12 +1093,14 @@ __global__ __launch_bounds__(kBlock) void k_field_planar32(const Ent* tab, int n
                                                            const float4* __restrict__ LO,
                                                            const float4* __restrict__ FAR,
                                                            double* __restrict__ part) {
-  __shared__ float4 shi[kChunk], slo[kChunk], sfar[2 * kChunk], sxy[kChunk];
+  __shared__ float4 shi[kChunk], slo[kChunk], sxy[kChunk];
+  __shared__ float4 sfar[2 * kChunk];
   __shared__ float2 szq[kChunk];
   const Tile tl = tile_of(tab, ne, true);
   const Ent& e = tl.e;
   const int m = e.m;
-  if (tl.bx * kBlock >= m) return;
+  const Targets32 tg(tl, e.split == 4);
+  if (tg.first >= m) return;
   const int n = st[e.slot].n;
   const int nchunks = (n + kChunk - 1) / kChunk;
   const int c0 = tl.by * e.cps;
@@ -1014,7 +1108,7 @@ __global__ __launch_bounds__(kBlock) void k_field_planar32(const Ent* tab, int n
   const int c1 = min(nchunks, c0 + e.cps);
   const DevGeom& g = desc[e.slot].g;
   if (g.kind != RD_GEOM_PLANAR) return;
-  const int p = tl.bx * kBlock + threadIdx.x;
+  const int p = tg.mine;
   const bool act = p < m;
   float4 h1 = make_float4(0, 0, 0, 0), l1 = make_float4(0, 0, 0, 0);
   if (act) {
@@ -1022,9 +1116,10 @@ __global__ __launch_bounds__(kBlock) void k_field_planar32(const Ent* tab, int n
     l1 = PLO[e.pbase + p];
   }
   double fx, fy, fz;
-  field_seg32(g, act, h1, l1, HI + e.base, LO + e.base, FAR ? FAR + 2 * (size_t)e.base : nullptr,
+  field_seg32(g, tg.split, act, h1, l1, HI + e.base, LO + e.base, FAR ? FAR + 2 * (size_t)e.base : nullptr,
               n, c0, c1, shi, slo, sfar, sxy, szq, fx, fy, fz);
-  if (act) {
+  if (tg.split) add_quarters(sfar, fx, fy, fz);
+  if (act && tg.writes) {
     double* P = part + e.part_off;
     const size_t S = (size_t)e.segs * m;
     P[0 * S + (size_t)tl.by * m + p] = fx;
@@ -1115,14 +1210,18 @@ int upload_tab(rd_ctx* c, const std::vector<Ent>& ents, Ent** dtab) {
   return RD_OK;
 }
 
-// Whether a simulation's mixed planar accelerations take the pair-symmetric
-// form: from its own particle bound alone, so that its result does not depend
-// on the other simulations of a pool.  Below kSymMin particles the gather
-// form, whose source segments spread one simulation over more workgroups,
-// finishes sooner.
+// The rule of a simulation's pair-symmetric mixed accelerations (e.nic_pair is
+// set), and whether it takes them: from its own particle bound alone, so that
+// its result does not depend on the other simulations of a pool.
+static bool sym_light(const rd_ctx* c, const Ent& e) {
+  return !c->slots[e.slot].desc.g.ic || e.nic_pair == 0;
+}
+static const SymRule& sym_rule(const rd_ctx* c, const Ent& e) {
+  return sym_light(c, e) ? kSymLight : kSymHeavy;
+}
 static bool sym_form(const rd_ctx* c, const Ent& e) {
-  return c->slots[e.slot].desc.g.kind == RD_GEOM_PLANAR && e.n_ub >= kSymMin && e.tts == 0 &&
-         !(c->force_opts & RD_FORCE_NO_SYMMETRIC);
+  return c->slots[e.slot].desc.g.kind == RD_GEOM_PLANAR && e.n_ub >= sym_rule(c, e).min &&
+         e.tts == 0 && !(c->force_opts & RD_FORCE_NO_SYMMETRIC);
 }
 
 // FP64 pair launches in bands: the fewest bands B for which one band's
@@ -1253,6 +1352,13 @@ static int launch_fp64_bands(rd_ctx* c, std::vector<Ent>& ents, bool points, hip
   return RD_OK;
 }
 
+// Target blocks of a mixed entry; sets e.split (Targets32).
+static int target_blocks32(Ent& e, int targets, bool share) {
+  e.split = share ? 4 : 1;
+  const int per = share ? 64 : kBlock;
+  return std::max(1, (targets + per - 1) / per);
+}
+
 int launch_accel(rd_ctx* c, const std::vector<Ent>& in, int precision, hipEvent_t k0,
                  hipEvent_t k1) {
   std::vector<Ent> ents;
@@ -1280,6 +1386,7 @@ int launch_accel(rd_ctx* c, const std::vector<Ent>& in, int precision, hipEvent_
   if (r) return r;
   for (Ent& e : ents) {
     e.nchunks_ub = (e.n_ub + kChunk - 1) / kChunk;
+    e.split = 0;
     e.banded = 0;
     e.acc_off = 0;
     e.d_off = 0;
@@ -1306,7 +1413,7 @@ int launch_accel(rd_ctx* c, const std::vector<Ent>& in, int precision, hipEvent_
     return RD_OK;
   }
   // Mixed.  Gather-form entries: one partial set each, kept to the finish;
-  // pair-symmetric entries: nb = ceil(n_ub / kSymBlock) slots, in B bands of
+  // pair-symmetric entries: nb = ceil(n_ub / block) slots, in B bands of
   // ceil(nb / B) block rows whose partials (reaction and direct) fit the
   // budget, after the gather partials.
   long long off = 0;
@@ -1318,13 +1425,14 @@ int launch_accel(rd_ctx* c, const std::vector<Ent>& in, int precision, hipEvent_
     e.wg0 = nwg;
     e.band0 = 0;
     if (sym_form(c, e)) {
-      e.segs = (e.n_ub + kSymBlock - 1) / kSymBlock;
-      e.cps = kSymBlock / kChunk;
+      const int block = e.n_ub < sym_rule(c, e).large ? kSymSmall : kSymLarge;
+      e.segs = (e.n_ub + block - 1) / block;
+      e.cps = block / kChunk;
       e.band1 = e.segs;
       sym.push_back((int)k);
     } else {
       segment(e.nchunks_ub, seg_limit(gx, kWantPair), e.segs, e.cps);
-      nwg += gx * e.segs;
+      nwg += target_blocks32(e, e.n_ub, true) * e.segs;
       e.band1 = e.segs;
       e.pslots = e.segs;
       e.d_ld = e.n_ub;
@@ -1339,7 +1447,7 @@ int launch_accel(rd_ctx* c, const std::vector<Ent>& in, int precision, hipEvent_
       for (int k : sym) {
         const Ent& e = ents[k];
         const long long K = (e.segs + b - 1) / b;
-        bytes += 24LL * K * (e.n_ub + (b > 1 ? (long long)e.segs * kSymBlock : 0));
+        bytes += 24LL * K * (e.n_ub + (b > 1 ? (long long)e.segs * e.cps * kChunk : 0));
       }
       return bytes;
     };
@@ -1356,7 +1464,7 @@ int launch_accel(rd_ctx* c, const std::vector<Ent>& in, int precision, hipEvent_
     off += 3LL * K * e.n_ub;
     if (B > 1) {
       e.banded = 1;
-      e.d_ld = K * kSymBlock;
+      e.d_ld = K * e.cps * kChunk;
       e.d_off = off;
       off += 3LL * e.segs * e.d_ld;
       e.acc_off = acc_n;
@@ -1369,8 +1477,12 @@ int launch_accel(rd_ctx* c, const std::vector<Ent>& in, int precision, hipEvent_
   if (!r && acc_n > 0) r = ensure(c, c->acc, sizeof(double) * (size_t)acc_n);
   if (r) return r;
   double* part = (double*)c->part.p;
-  // the table of band b: the symmetric entries' rows and workgroup offsets
-  auto band_table = [&](int b, int& nsym) {
+  // the table of band b: the rows of the symmetric entries, and the workgroup
+  // offsets of those of one form
+  auto sym_form_of = [&](const Ent& e) {
+    return (e.cps * kChunk == kSymLarge ? 2 : 0) + (sym_light(c, e) ? 1 : 0);
+  };
+  auto band_table = [&](int b, int form, int& nsym) {
     nsym = 0;
     std::vector<Ent> t = ents;
     for (Ent& e : t) {
@@ -1379,12 +1491,16 @@ int launch_accel(rd_ctx* c, const std::vector<Ent>& in, int precision, hipEvent_
       const int K = e.pslots;
       e.band0 = std::min(e.segs, b * K);
       e.band1 = std::min(e.segs, (b + 1) * K);
+      if (sym_form_of(e) != form) continue;
       for (int X = e.band0; X < e.band1; ++X) nsym += e.segs - X;
     }
     return t;
   };
+  bool forms[4] = {};
+  for (int k : sym) forms[sym_form_of(ents[k])] = true;
+  const int form0 = (int)(std::find(forms, forms + 4, true) - forms);  // 4: none
   int nsym = 0;
-  std::vector<Ent> t0 = band_table(0, nsym);
+  std::vector<Ent> t0 = band_table(0, form0, nsym);
   Ent* dt = nullptr;
   r = upload_tab(c, t0, &dt);
   if (r) return r;
@@ -1433,20 +1549,29 @@ int launch_accel(rd_ctx* c, const std::vector<Ent>& in, int precision, hipEvent_
         dt, ne, c->d_desc, c->d_state, (const float4*)c->pack_hi.p, (const float4*)c->pack_lo.p,
         (const float4*)c->img_hi.p, (const float4*)c->img_lo.p, part);
   for (int b = 0; b < B; ++b) {
-    if (b > 0) {
-      std::vector<Ent> tb = band_table(b, nsym);
-      r = upload_tab(c, tb, &dt);
-      if (r) return r;
-    }
-    if (nsym > 0) {
-      if (near)
-        k_accel_sym32<true><<<nsym, kSymBlock, 0, c->stream>>>(
-            dt, ne, c->d_desc, c->d_state, (const float4*)c->pack_hi.p,
-            (const float4*)c->pack_lo.p, part);
+    for (int form = 0; form < 4; ++form) {
+      if (!forms[form]) continue;
+      if (b > 0 || form != form0) {
+        std::vector<Ent> tb = band_table(b, form, nsym);
+        r = upload_tab(c, tb, &dt);
+        if (r) return r;
+      }
+      if (nsym == 0) continue;
+      const auto run = [&](auto kernel, int threads) {
+        kernel<<<nsym, threads, 0, c->stream>>>(dt, ne, c->d_desc, c->d_state,
+                                                (const float4*)c->pack_hi.p,
+                                                (const float4*)c->pack_lo.p, part);
+      };
+      if (form == 0)
+        run(near ? k_accel_sym32<true, kSymSmall, 1> : k_accel_sym32<false, kSymSmall, 1>,
+            kSymSmall);
+      else if (form == 1)
+        run(k_accel_sym32<true, kSymSmall, 2>, kSymSmall / 2);
+      else if (form == 2)
+        run(near ? k_accel_sym32<true, kSymLarge, 1> : k_accel_sym32<false, kSymLarge, 1>,
+            kSymLarge);
       else
-        k_accel_sym32<false><<<nsym, kSymBlock, 0, c->stream>>>(
-            dt, ne, c->d_desc, c->d_state, (const float4*)c->pack_hi.p,
-            (const float4*)c->pack_lo.p, part);
+        run(k_accel_sym32<true, kSymLarge, 2>, kSymLarge / 2);
     }
     if (B > 1)
       k_fold_sym<<<fin, 256, 0, c->stream>>>(dt, c->d_state, part, (double*)c->acc.p);
@@ -1484,6 +1609,10 @@ int launch_field(rd_ctx* c, const std::vector<Ent>& in, int mtot, int precision,
     const int gx = std::max(1, (e.m + kBlock - 1) / kBlock);
     e.nchunks_ub = nch;
     segment(nch, seg_limit(gx, kWantPair), e.segs, e.cps);
+    e.split = 0;
+    const bool share = c->slots[e.slot].desc.g.kind == RD_GEOM_TIP ||
+                       (e.m + 63) / 64 * (long long)e.segs <= kSplitWaves;
+    const int groups = precision == RD_PREC_FP64 ? gx : target_blocks32(e, e.m, share);
     maxn = std::max(maxn, e.n_ub);
     e.part_off = off;
     e.band0 = 0;
@@ -1493,7 +1622,7 @@ int launch_field(rd_ctx* c, const std::vector<Ent>& in, int mtot, int precision,
     e.acc_off = 0;
     off += 3LL * e.pslots * e.m;
     e.wg0 = nwg;
-    nwg += gx * e.segs;
+    nwg += groups * e.segs;
   }
   dim3 fin((maxm + 255) / 256, 1, ents.size());
   if (precision == RD_PREC_FP64 && !fixed) {
