@@ -717,8 +717,7 @@ __device__ __forceinline__ void tip_pair32_target(const float4 h1, const float4 
   const float dx = (h1.x - h2.x) + (l1.x - l2.x);
   const float dy = (h1.y - h2.y) + (l1.y - l2.y);
   const float dz = (h1.z - h2.z) + (l1.z - l2.z);
-  const float r2 = fmaxf(__builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx)), kR2Min);
-  const float ri = rsq(r2);
+  const float ri = rsq(__builtin_fmaf(dz, dz, lateral2(dx, dy)));
   const float r3 = ri * ri * ri;
   if (kt == 0.0f) {  // no image charge
     cx = h2.w * (dx * r3);
@@ -730,10 +729,9 @@ __device__ __forceinline__ void tip_pair32_target(const float4 h1, const float4 
   const float ex = (h2.x - ih1.x) + (l2.x - il1.x);
   const float ey = (h2.y - ih1.y) + (l2.y - il1.y);
   const float ez = (h2.z - ih1.z) + (l2.z - il1.z);
-  const float t2 = fmaxf(__builtin_fmaf(ez, ez, __builtin_fmaf(ey, ey, ex * ex)), kR2Min);
-  const float ti = rsq(t2);
-  const float p = h2.w * (r3 * (1.0f + kt));
-  const float w = (h2.w * kt) * (ih1.w * (ti * ti * ti));
+  const float ti = rsq(__builtin_fmaf(ez, ez, lateral2(ex, ey)));
+  const float p = (h2.w * (1.0f + kt)) * r3;  // the factors of the source come first: several
+  const float w = (h2.w * kt) * (ih1.w * (ti * ti * ti));  // targets share them
   cx = __builtin_fmaf(dx, p, w * ex);
   cy = __builtin_fmaf(dy, p, w * ey);
   cz = __builtin_fmaf(dz, p, w * ez);
@@ -749,8 +747,7 @@ __device__ __forceinline__ void tip_pair32_source(const float4 h1, const float4 
   const float dx = (h1.x - h2.x) + (l1.x - l2.x);
   const float dy = (h1.y - h2.y) + (l1.y - l2.y);
   const float dz = (h1.z - h2.z) + (l1.z - l2.z);
-  const float r2 = fmaxf(__builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx)), kR2Min);
-  const float ri = rsq(r2);
+  const float ri = rsq(__builtin_fmaf(dz, dz, lateral2(dx, dy)));
   const float r3 = ri * ri * ri;
   if (kt == 0.0f) {  // no image charge
     cx = h2.w * (dx * r3);
@@ -761,14 +758,13 @@ __device__ __forceinline__ void tip_pair32_source(const float4 h1, const float4 
   const float fx = (h1.x - ih2.x) + (l1.x - il2.x);
   const float fy = (h1.y - ih2.y) + (l1.y - il2.y);
   const float fz = (h1.z - ih2.z) + (l1.z - il2.z);
-  const float t2 = fmaxf(__builtin_fmaf(fz, fz, __builtin_fmaf(fy, fy, fx * fx)), kR2Min);
-  const float ti = rsq(t2);
+  const float ti = rsq(__builtin_fmaf(fz, fz, lateral2(fx, fy)));
   // x, y: d/r^3 + k_tip (d/r^3 - R f/(D t^3));  z: d/r^3 + k_tip (-d/r^3 + R f/(D t^3))
   const float w = (h2.w * kt) * (ih2.w * (ti * ti * ti));
-  const float p = h2.w * (r3 * (1.0f + kt));
+  const float p = (h2.w * (1.0f + kt)) * r3;
   cx = __builtin_fmaf(dx, p, -(w * fx));
   cy = __builtin_fmaf(dy, p, -(w * fy));
-  cz = __builtin_fmaf(dz, h2.w * (r3 * (1.0f - kt)), w * fz);
+  cz = __builtin_fmaf(dz, (h2.w * (1.0f - kt)) * r3, w * fz);
 }
 
 // Mixed (tip): FP64 sums of this wavefront's quarters of the packed sources of
