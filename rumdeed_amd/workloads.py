@@ -43,9 +43,10 @@ def grid_points(nx=SNAPSHOT_GRID, ny=SNAPSHOT_GRID, box=SNAPSHOT_BOX, z=0.0):
     return np.stack([gx.ravel(), gy.ravel(), np.full(nx * ny, z)], axis=1)
 
 
-# particles from which the mixed planar force is pair-symmetric: with image
-# partners n >= 1, and without
+# particles from which the planar force is pair-symmetric: mixed with image
+# partners n >= 1, and without; FP64 (256 pairs of 256-particle chunks)
 SYM_MIN, SYM_MIN_LIGHT = 5120, 12288
+SYM_MIN_FP64 = 23 * 256 + 1
 SYM_REACTION_FLOPS = 9  # reaction on the source: z terms 2, charge products 4, sums 3
 FAR_RHO_MAX = 0.42  # convergence ratio up to which the far partners are an expansion
 
@@ -65,13 +66,15 @@ def far_expansion_used(pos, d: float, n_ic_max: int) -> bool:
 
 def force_flops(n: int, n_ic_max: int, precision: str = "mixed", far_expansion=False) -> int:
     """Algorithmic flops of the pair kernel of one planar acceleration
-    evaluation of n particles: the gather form evaluates n (n - 1) ordered
-    pairs; the pair-symmetric form (mixed, n >= SYM_MIN or
-    SYM_MIN_LIGHT) evaluates n (n - 1) / 2 pairs, each with the reaction on the source added.  With
-    the far expansion the pair kernel takes the partners n <= 1 only (the
-    far ones are O(n) work in FP64, outside this count)."""
+    evaluation of n particles with image charges: the gather form evaluates
+    n (n - 1) ordered pairs; the pair-symmetric form (mixed, n >= SYM_MIN or
+    SYM_MIN_LIGHT; FP64, n >= SYM_MIN_FP64) n (n - 1) / 2 pairs, each with the
+    reaction on the source added.  With the far expansion the pair kernel takes
+    the partners n <= 1 only (the far ones are O(n) work in FP64, outside this
+    count)."""
     nic = min(n_ic_max, 1) if (precision == "mixed" and far_expansion) else n_ic_max
-    if precision == "mixed" and n >= (SYM_MIN if nic > 0 else SYM_MIN_LIGHT):
+    least = SYM_MIN_FP64 if precision != "mixed" else SYM_MIN if nic > 0 else SYM_MIN_LIGHT
+    if n >= least:
         return n * (n - 1) // 2 * (pair_flops(nic) + SYM_REACTION_FLOPS)
     return n * (n - 1) * pair_flops(nic)
 
