@@ -1992,7 +1992,7 @@ static int run_jumps(rd_ctx* c, const std::vector<Ent>& in, int C, int precision
       const unsigned char* b = (const unsigned char*)v;
       key.insert(key.end(), b, b + bytes);
     };
-    const int ints[] = {ne, nwg, (int)any_planar, (int)any_tip, (int)fp64, maxndim, C};
+    const int ints[] = {ne, nwg, (int)any_planar, (int)any_tip, (int)kind, maxndim, C};
     const void* ptrs[] = {dt, dall, c->d_desc, c->d_state, c->d_wf};
     a.it0 = 1;
     a.it1 = maxndim + 1;
