@@ -259,15 +259,15 @@ __device__ __forceinline__ void surface_far_coeffs(double q, double zb, double w
   c1 = make_float4(c[4], c[5], c[6], c[7]);
 }
 
-// acc + q sum_{m >= 1} a_m t^m, t = s / d^2 (a_0 is the same for every target).
-__device__ __forceinline__ float surface_far_acc(float t, float4 c0, float4 c1, float acc) {
+// q sum_m a_m t^m, t = s / d^2.
+__device__ __forceinline__ float surface_far_eval(float t, float4 c0, float4 c1) {
   float v = __builtin_fmaf(c1.w, t, c1.z);
   v = __builtin_fmaf(v, t, c1.y);
   v = __builtin_fmaf(v, t, c1.x);
   v = __builtin_fmaf(v, t, c0.w);
   v = __builtin_fmaf(v, t, c0.z);
   v = __builtin_fmaf(v, t, c0.y);
-  return __builtin_fmaf(v, t, acc);
+  return __builtin_fmaf(v, t, c0.x);
 }
 
 // q_j/q_0 times surface_sum32 for the packed target (h1, l1) on the cathode
@@ -284,19 +284,20 @@ __device__ __forceinline__ float surface_term32(const float4 h1, const float4 l1
 // The sums over the sources of a target on the cathode: terms in FP32, in blocks
 // of at most kSurfBlock, block sums in FP64.  Every term q z_b / r^3 of a block has
 // the sign of the charges (z_b >= 0, one species), so a block's FP32 sum is within
-// (kSurfBlock - 1) u = 15 * 2^-24 (< 1e-6) of its exact value; so have the far
-// series' terms beyond a_0: their sum over k != 0, negative, rises towards 0 with
-// s.  Per source a block saves the conversion and the FP64 add.
+// (kSurfBlock - 1) u = 15 * 2^-24 (< 1e-6) of its exact value; so has the
+// paired-image sum of a source with N_ic_max > 0 (positive for every z_b in (0, d),
+// rho and N_ic_max: the terms n and -n-1 pair off).  Per source a block saves the
+// conversion and the FP64 add.
 constexpr int kSurfBlock = 16;
 
-// acc + q z_b / r^3 of one source at the target t = (x, y, x_lo, y_lo): xy = (x, y,
-// x_lo, y_lo), zq = (z^2, q z); s receives the squared lateral distance.
-__device__ __forceinline__ float surface_acc32(float4 t, float4 xy, float2 zq, float& s,
-                                               float acc) {
+// base + q z_b / r^3 of one source at the target t = (x, y, x_lo, y_lo): xy = (x, y,
+// x_lo, y_lo), zq = (z^2, q z), base(s) of the squared lateral distance s.
+template <class B>
+__device__ __forceinline__ float surface_term32(float4 t, float4 xy, float2 zq, B&& base) {
   const float dx = (t.x - xy.x) + (t.z - xy.z), dy = (t.y - xy.y) + (t.w - xy.w);
-  s = __builtin_fmaf(dy, dy, dx * dx);
+  const float s = __builtin_fmaf(dy, dy, dx * dx);
   const float ri = rsq(s + zq.x);
-  return __builtin_fmaf(zq.y, ri * ri * ri, acc);
+  return __builtin_fmaf(zq.y, ri * ri * ri, base(s));
 }
 
 // True when every active target of the wavefront lies on the plane z = 0 and
@@ -470,14 +471,16 @@ __device__ __forceinline__ double surface_chunk32(float4 t1, const float4* sxy, 
   double f = 0.0;
   for (int jb = 0; jb < cnt; jb += kSurfBlock) {
     const int je = min(cnt, jb + kSurfBlock);
-    float acc = 0.f, s;
+    float acc = 0.f;
 #pragma unroll 4
     for (int jj = jb; jj < je; ++jj) {
-      acc = surface_acc32(t1, sxy[jj], szq[jj], s, acc);
-      // the coefficients through the scalar cache, beside the LDS reads
-      if (FAR)
-        acc = surface_far_acc(s * inv_d2, load_uniform(far, 2 * jj), load_uniform(far, 2 * jj + 1),
-                              acc);
+      if (FAR)  // the coefficients through the scalar cache, beside the LDS reads
+        acc += surface_term32(t1, sxy[jj], szq[jj], [&](float s) {
+          return surface_far_eval(s * inv_d2, load_uniform(far, 2 * jj),
+                                  load_uniform(far, 2 * jj + 1));
+        });
+      else
+        acc = surface_term32(t1, sxy[jj], szq[jj], [&](float) { return acc; });
     }
     f += (double)acc;
   }
@@ -509,12 +512,12 @@ __device__ __forceinline__ void add_quarters(void* lds, double& fx, double& fy, 
 // of chunks [c0, c1) at the packed target (h1, l1); split: of this wavefront's
 // quarters of them.
 //
-// On the cathode the pair terms are bound by VALU issue (the far series 21
+// On the cathode the pair terms are bound by VALU issue (the far series 22
 // instructions a pair, without 11; two or four targets per lane, which halve and
 // quarter the LDS and scalar reads, measured the same).  65 536 electrons at 256
-// x 256 points: 2.02 -> 1.81 ms with the far series, 1.37 -> 1.12 without, by terms
-// without a product or an addition of their own (charge and a_0 taken out of the
-// series, z^2 and q z formed at staging).
+// x 256 points: 2.02 -> 1.87 ms with the far series, 1.37 -> 1.18 without, by terms
+// without products or additions of their own (charge in the series, z^2 and q z
+// formed at staging, the direct term added by the product).
 __device__ __forceinline__ void field_seg32(const DevGeom& g, bool split, bool act, float4 h1,
                                             float4 l1,
                                             const float4* __restrict__ hi,
@@ -540,7 +543,6 @@ __device__ __forceinline__ void field_seg32(const DevGeom& g, bool split, bool a
                  act ? -h1.y : 3e38f};  // min x, -max x, min y, -max y
   if (boxes) wave_min4(tb);
   __shared__ float sbox[4][kBlock / 64];
-  __shared__ double sa0[kBlock / 64];  // far series: the chunk's sum of q a_0
   fx = 0.0;
   fy = 0.0;
   fz = 0.0;
@@ -548,7 +550,6 @@ __device__ __forceinline__ void field_seg32(const DevGeom& g, bool split, bool a
     const int jb = c * kChunk;
     __syncthreads();
     float sb[4] = {3e38f, 3e38f, 3e38f, 3e38f};
-    double a0 = 0.0;
     if (jb + t < n) {
       const float4 hv = hi[jb + t], lv = lo[jb + t];
       shi[t] = hv;
@@ -556,10 +557,8 @@ __device__ __forceinline__ void field_seg32(const DevGeom& g, bool split, bool a
       sxy[t] = make_float4(hv.x, hv.y, lv.x, lv.y);
       szq[t] = make_float2(fmaxf(hv.z * hv.z, kR2Min), hv.w * hv.z);
       if (boxes) {
-        const float4 cv = far[2 * (jb + t)];
-        sfar[2 * t] = cv;
+        sfar[2 * t] = far[2 * (jb + t)];
         sfar[2 * t + 1] = far[2 * (jb + t) + 1];
-        a0 = (double)cv.x;
       }
       sb[0] = hv.x;
       sb[1] = -hv.x;
@@ -568,19 +567,14 @@ __device__ __forceinline__ void field_seg32(const DevGeom& g, bool split, bool a
     }
     if (boxes) {
       wave_min4(sb);
-      for (int o = 32; o > 0; o >>= 1) a0 += __shfl_xor(a0, o);
-      if ((t & 63) == 0) {
+      if ((t & 63) == 0)
         for (int q = 0; q < 4; ++q) sbox[q][t >> 6] = sb[q];
-        sa0[t >> 6] = a0;
-      }
     }
     __syncthreads();
     const ChunkPart part(split, wv, min(kChunk, n - jb));
     const int pc = part.j1 - part.j0;
     bool inside = false;
     if (boxes) {
-      a0 = 0.0;
-      for (int u = 0; u < kBlock / 64; ++u) a0 += sa0[u];
       for (int q = 0; q < 4; ++q) {
         sb[q] = sbox[q][0];
         for (int u = 1; u < kBlock / 64; ++u) sb[q] = fminf(sb[q], sbox[q][u]);
@@ -595,21 +589,17 @@ __device__ __forceinline__ void field_seg32(const DevGeom& g, bool split, bool a
     if (surf && !boxes) {  // N_ic_max = 0; fz: without the factor -2 until the end
       fz += surface_chunk32<false>(t1, sxy + part.j0, szq + part.j0, nullptr, pc, inv_d2);
     } else if (surf && inside) {
-      if (split && wv > 0) a0 = 0.0;  // the chunk's, once
-      fz += a0 + surface_chunk32<true>(t1, sxy + part.j0, szq + part.j0, far + 2 * (jb + part.j0), pc,
+      fz += surface_chunk32<true>(t1, sxy + part.j0, szq + part.j0, far + 2 * (jb + part.j0), pc,
                                        inv_d2);
     } else if (surf) {
       for (int jb2 = part.j0; jb2 < part.j1; jb2 += kSurfBlock) {
         const int je2 = min(part.j1, jb2 + kSurfBlock);
-        float acc = 0.f, s;
-        for (int jj = jb2; jj < je2; ++jj) {
-          acc = surface_acc32(t1, sxy[jj], szq[jj], s, acc);
-          if (s <= slim)
-            acc += surface_far_acc(s * inv_d2, sfar[2 * jj], sfar[2 * jj + 1], sfar[2 * jj].x);
-          else
-            acc = __builtin_fmaf(shi[jj].w, surface_far32(shi[jj].z, slo[jj].w, s, nic, dnm, 0.f),
-                                 acc);
-        }
+        float acc = 0.f;
+        for (int jj = jb2; jj < je2; ++jj)
+          acc += surface_term32(t1, sxy[jj], szq[jj], [&](float s) {
+            if (s <= slim) return surface_far_eval(s * inv_d2, sfar[2 * jj], sfar[2 * jj + 1]);
+            return shi[jj].w * surface_far32(shi[jj].z, slo[jj].w, s, nic, dnm, 0.f);
+          });
         fz += (double)acc;
       }
     } else if (act) {

@@ -439,7 +439,7 @@ struct HeldSrc {
 
 // N_ic_max = 0 (planar, image charge on): sums of q z / r^3 at T chains' points
 // over this lane's particles of slice w; FP32 blocks of at most kSurfBlock
-// terms of one sign (see surface_acc32), block sums in FP64.  The offsets are
+// terms of one sign (see kSurfBlock), block sums in FP64.  The offsets are
 // FP64 differences rounded to FP32: two instructions where the difference of
 // two-part FP32 coordinates takes three, and exact before the rounding.  HELD:
 // the particles are in `own`.

@@ -65,7 +65,7 @@ __device__ __forceinline__ Tile tile_of(const Ent* tab, int ne, bool points, int
 // image term 88 / 55, 2861 of the tip 113 / 70, 11 000 174 / 157; the field at 777
 // points over 2861, tip 99 / 67, ten image terms 296 / 114; 5000 over 8000 161 /
 // 146.  On the cathode, where a pair takes 11 to 21 instructions, the staging of
-// the sources shows from 8000 wavefronts on: kernel 1.81 / 2.39 ms at 256 x 256
+// the sources shows from 8000 wavefronts on: kernel 1.87 / 2.39 ms at 256 x 256
 // points over 65 536, equal at 40 x 40 over 37 409 (3675 wavefronts).
 constexpr int kSplitWaves = 4096;  // most wavefronts of a planar field that shares
 struct Targets32 {
