@@ -1092,6 +1092,18 @@ int rd_set_solo_jumps(rd_ctx* c, int32_t on) {
   return RD_OK;
 }
 
+int rd_set_jump_wait(rd_ctx* c, int64_t nanoseconds) {
+  if (!c) return fail(RD_ERR_ARG, "null context");
+  c->jump_wait = nanoseconds < 0 ? -1 : nanoseconds / 10;
+  return RD_OK;
+}
+
+int rd_jump_repeats(rd_ctx* c, int64_t* steps) {
+  if (!c || !steps) return fail(RD_ERR_ARG, "null argument");
+  *steps = c->jump_repeats;
+  return RD_OK;
+}
+
 int rd_time_copy(rd_ctx* c, int64_t bytes, int32_t reps, double* kernel_ms) {
   if (!c) return fail(RD_ERR_ARG, "null context");
   if (bytes < 16 || bytes % 16 != 0 || bytes > (int64_t(1) << 34))

@@ -1939,6 +1939,7 @@ static int run_jumps(rd_ctx* c, const std::vector<Ent>& in, int C, int precision
   }
   a.C = C;
   a.fits = nwg <= room;
+  a.wait = c->jump_wait;
   const size_t nr = (size_t)maxndim * C;
   r = ensure(c, c->rnd, sizeof(double) * 3 * nr);
   if (r) return r;
@@ -2042,6 +2043,7 @@ static int run_jumps(rd_ctx* c, const std::vector<Ent>& in, int C, int precision
   RD_HIP(hipMemcpyAsync(c->h_stop, a.stop, sizeof(int), hipMemcpyDeviceToHost, c->stream));
   RD_HIP(hipStreamSynchronize(c->stream));
   if (*c->h_stop) {
+    ++c->jump_repeats;
     random();
     one_by_one();
     RD_HIP(hipGetLastError());

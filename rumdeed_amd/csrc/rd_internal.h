@@ -256,6 +256,8 @@ struct rd_ctx {
   int jump_room[4] = {};       // resident jump workgroups per form; 0: not asked yet
   bool solo_jumps = true;      // all jumps of a step in one launch (rd_set_solo_jumps)
   int* h_stop = nullptr;       // pinned: a jump workgroup's wait gave up
+  long long jump_wait = -1;    // bound of its waits, ticks of 10 ns; negative: the default
+  int64_t jump_repeats = 0;    // steps whose jumps were repeated after that
   std::vector<unsigned char> jump_key;
 };
 

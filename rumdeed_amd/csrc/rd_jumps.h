@@ -88,6 +88,7 @@ struct JumpArgs {
   int it0, it1;                   // jumps it0 .. it1 - 1 of this launch
   int spin;                       // 1: all jumps in this launch; 0: a launch per jump
   int fits;                       // all workgroups of the launch can be resident at once
+  long long wait;                 // bound of the waits (ticks); negative: the default
 };
 
 // Per entry: the width and rate of the jumps of either parity (a launch per
@@ -248,6 +249,7 @@ struct JumpWidth {
   int first, fe;
   unsigned long long* w;  // counter words of jump 1
   int words, groups, grp, spin, fits;
+  long long wait;
   int* stop;
   double* slot;
   long long t0 = wall_clock64();
@@ -256,7 +258,7 @@ struct JumpWidth {
                                        const JumpArgs& a, int grp_)
       : mh(S.MH_std), rate(S.a_rate), first(nint(s.ndim * 0.25)),
         fe(s.mode == RD_EMIT_PLANAR_FE), w(a.cnt + e.part_off), words(e.pslots), groups(e.segs),
-        grp(grp_), spin(a.spin), fits(a.fits), stop(a.stop),
+        grp(grp_), spin(a.spin), fits(a.fits), wait(a.wait), stop(a.stop),
         slot(a.width + (size_t)kWidthSlots * e.acc_off) {
     if (fe && !spin && a.it0 >= 2) {  // as the launch of the jump before left it
       mh = slot[(a.it0 - 1) & 1];
@@ -266,8 +268,9 @@ struct JumpWidth {
   // The width after jump `it`.
   __device__ __forceinline__ bool after(int it) {
     if (groups > 1 || !spin) {
-      const long long ticks =
-          it == 1 && fits ? kFirstTicks + 4 * (wall_clock64() - t0) : kSpinTicks;
+      const long long ticks = wait >= 0          ? wait
+                              : it == 1 && fits ? kFirstTicks + 4 * (wall_clock64() - t0)
+                                                : kSpinTicks;
       if (!counts_wait(w + (size_t)(it - 1) * words, groups, spin, stop, ticks, na, nr))
         return false;
     }

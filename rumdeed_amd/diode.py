@@ -143,6 +143,18 @@ class Diode:
         results are identical (rd_set_solo_jumps)."""
         check(self._lib.rd_set_solo_jumps(self._h, int(bool(on))))
 
+    def set_jump_wait(self, nanoseconds: int = -1):
+        """Bound of a jump workgroup's waits for the others (rd_set_jump_wait;
+        negative: the default)."""
+        check(self._lib.rd_set_jump_wait(self._h, int(nanoseconds)))
+
+    def jump_repeats(self) -> int:
+        """Steps whose jumps were repeated with a launch per jump after a wait
+        passed its bound (rd_jump_repeats)."""
+        v = ctypes.c_int64()
+        check(self._lib.rd_jump_repeats(self._h, ctypes.byref(v)))
+        return v.value
+
     def set_seed(self, seed: int, stream: int = 0):
         check(self._lib.rd_set_seed(self._h, int(seed), int(stream)))
 
