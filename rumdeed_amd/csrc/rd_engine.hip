@@ -36,6 +36,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <cstring>
 #include <type_traits>
 
@@ -1808,15 +1809,17 @@ static int reset_counters(rd_ctx* c, const std::vector<Ent>& ents) {
 // Forms of the jump kernels: FP64; mixed, a lone simulation of few or many
 // particles, a pool (JumpForm).
 enum JumpKind { kJumpFp64, kJumpLone, kJumpMany, kJumpPool, kJumpKinds };
-static_assert(kJumpKinds == sizeof(rd_ctx::jump_room) / sizeof(int), "a room per form");
+static_assert(3 * kJumpKinds == sizeof(rd_ctx::jump_room) / sizeof(int), "one per kernel");
 
-// Instructions of one chain's pair terms per SIMD and jump over n particles.
+// Instructions of one chain's pair terms per SIMD and jump over n particles; of the
+// mixed planar forms as measured against each other (20 000 electrons, 24 chains a
+// workgroup, us a jump: N_ic_max = 0 55, 1 110, 10 433; without images 94 for 32).
 static double jump_work(const DevGeom& g, JumpKind kind, int n) {
   const int waves = kind == kJumpMany ? 16 : 4;  // slices: the wavefronts a chain is spread over
   const double rounds = std::max(1, (n + 64 * waves - 1) / (64 * waves)) * (waves / 4);
   if (g.kind == RD_GEOM_TIP) return rounds * (kind == kJumpFp64 ? 160.0 : 50.0);
   if (kind == kJumpFp64) return rounds * 40.0 * (g.ic ? 1 + 2 * g.nic : 1);
-  return rounds * (g.ic ? 12.0 + 20.0 * g.nic : 25.0);
+  return rounds * (g.ic ? 12.0 + 10.0 * g.nic : 17.0);
 }
 
 // Chains a workgroup of the jump kernels takes for an entry of m chains: about
@@ -1860,35 +1863,48 @@ static int run_jumps(rd_ctx* c, const std::vector<Ent>& in, int C, int precision
   a.LO = (const float4*)c->pack_lo.p;
   a.SRX = (const double2*)c->pack_srx.p;
   a.SRZ = (const float2*)c->pack_srz.p;
-  bool any_planar = false, any_tip = false;
-  for (const Ent& e : ents)
-    (c->slots[e.slot].desc.g.kind == RD_GEOM_TIP ? any_tip : any_planar) = true;
+  bool any[3] = {};  // the kernels of JumpForms the entries take
+  for (const Ent& e : ents) {
+    const DevGeom& g = c->slots[e.slot].desc.g;
+    any[g.kind == RD_GEOM_TIP ? 2 : jump_series(g) ? 1 : 0] = true;
+  }
   const JumpKind kind = fp64                  ? kJumpFp64
                         : c->nslots_max > 1   ? kJumpPool
                         : ents[0].n_ub < kJumpLarge ? kJumpLone
                                                     : kJumpMany;
   using Kernel = void (*)(const Ent*, int, const SimDesc*, const SimState*, const double*, Chains,
                           Chains, JumpArgs);
+  // cathode with N_ic_max = 0 (FP64: planar), other planar forms (mixed), tip
   static const struct {
-    Kernel planar, tip;
+    Kernel k[3];
     int threads;
   } forms[kJumpKinds] = {
-      {k_mh_jumps64<RD_GEOM_PLANAR>, k_mh_jumps64<RD_GEOM_TIP>, kJump64Threads},
-      {k_mh_jumps32<RD_GEOM_PLANAR, LoneForm>, k_mh_jumps32<RD_GEOM_TIP, LoneForm>,
-       64 * LoneForm::kWaves},
-      {k_mh_jumps32<RD_GEOM_PLANAR, LargeForm>, k_mh_jumps32<RD_GEOM_TIP, LargeForm>,
-       64 * LargeForm::kWaves},
-      {k_mh_jumps32<RD_GEOM_PLANAR, PoolForm>, k_mh_jumps32<RD_GEOM_TIP, PoolForm>,
-       64 * PoolForm::kWaves}};
+      {{k_mh_jumps64<RD_GEOM_PLANAR>, k_mh_jumps64<RD_GEOM_PLANAR>, k_mh_jumps64<RD_GEOM_TIP>},
+       kJump64Threads},
+#define RD_JUMPS32(FORM)                                                                   \
+  {                                                                                        \
+    {k_mh_jumps32<RD_GEOM_PLANAR, false, FORM>, k_mh_jumps32<RD_GEOM_PLANAR, true, FORM>, \
+     k_mh_jumps32<RD_GEOM_TIP, false, FORM>},                                              \
+        64 * FORM::kWaves                                                                  \
+  }
+      RD_JUMPS32(LoneForm), RD_JUMPS32(LargeForm), RD_JUMPS32(PoolForm)};
+#undef RD_JUMPS32
   const auto& form = forms[kind];
-  // workgroups that can be resident at once
-  int& room = c->jump_room[kind];
-  if (room == 0) {
-    int cus = 0, p = 0, q = 0;
+  if (fp64) {  // one planar kernel
+    any[0] |= any[1];
+    any[1] = false;
+  }
+  // workgroups of the kernels taken that can be resident at once
+  int& cus = c->cus;
+  if (cus == 0)
     RD_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device));
-    RD_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&p, form.planar, form.threads, 0));
-    RD_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&q, form.tip, form.threads, 0));
-    room = std::max(1, cus * std::min(p, q));
+  int room = INT_MAX;
+  for (int k = 0; k < 3; ++k) {
+    if (!any[k]) continue;
+    int& per_cu = c->jump_room[kind][k];
+    if (per_cu == 0)
+      RD_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, form.k[k], form.threads, 0));
+    room = std::min(room, std::max(1, cus * per_cu));
   }
   // The largest first, so that their workgroups start together and the small
   // simulations fill up behind them.
@@ -1967,12 +1983,10 @@ static int run_jumps(rd_ctx* c, const std::vector<Ent>& in, int C, int precision
     a.it0 = it0;
     a.it1 = it1;
     a.spin = sp;
-    if (any_planar)
-      form.planar<<<nwg, form.threads, 0, c->stream>>>(dt, ne, c->d_desc, c->d_state, c->d_wf,
+    for (int k = 0; k < 3; ++k)
+      if (any[k])
+        form.k[k]<<<nwg, form.threads, 0, c->stream>>>(dt, ne, c->d_desc, c->d_state, c->d_wf,
                                                        from, R, a);
-    if (any_tip)
-      form.tip<<<nwg, form.threads, 0, c->stream>>>(dt, ne, c->d_desc, c->d_state, c->d_wf, from,
-                                                    R, a);
   };
   auto one_by_one = [&]() {
     for (int it = 1; it <= maxndim + 1; ++it) jumps(it == 1 ? V : R, it, it + 1, false);
@@ -1993,7 +2007,7 @@ static int run_jumps(rd_ctx* c, const std::vector<Ent>& in, int C, int precision
       const unsigned char* b = (const unsigned char*)v;
       key.insert(key.end(), b, b + bytes);
     };
-    const int ints[] = {ne, nwg, (int)any_planar, (int)any_tip, (int)kind, maxndim, C};
+    const int ints[] = {ne, nwg, any[0], any[1], any[2], (int)kind, maxndim, C};
     const void* ptrs[] = {dt, dall, c->d_desc, c->d_state, c->d_wf};
     a.it0 = 1;
     a.it1 = maxndim + 1;

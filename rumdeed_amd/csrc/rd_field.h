@@ -186,9 +186,10 @@ __device__ __forceinline__ void ic_planar32(float zsum, float wsum, float dzab, 
 //   cz = -2 sum_{k=-nic..nic} u_k / (dxy2 + u_k^2)^(3/2),  u_k = z_b + 2kd,
 //   cxy = 0,
 // the same series as ic_planar32 plus the direct term, with 2 nic + 1 distances
-// instead of 4 nic + 2.  surface_sum32 returns the sum without the factor -2,
-// which the callers apply once to their FP64 total (exactly: a power of two).
-// zb = z_b, wb = d - z_b and dnm = d (nm); the partners below the cathode are
+// instead of 4 nic + 2.  The kernels sum without the factor -2 and apply it
+// once to their FP64 total (exactly: a power of two).  zb = z_b, wb = d - z_b and
+// dnm = d (nm); the source height is its high part alone (the float sum of both
+// parts rounds to it but for ties), and the partners below the cathode are
 // formed from wb, as ic_planar32 forms the anode image.
 // surface_far32: w plus the partners k != 0 of that series, one by one.
 __device__ __forceinline__ float surface_far32(float zb, float wb, float dxy2, int nic, float dnm,
@@ -206,13 +207,6 @@ __device__ __forceinline__ float surface_far32(float zb, float wb, float dxy2, i
     um -= two_d;
   }
   return w;
-}
-
-__device__ __forceinline__ float surface_sum32(float zb, float wb, float dxy2, int nic,
-                                               float dnm) {
-  float r2 = fmaxf(__builtin_fmaf(zb, zb, dxy2), kR2Min);
-  float ri = rsq(r2);
-  return surface_far32(zb, wb, dxy2, nic, dnm, zb * (ri * ri * ri));
 }
 
 // The partners k != 0 of the series above as a power series in s = dxy2.
@@ -268,17 +262,6 @@ __device__ __forceinline__ float surface_far_eval(float t, float4 c0, float4 c1)
   v = __builtin_fmaf(v, t, c0.z);
   v = __builtin_fmaf(v, t, c0.y);
   return __builtin_fmaf(v, t, c0.x);
-}
-
-// q_j/q_0 times surface_sum32 for the packed target (h1, l1) on the cathode
-// and the packed source (h2, l2).  The source height is its high part alone
-// (the float sum of both parts rounds to it but for ties).
-__device__ __forceinline__ float surface_term32(const float4 h1, const float4 l1, const float4 h2,
-                                                const float4 l2, int nic, float dnm) {
-  const float dx = (h1.x - h2.x) + (l1.x - l2.x);
-  const float dy = (h1.y - h2.y) + (l1.y - l2.y);
-  const float dxy2 = __builtin_fmaf(dy, dy, dx * dx);
-  return h2.w * surface_sum32(h2.z, l2.w, dxy2, nic, dnm);
 }
 
 // The sums over the sources of a target on the cathode: terms in FP32, in blocks

@@ -253,7 +253,8 @@ struct rd_ctx {
   // while they are unchanged.
   int graphs = 0;
   hipGraphExec_t jump_exec = nullptr;
-  int jump_room[4] = {};       // resident jump workgroups per form; 0: not asked yet
+  int cus = 0;                 // compute units; 0: not asked yet
+  int jump_room[4][3] = {};    // workgroups of each jump kernel a CU holds; 0: not asked yet
   bool solo_jumps = true;      // all jumps of a step in one launch (rd_set_solo_jumps)
   int* h_stop = nullptr;       // pinned: a jump workgroup's wait gave up
   long long jump_wait = -1;    // bound of its waits, ticks of 10 ns; negative: the default

@@ -524,40 +524,80 @@ __device__ __forceinline__ void jump_surf0(const HeldSrc<Form>& own, const doubl
 }
 
 // Other planar forms, on the cathode with N_ic_max > 0 (-1/2 of the field sum,
-// as surface_sum32) or without image charges: FP32 terms, FP64 sums.
-template <class Form, int T>
-__device__ __forceinline__ void jump_planar(int ic, int nic, float dnm, const float4* hi,
+// the series of surface_far32) or without image charges: FP32 terms, FP64 sums.  The next
+// round's particle is in flight during a round, and the chains go through the
+// image series side by side: they share the partners' heights, and their
+// dependent operations overlap (a partner is a square root and three products in
+// sequence).  Large simulations take eight chains a pass, which halves the reads
+// of the particles.
+template <class Form, int T, bool IC>
+__device__ __forceinline__ void jump_planar(int nic, float dnm, const float4* hi,
                                             const float4* lo, int n, int w, int lane,
                                             const double2* tgt, double (&d)[T]) {
-  float4 h1[T], l1[T];
+  float hx[T], hy[T], lx[T], ly[T];
 #pragma unroll
   for (int u = 0; u < T; ++u) {
-    float4 p;
-    split(tgt[u].x, p.x, p.z);
-    split(tgt[u].y, p.y, p.w);
-    h1[u] = make_float4(uniform_f(p.x), uniform_f(p.y), 0.0f, 0.0f);
-    l1[u] = make_float4(uniform_f(p.z), uniform_f(p.w), 0.0f, 0.0f);
+    split(tgt[u].x, hx[u], lx[u]);
+    split(tgt[u].y, hy[u], ly[u]);
+    hx[u] = uniform_f(hx[u]);
+    hy[u] = uniform_f(hy[u]);
+    lx[u] = uniform_f(lx[u]);
+    ly[u] = uniform_f(ly[u]);
     d[u] = 0.0;
   }
   const int R = jump_rounds<Form>(n);
+  float4 hn = make_float4(0, 0, 0, 0), ln = hn;
+  if (w * 64 + lane < n) {
+    hn = hi[w * 64 + lane];
+    ln = lo[w * 64 + lane];
+  }
 #pragma unroll 1
   for (int r = 0; r < R; ++r) {
-    const int j = r * Form::kRound + w * 64 + lane;
-    if (j >= n) continue;
-    const float4 h2 = hi[j], l2 = lo[j];
+    const float4 h2 = hn, l2 = ln;
+    const int j = (r + 1) * Form::kRound + w * 64 + lane;
+    if (r + 1 < R) {  // the next round's particle
+      const int i = j < n ? j : 0;
+      hn = hi[i];
+      ln = lo[i];
+    }
+    const float q = j - Form::kRound < n ? h2.w : 0.0f;  // padding has no charge
+    float s[T], f[T];
 #pragma unroll
     for (int u = 0; u < T; ++u) {
-      if (ic) {
-        d[u] += (double)surface_term32(h1[u], l1[u], h2, l2, nic, dnm);
-      } else {
-        const float dx = (h1[u].x - h2.x) + (l1[u].x - l2.x);
-        const float dy = (h1[u].y - h2.y) + (l1[u].y - l2.y);
-        const float dz = -h2.z - l2.z;
-        const float r2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
-        const float ri = rsq(fmaxf(r2, kR2Min));
-        d[u] += (double)(h2.w * (dz * (ri * ri * ri)));
+      const float dx = (hx[u] - h2.x) + (lx[u] - l2.x);
+      const float dy = (hy[u] - h2.y) + (ly[u] - l2.y);
+      s[u] = lateral2(dx, dy);
+    }
+    if (IC) {  // surface_far32 of every chain
+#pragma unroll
+      for (int u = 0; u < T; ++u) {
+        const float ri = rsq(__builtin_fmaf(h2.z, h2.z, s[u]));
+        f[u] = h2.z * (ri * ri * ri);
+      }
+      const float two_d = dnm + dnm;
+      float up = h2.z, um = -(l2.w + dnm);
+#pragma unroll 1
+      for (int k = 1; k <= nic; ++k) {
+        up += two_d;
+#pragma unroll
+        for (int u = 0; u < T; ++u) {
+          float ri = rsq(__builtin_fmaf(up, up, s[u]));
+          f[u] = __builtin_fmaf(up, ri * ri * ri, f[u]);
+          ri = rsq(__builtin_fmaf(um, um, s[u]));
+          f[u] = __builtin_fmaf(um, ri * ri * ri, f[u]);
+        }
+        um -= two_d;
+      }
+    } else {
+      const float dz = -h2.z - l2.z;
+#pragma unroll
+      for (int u = 0; u < T; ++u) {
+        const float ri = rsq(__builtin_fmaf(dz, dz, s[u]));
+        f[u] = dz * (ri * ri * ri);
       }
     }
+#pragma unroll
+    for (int u = 0; u < T; ++u) d[u] += (double)(q * f[u]);
   }
 }
 
@@ -626,12 +666,18 @@ __device__ __forceinline__ void jump_passes(int nc, int ng, int g, F&& pass) {
     run(std::integral_constant<int, 1>{});
 }
 
-template <int KIND, class Form>
+// SERIES: the planar forms of jump_planar, in a kernel of their own: neither's
+// registers crowd the other's, and without the held particles the compute units
+// hold more of its workgroups.
+__host__ __device__ inline bool jump_series(const DevGeom& g) {
+  return g.kind == RD_GEOM_PLANAR && !(g.ic && g.nic == 0);
+}
+template <int KIND, bool SERIES, class Form>
 __global__ __launch_bounds__(64 * Form::kWaves, Form::kOccupancy) void k_mh_jumps32(
     const Ent* tab, int ne, const SimDesc* desc, const SimState* st, const double* wf, Chains in,
     Chains out, JumpArgs a) {
   constexpr int WAVES = Form::kWaves, kJumpSlices = Form::kSlices;
-  constexpr bool kTip = KIND == RD_GEOM_TIP;
+  constexpr bool kTip = KIND == RD_GEOM_TIP, kSurf0 = !kTip && !SERIES;
   __shared__ float4 tgt[kTip ? 4 : 1][kTip ? kJumpLanes : 1];
   __shared__ double2 tgt2[kTip ? 1 : kJumpLanes];  // planar: x, y (nm)
   __shared__ double red[kTip ? 3 : 1][kJumpSlices][kJumpLanes];
@@ -640,7 +686,7 @@ __global__ __launch_bounds__(64 * Form::kWaves, Form::kOccupancy) void k_mh_jump
   __shared__ ChainStore store;
   const Ent e = tab[find_entry(tab, ne, blockIdx.x)];
   const SimDesc s = desc[e.slot];  // a copy: references would be read again after every barrier
-  if (s.g.kind != KIND) return;
+  if (s.g.kind != KIND || jump_series(s.g) != SERIES) return;
   const DevGeom& g = s.g;
   const int t = threadIdx.x, lane = t & 63;
   const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -672,10 +718,9 @@ __global__ __launch_bounds__(64 * Form::kWaves, Form::kOccupancy) void k_mh_jump
   const int ic = g.ic, nic = g.nic;
   const float dnm = 0.5f * (float)(2.0 * g.d * 1e9);
   const float kt = g.ic ? (float)g.ktip : 0.0f;
-  const bool surf0 = !kTip && ic && nic == 0;
   // few particles stay in LDS for all jumps (padding: no charge)
   const int padded = jump_rounds<Form>(n) * Form::kRound;
-  const bool held = surf0 && padded <= Form::kHeld;
+  const bool held = kSurf0 && padded <= Form::kHeld;
   if (held)
     for (int j = t; j < padded; j += 64 * WAVES) {
       own[0].xy[j] = srx[j < n ? j : 0];
@@ -734,7 +779,7 @@ __global__ __launch_bounds__(64 * Form::kWaves, Form::kOccupancy) void k_mh_jump
           red[kTip ? 2 : 0][w][k] = vz;
         }
       });
-    } else if (surf0) {
+    } else if (kSurf0) {
       jump_passes<8>(nc, NG, group, [&](auto tt, int tb) {
         constexpr int T = decltype(tt)::value;
         double d[T];
@@ -746,10 +791,13 @@ __global__ __launch_bounds__(64 * Form::kWaves, Form::kOccupancy) void k_mh_jump
         if ((lane & 7) == 0) red[0][w][tb + wave_slot<T>(lane)] = v;
       });
     } else {
-      jump_passes<4>(nc, NG, group, [&](auto tt, int tb) {
+      jump_passes<8>(nc, NG, group, [&](auto tt, int tb) {
         constexpr int T = decltype(tt)::value;
         double d[T];
-        jump_planar<Form, T>(ic, nic, dnm, hi, lo, n, w, lane, &tgt2[tb], d);
+        if (ic)
+          jump_planar<Form, T, true>(nic, dnm, hi, lo, n, w, lane, &tgt2[tb], d);
+        else
+          jump_planar<Form, T, false>(nic, dnm, hi, lo, n, w, lane, &tgt2[tb], d);
         const double v = wave_sums<T>(d, lane);
         if ((lane & 7) == 0) red[0][w][tb + wave_slot<T>(lane)] = v;
       });
