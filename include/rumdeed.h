@@ -292,8 +292,7 @@ int rd_set_jump_pairing(rd_ctx* ctx, int64_t min_workgroups);
 int rd_set_solo_jumps(rd_ctx* ctx, int32_t on);
 
 /* Bound of those waits in nanoseconds (negative, the default: 0.25 s, and in the
- * first jump of a launch whose workgroups all fit the device 2 ms and four times
- * the workgroup's own jump).  A step in which a wait passes its bound, because
+ * first jump 2 ms and eight times the workgroup's own jump).  A step in which a wait passes its bound, because
  * another context's work keeps workgroups off the device, repeats its jumps from
  * their start with a launch per jump, with the same results; a small bound
  * forces that.  Library control, no reference counterpart. */

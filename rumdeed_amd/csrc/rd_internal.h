@@ -182,10 +182,14 @@ struct Slot {
 // Instructions of pair terms per SIMD and jump a jump workgroup aims at, at
 // least (jump_chains).
 constexpr double kJumpTarget = 400.0;
-// Most chains per workgroup with a launch per jump: fewer read the particles
-// more often, more leave CUs idle (85k electrons, 150k chains, ms per step: 8
-// chains 171.9, 16 156.5, 32 150.6, 64 193.4).
+// With a launch per jump: most chains per workgroup (85k electrons, ms per step: 8
+// chains 171.9, 16 156.5, 32 150.6, 64 193.4), and the time a workgroup takes
+// beside its pair terms, in their instructions (about 2.2 ns): workgroups of eight
+// wavefronts overlap with another one, those of sixteen (large lone simulations)
+// have a CU to themselves.  24 diodes of 3400 electrons, us a jump, 8 / 16 / 32
+// chains: N_ic_max = 0 95 / 68 / 62, 1 121 / 103 / 110, 10 374 / 383 / 433.
 constexpr int kJumpApart = 32;
+constexpr double kJumpStart[2] = {1600.0, 4500.0};
 
 // Partial sums of one pair launch are bounded by this many bytes (512 MiB);
 // larger launches run in bands whose partials are folded, in order, into

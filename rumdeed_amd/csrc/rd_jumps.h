@@ -24,17 +24,19 @@
 // chains) 5.4 -> 3.9 ms; thermal-field mixed 5.5 -> 4.8 ms; 64 diodes of a pool
 // mixed 14.0 -> 12.2 ms, FP64 38.7 -> 26.6 ms.
 //
-// Every workgroup of a simulation has to be resident for the wait to end.
-// The host bounds the workgroups of one simulation, and a launch's workgroups
-// start in order, so the earliest unfinished simulation always is, unless
-// another context's work holds the CUs.  The wait is bounded all the same: past
-// its bound the workgroup raises `stop` and leaves; results go to arrays of
-// their own (`out`), so the host then repeats the step's jumps with a launch
-// per jump (spin = 0), where the end of the launch takes the place of the wait,
-// with the same results.  Once the first jump's counts are in, every workgroup
-// is resident, so two contexts that keep each other's workgroups out find that
-// out in the first wait; where all workgroups of the launch fit at once it is
-// short (kFirstTicks and four times the workgroup's own first jump).
+// Every workgroup of a simulation has to be resident for the wait to end, so the
+// host starts workgroups that wait only where the whole launch fits the device,
+// and else a launch per jump (spin = 0), where the end of the launch takes the
+// place of the wait.  (One launch whose later simulations wait for room lost to
+// it: 40 diodes of 3400 electrons, ten image terms, mixed 181 against 129 ms;
+// FP64 1226 against 714, the wait's bound passed.)  Another context's work can
+// still hold the CUs, so the wait is bounded: past its bound the workgroup raises
+// `stop` and leaves; results go to arrays of their own (`out`), and the host
+// repeats the step's jumps with a launch per jump, with the same results.  Once
+// the first jump's counts are in, every workgroup is resident, so two contexts
+// that keep each other's workgroups out find that out in the first wait, which is
+// short (kFirstTicks and eight times the workgroup's own first jump: the
+// workgroups of a simulation differ by one chain, and by their CU's other load).
 //
 // The sums' order depends on the simulation's particle count and the kind of
 // context alone: with S slices, lane l of slice w takes particles
@@ -87,7 +89,6 @@ struct JumpArgs {
   int C;                          // chains in all
   int it0, it1;                   // jumps it0 .. it1 - 1 of this launch
   int spin;                       // 1: all jumps in this launch; 0: a launch per jump
-  int fits;                       // all workgroups of the launch can be resident at once
   long long wait;                 // bound of the waits (ticks); negative: the default
 };
 
@@ -248,7 +249,7 @@ struct JumpWidth {
   int na = 0, nr = 0;
   int first, fe;
   unsigned long long* w;  // counter words of jump 1
-  int words, groups, grp, spin, fits;
+  int words, groups, grp, spin;
   long long wait;
   int* stop;
   double* slot;
@@ -258,7 +259,7 @@ struct JumpWidth {
                                        const JumpArgs& a, int grp_)
       : mh(S.MH_std), rate(S.a_rate), first(nint(s.ndim * 0.25)),
         fe(s.mode == RD_EMIT_PLANAR_FE), w(a.cnt + e.part_off), words(e.pslots), groups(e.segs),
-        grp(grp_), spin(a.spin), fits(a.fits), wait(a.wait), stop(a.stop),
+        grp(grp_), spin(a.spin), wait(a.wait), stop(a.stop),
         slot(a.width + (size_t)kWidthSlots * e.acc_off) {
     if (fe && !spin && a.it0 >= 2) {  // as the launch of the jump before left it
       mh = slot[(a.it0 - 1) & 1];
@@ -268,9 +269,9 @@ struct JumpWidth {
   // The width after jump `it`.
   __device__ __forceinline__ bool after(int it) {
     if (groups > 1 || !spin) {
-      const long long ticks = wait >= 0          ? wait
-                              : it == 1 && fits ? kFirstTicks + 4 * (wall_clock64() - t0)
-                                                : kSpinTicks;
+      const long long ticks = wait >= 0 ? wait
+                              : it == 1 ? kFirstTicks + 8 * (wall_clock64() - t0)
+                                        : kSpinTicks;
       if (!counts_wait(w + (size_t)(it - 1) * words, groups, spin, stop, ticks, na, nr))
         return false;
     }
@@ -425,6 +426,12 @@ __device__ __forceinline__ void store_site(const SimDesc& s, const double* wf, C
 }
 __device__ __forceinline__ SiteTerms stored_site(const ChainStore& m, int k) {
   return SiteTerms{m.d[12][k], m.d[13][k]};
+}
+
+// First chain of a simulation's workgroup: as many for each, but for one, so that
+// no workgroup waits long for the others.
+__device__ __forceinline__ int jump_first(const Ent& e, int grp) {
+  return (int)((long long)grp * e.nch / e.segs);
 }
 
 template <class Form>
@@ -646,24 +653,25 @@ __device__ __forceinline__ void jump_tip(float kt, const float4* hi, const float
   }
 }
 
-// Calls pass(T, first chain) over nc chains dealt to NG groups of wavefronts,
-// group g taking T chains at a time (T a power of two up to TM).
-template <int TM, class F>
-__device__ __forceinline__ void jump_passes(int nc, int ng, int g, F&& pass) {
-  const int q = (nc + ng - 1) / ng;  // chains a group
-  auto run = [&](auto tt) {
-    constexpr int T = decltype(tt)::value;
+// Calls pass(T, first chain) over chains [c0, c1), T at a time: TM, then fewer for
+// the rest.  A rest of five or six takes TM = 8 with idle places where a term is
+// cheap (its reads and set-up count), and 4 + 1 or 4 + 2 where the image series
+// makes it dear (EXACT).
+template <int TM, bool EXACT, class F>
+__device__ __forceinline__ void jump_passes(int c0, int c1, F&& pass) {
+  int tb = c0;
 #pragma unroll 1
-    for (int tb = g * T; tb < nc; tb += ng * T) pass(tt, tb);
-  };
-  if (TM >= 8 && (q > 12 || (q > 4 && q <= 8)))  // 9 .. 12: three passes of four
-    run(std::integral_constant<int, TM>{});
-  else if (q > 2)
-    run(std::integral_constant<int, 4>{});
-  else if (q == 2)
-    run(std::integral_constant<int, 2>{});
-  else
-    run(std::integral_constant<int, 1>{});
+  for (; c1 - tb >= (TM == 8 ? (EXACT ? 7 : 5) : 3); tb += TM)
+    pass(std::integral_constant<int, TM>{}, tb);
+  if (TM == 8 && c1 - tb >= 3) {
+    pass(std::integral_constant<int, 4>{}, tb);
+    tb += 4;
+  }
+  if (c1 - tb >= 2) {
+    pass(std::integral_constant<int, 2>{}, tb);
+    tb += 2;
+  }
+  if (c1 > tb) pass(std::integral_constant<int, 1>{}, tb);
 }
 
 // SERIES: the planar forms of jump_planar, in a kernel of their own: neither's
@@ -693,7 +701,9 @@ __global__ __launch_bounds__(64 * Form::kWaves, Form::kOccupancy) void k_mh_jump
   const int w = wv % kJumpSlices, group = wv / kJumpSlices;  // the wavefront's slice and chains
   constexpr int NG = WAVES / kJumpSlices;
   const int grp = blockIdx.x - e.wg0;
-  const int k0 = grp * e.cps, nc = min(e.cps, e.nch - k0);
+  const int k0 = jump_first(e, grp), nc = jump_first(e, grp + 1) - k0;
+  const int share = (nc + NG - 1) / NG;  // chains [g0, g1) of the group
+  const int g0 = min(nc, group * share), g1 = min(nc, g0 + share);
   const int c = e.cbase + k0 + lane;
   const bool mine = wv == 0 && lane < nc;  // this lane proposes and decides for a chain
   const int n = st[e.slot].n;
@@ -766,21 +776,21 @@ __global__ __launch_bounds__(64 * Form::kWaves, Form::kOccupancy) void k_mh_jump
     if (mine) store_site(s, wf, store, lane, it > a.it0);
     if (wv == 0) __builtin_amdgcn_s_setprio(0);
     if (kTip) {
-      jump_passes<4>(nc, NG, group, [&](auto tt, int tb) {
+      jump_passes<4, true>(g0, g1, [&](auto tt, int tb) {
         constexpr int T = decltype(tt)::value;
         double dx[T], dy[T], dz[T];
         jump_tip<Form, T>(kt, hi, lo, n, w, lane, &tgt[0][0], tb, dx, dy, dz);
         const double vx = wave_sums<T>(dx, lane), vy = wave_sums<T>(dy, lane),
                      vz = wave_sums<T>(dz, lane);
-        if ((lane & 7) == 0) {
-          const int k = tb + wave_slot<T>(lane);
+        const int k = tb + wave_slot<T>(lane);
+        if ((lane & 7) == 0 && k < g1) {
           red[0][w][k] = vx;
           red[kTip ? 1 : 0][w][k] = vy;
           red[kTip ? 2 : 0][w][k] = vz;
         }
       });
     } else if (kSurf0) {
-      jump_passes<8>(nc, NG, group, [&](auto tt, int tb) {
+      jump_passes<8, SERIES>(g0, g1, [&](auto tt, int tb) {
         constexpr int T = decltype(tt)::value;
         double d[T];
         if (held)
@@ -788,10 +798,11 @@ __global__ __launch_bounds__(64 * Form::kWaves, Form::kOccupancy) void k_mh_jump
         else
           jump_surf0<Form, T, false>(own[0], srx, srz, n, w, lane, &tgt2[tb], d);
         const double v = wave_sums<T>(d, lane);
-        if ((lane & 7) == 0) red[0][w][tb + wave_slot<T>(lane)] = v;
+        const int k = tb + wave_slot<T>(lane);
+        if ((lane & 7) == 0 && k < g1) red[0][w][k] = v;
       });
     } else {
-      jump_passes<8>(nc, NG, group, [&](auto tt, int tb) {
+      jump_passes<8, SERIES>(g0, g1, [&](auto tt, int tb) {
         constexpr int T = decltype(tt)::value;
         double d[T];
         if (ic)
@@ -799,7 +810,8 @@ __global__ __launch_bounds__(64 * Form::kWaves, Form::kOccupancy) void k_mh_jump
         else
           jump_planar<Form, T, false>(nic, dnm, hi, lo, n, w, lane, &tgt2[tb], d);
         const double v = wave_sums<T>(d, lane);
-        if ((lane & 7) == 0) red[0][w][tb + wave_slot<T>(lane)] = v;
+        const int k = tb + wave_slot<T>(lane);
+        if ((lane & 7) == 0 && k < g1) red[0][w][k] = v;
       });
     }
     __syncthreads();
@@ -908,7 +920,7 @@ __global__ __launch_bounds__(kJump64Threads, 3) void k_mh_jumps64(
   const int t = threadIdx.x, lane = t & 63;
   const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
   const int grp = blockIdx.x - e.wg0;
-  const int k0 = grp * e.cps, nc = min(e.cps, e.nch - k0);
+  const int k0 = jump_first(e, grp), nc = jump_first(e, grp + 1) - k0;
   const int c = e.cbase + k0 + lane;
   const bool mine = wv == 0 && lane < nc;
   const int n = st[e.slot].n;
