@@ -274,12 +274,14 @@ __device__ __forceinline__ float surface_far_eval(float t, float4 c0, float4 c1)
 constexpr int kSurfBlock = 16;
 
 // base + q z_b / r^3 of one source at the target t = (x, y, x_lo, y_lo): xy = (x, y,
-// x_lo, y_lo), zq = (z^2, q z), base(s) of the squared lateral distance s.
+// x_lo, y_lo), zq = (z, q z), base(s) of the squared lateral distance s.  z^2 goes
+// into the fused sum unrounded: staged as a product of its own, it raised the rms
+// error of a pair term (see kSurfBlock) with no instruction saved.
 template <class B>
 __device__ __forceinline__ float surface_term32(float4 t, float4 xy, float2 zq, B&& base) {
   const float dx = (t.x - xy.x) + (t.z - xy.z), dy = (t.y - xy.y) + (t.w - xy.w);
-  const float s = __builtin_fmaf(dy, dy, dx * dx);
-  const float ri = rsq(s + zq.x);
+  const float s = lateral2(dx, dy);
+  const float ri = rsq(__builtin_fmaf(zq.x, zq.x, s));
   return __builtin_fmaf(zq.y, ri * ri * ri, base(s));
 }
 
@@ -538,7 +540,7 @@ __device__ __forceinline__ void field_seg32(const DevGeom& g, bool split, bool a
       shi[t] = hv;
       slo[t] = lv;
       sxy[t] = make_float4(hv.x, hv.y, lv.x, lv.y);
-      szq[t] = make_float2(fmaxf(hv.z * hv.z, kR2Min), hv.w * hv.z);
+      szq[t] = make_float2(hv.z, hv.w * hv.z);
       if (boxes) {
         sfar[2 * t] = far[2 * (jb + t)];
         sfar[2 * t + 1] = far[2 * (jb + t) + 1];
