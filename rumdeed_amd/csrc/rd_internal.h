@@ -224,7 +224,7 @@ struct rd_ctx {
   // work buffers (grown on demand, never shrunk)
   rd::Buf part, pack_hi, pack_lo, pts, fld, pts_hi, pts_lo, stage, img64, tab, red, chains;
   rd::Buf pack_far;  // far-partner series of the particles (surface_far_coeffs)
-  rd::Buf pack_srx, pack_srz;  // cathode-surface sums of the jumps: (x, y) FP64, (z^2, q z) FP32, nm
+  rd::Buf pack_srx, pack_srz;  // cathode-surface sums of the jumps: (x, y) FP64, (z, q z) FP32, nm
   rd::Buf rnd;  // random numbers of the Metropolis-Hastings jumps of a step
   rd::Buf cnt;  // acceptance counters and widths of a step's jumps (rd_jumps.h)
   rd::Buf img_hi, img_lo;  // packed sphere images of the particles (mixed, tip)

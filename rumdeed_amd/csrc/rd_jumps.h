@@ -81,7 +81,7 @@ struct JumpArgs {
   const double *X, *Y, *Z, *Q;    // FP64 sources
   const float4 *HI, *LO;          // packed sources (mixed)
   const double2* SRX;             // (x, y) nm (mixed, cathode surface)
-  const float2* SRZ;              // (z^2, q z) nm
+  const float2* SRZ;              // (z, q z) nm
   const double *ru1, *ru2, *rlr;  // per jump and chain: unit normals, log-uniform ([it-1][C])
   unsigned long long* cnt;        // acceptance counters (jump_counter)
   double* width;                  // per entry: kWidthSlots values
@@ -466,13 +466,13 @@ __device__ __forceinline__ void jump_surf0(const HeldSrc<Form>& own, const doubl
     acc[u] = 0.0f;
     d[u] = 0.0;
   }
-  // r^2 = dx^2 + (dy^2 + z^2): as many roundings as (dx^2 + dy^2) + z^2, one
-  // instruction fewer; z^2 is at least kR2Min
-  auto term = [&](const double2 xy, float z2, float qz) {
+  // z^2 goes into the fused sum unrounded: a product of its own would save an
+  // instruction and bias all of a source's terms alike
+  auto term = [&](const double2 xy, float z, float qz) {
 #pragma unroll
     for (int u = 0; u < T; ++u) {
       const float dx = (float)(tx[u] - xy.x), dy = (float)(ty[u] - xy.y);
-      const float ri = rsq(__builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, z2)));
+      const float ri = rsq(__builtin_fmaf(z, z, lateral2(dx, dy)));
       acc[u] = __builtin_fmaf(qz, ri * ri * ri, acc[u]);
     }
   };

@@ -442,7 +442,7 @@ __global__ void k_pack_particles(const Ent* tab, const SimDesc* desc, const SimS
   lo[gi] = l;
   if (srx) {
     srx[gi] = make_double2(X[gi] * 1.0e9, Y[gi] * 1.0e9);
-    srz[gi] = make_float2(fmaxf(h.z * h.z, kR2Min), h.w * h.z);
+    srz[gi] = make_float2(h.z, h.w * h.z);
   }
 }
 
