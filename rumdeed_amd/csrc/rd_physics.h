@@ -154,19 +154,22 @@ RD_HD GtfConsts gtf_consts() {
   return k;
 }
 
+// `ok` turns false where a numerator, a difference of exponentials, is so small
+// that the residual of M's quotient would be subnormal and no longer exact (n is
+// ordinary, so the quotients are above num 2^-203 and the residuals above
+// num 2^-106).
 template <class M>
-__device__ __forceinline__ double gtf_Nns(double n, double s) {
+__device__ __forceinline__ double gtf_Nns(double n, double s, bool& ok) {
   if (n == 1.0) return (s + 1.0) * rd_exp(-s);
   double x = n * n;
   double y = M::rcp(x);
   double z = (n - 1.0) * s;
   const double es = rd_exp(-s), ens = rd_exp(-n * s);
-  double sng;
-  if (__builtin_fabs(z) > 1.0e-5)
-    sng = typename M::Div(x - 1.0)((x + 1.0) * (x * es - ens));
-  else
-    sng = typename M::Div(n + 1.0)(0.5 * (x + 1.0) * es) *
-          ((1.0 - n) * (s * s) + 2.0 * (1.0 + n) + 2.0 * s);
+  const bool apart = __builtin_fabs(z) > 1.0e-5;
+  const double num = apart ? (x + 1.0) * (x * es - ens) : 0.5 * (x + 1.0) * es;
+  ok = ok && (num == 0.0 || __builtin_fabs(num) >= 0x1p-800);
+  double sng = typename M::Div(apart ? x - 1.0 : n + 1.0)(num);
+  if (!apart) sng = sng * ((1.0 - n) * (s * s) + 2.0 * (1.0 + n) + 2.0 * s);
   double sn = -x * (0.10593434 * x + 0.35506593);
   double sd = -y * (0.10593434 * y + 0.35506593);
   double sfn = x * es;
@@ -223,7 +226,7 @@ __device__ __forceinline__ double gtf_current_by(double F, double To, double Phi
     sft = theta + betaT * (Em - chem);
   }
   ok = ok && f64_ordinary(nft) && nft != 0.0;
-  double J = k.Arld * gtf_Nns<M>(nft, sft) * (To * To);
+  double J = k.Arld * gtf_Nns<M>(nft, sft, ok) * (To * To);
   return J * 1.0e4;
 }
 
