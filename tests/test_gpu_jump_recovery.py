@@ -33,7 +33,7 @@ def _setup(dd, k):
                                       rng.uniform(30, 180, n)]) * NM)
 
 
-def _run(prec, pool, graphs, wait):
+def _run(prec, pool, graphs, wait, one=True):
     from rumdeed_amd.diode import Diode, Pool
 
     if pool:
@@ -47,6 +47,7 @@ def _run(prec, pool, graphs, wait):
         _setup(dd, 0)
     dd.set_graphs(graphs)
     dd.set_jump_wait(wait)
+    dd.set_solo_jumps(one)
     print(prec, "pool" if pool else "lone", "graphs" if graphs else "", "wait", wait, flush=True)
     if pool:
         recs = []
@@ -80,6 +81,12 @@ def test_repeated_jumps_equal_an_undisturbed_run(prec, pool, graphs):
         for a, b in zip(states, s):
             for f in STATE:
                 assert np.array_equal(a[f], b[f]), f
+
+
+@pytest.mark.parametrize("pool", [False, True])
+@pytest.mark.parametrize("prec", ["mixed", "fp64"])
+def test_graphs_leave_a_launch_per_jump_alone(prec, pool):
+    assert _run(prec, pool, True, -1, one=False)[0] == _run(prec, pool, False, -1)[0]
 
 
 def test_arguments():
