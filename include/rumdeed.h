@@ -287,16 +287,19 @@ int rd_set_jump_pairing(rd_ctx* ctx, int64_t min_workgroups);
 /* All Metropolis-Hastings jumps of a step in one launch (on != 0, the
  * default), or a launch per jump.  In one launch the workgroups of a planar FE
  * simulation wait, within a bound, for each other's acceptance counts of every
- * jump; a step in which they cannot all be resident takes a launch per jump by
- * itself.  Results are identical either way, in both precisions.  Library
- * control, no reference counterpart. */
+ * jump; a step in which a simulation would wait long for its last workgroup to
+ * find a place on the device takes a launch per jump by itself.  Results are
+ * identical either way, in both precisions.  Library control, no reference
+ * counterpart. */
 int rd_set_solo_jumps(rd_ctx* ctx, int32_t on);
 
 /* Bound of those waits in nanoseconds (negative, the default: 0.25 s, and in the
- * first jump 2 ms and eight times the workgroup's own jump).  A step in which a wait passes its bound, because
- * another context's work keeps workgroups off the device, repeats its jumps from
- * their start with a launch per jump, with the same results; a small bound
- * forces that.  Library control, no reference counterpart. */
+ * first jump of a launch whose workgroups all fit the device 2 ms; in the first jump
+ * eight times the workgroup's own jump is added).  A step in which a wait passes
+ * its bound, because another context's work keeps workgroups off the device,
+ * repeats its jumps from their start with a launch per jump, with the same
+ * results; a small bound forces that.  Library control, no reference
+ * counterpart. */
 int rd_set_jump_wait(rd_ctx* ctx, int64_t nanoseconds);
 /* Steps of this context whose jumps were repeated so. */
 int rd_jump_repeats(rd_ctx* ctx, int64_t* steps);
@@ -304,9 +307,10 @@ int rd_jump_repeats(rd_ctx* ctx, int64_t* steps);
 /* Forms of the mixed-precision planar accelerations (flags, 0 = both on,
  * the default).  RD_FORCE_NO_SYMMETRIC: every simulation takes the gather
  * form (each ordered pair evaluated at its target) instead of the
- * pair-symmetric form from 16384 particles.  RD_FORCE_NO_FAR_EXPANSION: the
- * image partners n >= 2 of the planar series are summed pair by pair in
- * FP32 instead of as one FP64 expansion of their field over all particles.
+ * pair-symmetric form from 5120 particles (12288 without image partners
+ * n >= 1).  RD_FORCE_NO_FAR_EXPANSION: the image partners n >= 2 of the planar
+ * series are summed pair by pair in FP32 instead of as one FP64 expansion of
+ * their field over all particles.
  * Library control for measurement and testing, no reference counterpart;
  * FP64 accelerations are not affected. */
 #define RD_FORCE_NO_SYMMETRIC 1

@@ -538,11 +538,11 @@ __global__ __launch_bounds__(256) void k_mh_start_check(const Ent* tab, const Si
 
 // Gaussian proposal of jump `it` (1-based) for a chain at (cx, cy) whose site
 // is (ox, oy, oz), with the width MH of the start of the jump and the unit
-// normal pair (u1, u2) of the chain's (step, jump) stream (box_muller_unit).  (a, b) are the chain coordinates
-// (planar x, y; tip xi, phi) and (x, y, z) the surface point whose field the
-// accept step needs.  valid: 1 proposal inside the patch, 0 tip proposal
-// outside it, -1 chain without a start site (the point is its final site and
-// nothing is recorded).
+// normal pair (u1, u2) of the chain's (step, jump) stream (box_muller_unit).
+// (a, b) are the chain coordinates (planar x, y; tip xi, phi) and (x, y, z) the
+// surface point whose field the accept step needs.  valid: 1 proposal inside the
+// patch, 0 tip proposal outside it, -1 chain without a start site (the point is
+// its final site and nothing is recorded).
 struct Proposal {
   double a, b, x, y, z;
   int valid;
@@ -1823,6 +1823,67 @@ static double jump_work(const DevGeom& g, JumpKind kind, int n) {
   return rounds * (g.ic ? 12.0 + 10.0 * g.nic : 17.0);
 }
 
+// The instructions a workgroup of nc chains keeps a CU's SIMDs busy for in a jump,
+// its own start and decision among them (FP64: whole passes of four chains by
+// four chunks, tip two).
+static double jump_time(const DevGeom& g, JumpKind kind, int n, int nc) {
+  if (kind == kJumpFp64) {
+    const int chunks = g.kind == RD_GEOM_TIP ? 2 : 4;
+    n = (n + chunks * kChunk - 1) / (chunks * kChunk) * (chunks * kChunk);
+    nc = (nc + kJump64T - 1) / kJump64T * kJump64T;
+  }
+  return nc * jump_work(g, kind, n) + kJumpStart[kind == kJumpMany];
+}
+
+// What a launch of the entries' workgroups in their order over `room` places takes,
+// and the longest wait of a simulation's first workgroup for its last one to be
+// given a place, both in instructions (jump_time).
+struct JumpSpan {
+  double time = 0.0, wait = 0.0;
+};
+static JumpSpan jump_span(const rd_ctx* c, const std::vector<Ent>& ents, JumpKind kind, int room,
+                          int per_cu) {
+  JumpSpan s;
+  using Places = std::pair<double, int>;  // places and the time they become free
+  std::vector<Places> free{{0.0, room}}, taken;  // latest first
+  free.reserve(ents.size() + 1);
+  auto give = [&](double t, int k) {
+    free.insert(std::upper_bound(free.begin(), free.end(), t,
+                                 [](double x, const Places& p) { return x > p.first; }),
+                {t, k});
+  };
+  for (const Ent& e : ents) {
+    const SimDesc& d = c->slots[e.slot].desc;
+    const double t = d.ndim * per_cu *
+                     jump_time(d.g, kind, e.n_ub, (e.nch + e.segs - 1) / e.segs);
+    const bool waits = e.segs > 1 && d.mode == RD_EMIT_PLANAR_FE;
+    if (waits && e.segs > room) s.wait = INFINITY;  // never resident
+    const double first = free.back().first;
+    double last = first;
+    for (int need = e.segs; need > 0;) {
+      Places& p = free.back();
+      const int k = std::min(need, p.second);
+      last = p.first;
+      taken.push_back({last, k});
+      need -= k;
+      if ((p.second -= k) == 0) free.pop_back();
+      if (need > 0 && free.empty()) {  // more workgroups than places: the first again
+        for (const Places& u : taken) give(u.first + t, u.second);
+        taken.clear();
+      }
+    }
+    if (waits) {
+      give(last + t, e.segs);
+      s.wait = std::max(s.wait, last - first);
+    } else {
+      for (const Places& u : taken) give(u.first + t, u.second);
+    }
+    taken.clear();
+    s.time = std::max(s.time, last + t);
+  }
+  return s;
+}
+
 // Chains a workgroup of the jump kernels takes: about `target` instructions per
 // SIMD and jump, in a number that the wavefronts can share evenly, at least two
 // where each particle is read from memory in every jump.  FILL: at least the
@@ -1844,6 +1905,28 @@ static int jump_chains(JumpKind kind, double work, double target) {
     if (FILL || k <= want) cw = k;
   }
   return cw;
+}
+
+// A launch per jump: the chains per workgroup with the least time, of the fullest
+// compute unit or the longest workgroup, and that time with the launch
+// (jump_time's instructions).
+static double jump_apart(const rd_ctx* c, const std::vector<Ent>& ents, JumpKind kind, int cus,
+                         int* chains) {
+  double best = INFINITY;
+  for (int k = kJumpApart; k >= 4; k -= 4) {
+    double total = 0.0, longest = 0.0;
+    for (const Ent& e : ents) {
+      const double t = jump_time(c->slots[e.slot].desc.g, kind, e.n_ub, std::min(k, e.nch));
+      total += t * ((e.nch + k - 1) / k);
+      longest = std::max(longest, t);
+    }
+    const double time = std::max(std::ceil(total / longest / cus), 1.0) * longest;
+    if (time < best) {
+      best = time;
+      *chains = k;
+    }
+  }
+  return best + kJumpLaunch;
 }
 
 // The Metropolis-Hastings jumps 1..maxndim of the chain entries `in` (C chains
@@ -1938,39 +2021,60 @@ static int run_jumps(rd_ctx* c, const std::vector<Ent>& in, int C, int precision
     }
   };
   lay_out([&](double work) { return jump_chains<false>(kind, work, kJumpTarget); });
-  for (double target = kJumpTarget; nwg > room;) {
-    int least = kJumpLanes;
-    target *= 1.05;
-    lay_out([&](double work) {
-      const int cw = jump_chains<true>(kind, work, target);
-      least = std::min(least, cw);
-      return cw;
-    });
-    if (least == kJumpLanes) break;  // every workgroup is full
-  }
-  // Workgroups that wait for each other have to be resident together; where they
-  // cannot, or by choice, a launch per jump.
-  const bool spin = c->solo_jumps && (!waits || nwg <= room);
-  if (!spin) {
-    // nothing has to be resident: the number of chains with the least time of
-    // the fullest compute unit
-    double total = 0.0, best = 0.0;
-    for (const Ent& e : ents) total += e.nch * jump_work(c->slots[e.slot].desc.g, kind, e.n_ub);
-    int least = kJumpApart;
-    for (int k = kJumpApart; k >= 4; k -= 4) {
-      long long groups = 0;
-      for (const Ent& e : ents) groups += (e.nch + k - 1) / k;
-      const double time =
-          (double)((groups + cus - 1) / cus) * (k * (total / C) + kJumpStart[kind == kJumpMany]);
-      if (k == kJumpApart || time < best) {
-        best = time;
-        least = k;
+  // Beyond the device's room: larger targets, by their estimated times, or
+  // - the smallest with all workgroups resident (pools of like diodes, lone ones),
+  // - one of fewer chains and more workgroups, the large simulations' first and
+  //   the small ones' in the places that become free (pools of uneven diodes), if
+  //   no simulation waits long for its last workgroup's place,
+  // - a launch per jump, where nothing has to be resident.
+  bool spin = c->solo_jumps;
+  if (nwg > room) {
+    double best = INFINITY, best_target = 0.0;
+    int least = 0;
+    auto fill = [&](double target) {
+      least = kJumpLanes;
+      lay_out([&](double work) {
+        const int cw = jump_chains<true>(kind, work, target);
+        least = std::min(least, cw);
+        return cw;
+      });
+      return nwg <= room;
+    };
+    auto consider = [&](double target, double handicap) {
+      const JumpSpan span = jump_span(c, ents, kind, room, room / cus);
+      if (waits && span.wait > kJumpLate) return;
+      if (span.time * handicap < best) {
+        best = span.time * handicap;
+        best_target = target;
       }
+    };
+    double target = kJumpTarget;
+    bool fits = false;
+    do {
+      target *= 1.2;
+      fits = fill(target);
+      if (!fits && nwg <= 2 * room) consider(target, 1.0);
+    } while (!fits && least < kJumpLanes);
+    if (fits) {
+      for (target /= 1.2; !fill(target *= 1.05);) {
+      }
+      consider(target, kJumpFits[fp64]);
+    } else {
+      consider(target, 1.0);
     }
-    lay_out([&](double) { return least; });
+    int k = 0;
+    spin = spin && best_target > 0.0 &&
+           (!waits || best < maxndim * jump_apart(c, ents, kind, cus, &k));
+    if (spin) fill(best_target);
+  }
+  if (!spin) {
+    int k = 0;
+    jump_apart(c, ents, kind, cus, &k);
+    lay_out([&](double) { return k; });
   }
   a.C = C;
-  a.wait = c->jump_wait;
+  a.later = c->jump_wait >= 0 ? c->jump_wait : kSpinTicks;
+  a.first = c->jump_wait >= 0 ? c->jump_wait : nwg <= room ? kFirstTicks : kSpinTicks;
   const size_t nr = (size_t)maxndim * C;
   r = ensure(c, c->rnd, sizeof(double) * 3 * nr);
   if (r) return r;

@@ -190,6 +190,16 @@ constexpr double kJumpTarget = 400.0;
 // chains: N_ic_max = 0 95 / 68 / 62, 1 121 / 103 / 110, 10 374 / 383 / 433.
 constexpr int kJumpApart = 32;
 constexpr double kJumpStart[2] = {1600.0, 4500.0};
+// A launch in those instructions (6 us), and the longest estimated wait of a
+// simulation for its last workgroup's place (20 ms; the wait's bound is 0.25 s).
+constexpr double kJumpLaunch = 2700.0, kJumpLate = 9.0e6;
+// Estimated time of a launch that fits the device, as a part of itself, below
+// which it is taken before one of more workgroups: mixed (two workgroups on a CU,
+// whose second one overlaps) and FP64.  Serving streams of 64 / 128 / 24 uneven
+// diodes, simulations an hour in thousands, fitting launches alone / by this
+// rule: mixed 153 / 147, 117 / 143, 86.5 / 85.5 (launches cut off after 24 steps of
+// the search, as they were: 141, 123, 84), FP64 64 and 24 30 / 43, 32.5 / 32.3 (38, 28).
+constexpr double kJumpFits[2] = {0.6, 0.9};
 
 // Partial sums of one pair launch are bounded by this many bytes (512 MiB);
 // larger launches run in bands whose partials are folded, in order, into

@@ -24,18 +24,19 @@
 // chains) 5.4 -> 3.9 ms; thermal-field mixed 5.5 -> 4.8 ms; 64 diodes of a pool
 // mixed 14.0 -> 12.2 ms, FP64 38.7 -> 26.6 ms.
 //
-// Every workgroup of a simulation has to be resident for the wait to end, so the
-// host starts workgroups that wait only where the whole launch fits the device,
-// and else a launch per jump (spin = 0), where the end of the launch takes the
-// place of the wait.  (One launch whose later simulations wait for room lost to
-// it: 40 diodes of 3400 electrons, ten image terms, mixed 181 against 129 ms;
-// FP64 1226 against 714, the wait's bound passed.)  Another context's work can
-// still hold the CUs, so the wait is bounded: past its bound the workgroup raises
-// `stop` and leaves; results go to arrays of their own (`out`), and the host
-// repeats the step's jumps with a launch per jump, with the same results.  Once
-// the first jump's counts are in, every workgroup is resident, so two contexts
-// that keep each other's workgroups out find that out in the first wait, which is
-// short (kFirstTicks and eight times the workgroup's own first jump: the
+// Every workgroup of a simulation has to be resident for the wait to end.  A
+// launch's workgroups start in order and no simulation has more than the device
+// holds, so the earliest unfinished simulation always is.  The host (run_jumps)
+// also sees to it that none waits long for its last workgroup's place: a launch
+// fits the device, or small simulations follow large ones in the places that
+// become free (uneven pools), or each jump is a launch (spin = 0), where the end of
+// the launch takes the place of the wait.  Another context's work can still hold
+// the CUs, so the wait is bounded: past its bound the workgroup raises `stop` and
+// leaves; results go to arrays of their own (`out`), and the host repeats the
+// step's jumps with a launch per jump, with the same results.  Once the first
+// jump's counts are in, every workgroup is resident, so two contexts that keep each
+// other's workgroups out find that out in the first wait; where the launch fits
+// that is short (kFirstTicks and eight times the workgroup's own first jump: the
 // workgroups of a simulation differ by one chain, and by their CU's other load).
 //
 // The sums' order depends on the simulation's particle count and the kind of
@@ -47,10 +48,10 @@
 // simulation takes workgroups of four wavefronts, a slice each, over many
 // CUs, or, with many particles, of sixteen wavefronts and slices, which hide
 // the particles' loads; a pool workgroups of eight wavefronts that share four
-// slices, two of them on a CU, so that one's decisions overlap the other's sums.  FP64: the canonical order (partials of 256
-// particles, each in sequence, added in order): the lanes form the terms in
-// parallel, LDS holds them, and a lane per (chain, chunk) adds its 256 in
-// sequence.
+// slices, two of them on a CU, so that one's decisions overlap the other's sums.
+// FP64: the canonical order (partials of 256 particles, each in sequence, added in
+// order): the lanes form the terms in parallel, LDS holds them, and a lane per
+// (chain, chunk) adds its 256 in sequence.
 #pragma once
 
 namespace rd {
@@ -89,7 +90,7 @@ struct JumpArgs {
   int C;                          // chains in all
   int it0, it1;                   // jumps it0 .. it1 - 1 of this launch
   int spin;                       // 1: all jumps in this launch; 0: a launch per jump
-  long long wait;                 // bound of the waits (ticks); negative: the default
+  long long first, later;         // bounds of the waits after jump 1 and later (ticks)
 };
 
 // Per entry: the width and rate of the jumps of either parity (a launch per
@@ -250,7 +251,7 @@ struct JumpWidth {
   int first, fe;
   unsigned long long* w;  // counter words of jump 1
   int words, groups, grp, spin;
-  long long wait;
+  long long first_wait, later_wait;
   int* stop;
   double* slot;
   long long t0 = wall_clock64();
@@ -259,7 +260,7 @@ struct JumpWidth {
                                        const JumpArgs& a, int grp_)
       : mh(S.MH_std), rate(S.a_rate), first(nint(s.ndim * 0.25)),
         fe(s.mode == RD_EMIT_PLANAR_FE), w(a.cnt + e.part_off), words(e.pslots), groups(e.segs),
-        grp(grp_), spin(a.spin), wait(a.wait), stop(a.stop),
+        grp(grp_), spin(a.spin), first_wait(a.first), later_wait(a.later), stop(a.stop),
         slot(a.width + (size_t)kWidthSlots * e.acc_off) {
     if (fe && !spin && a.it0 >= 2) {  // as the launch of the jump before left it
       mh = slot[(a.it0 - 1) & 1];
@@ -269,9 +270,7 @@ struct JumpWidth {
   // The width after jump `it`.
   __device__ __forceinline__ bool after(int it) {
     if (groups > 1 || !spin) {
-      const long long ticks = wait >= 0 ? wait
-                              : it == 1 ? kFirstTicks + 8 * (wall_clock64() - t0)
-                                        : kSpinTicks;
+      const long long ticks = it == 1 ? first_wait + 8 * (wall_clock64() - t0) : later_wait;
       if (!counts_wait(w + (size_t)(it - 1) * words, groups, spin, stop, ticks, na, nr))
         return false;
     }

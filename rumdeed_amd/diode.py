@@ -118,8 +118,8 @@ class Diode:
 
     def set_force_options(self, no_symmetric: bool = False, no_far_expansion: bool = False):
         """Forms of the mixed planar accelerations (rd_set_force_options):
-        by default the pair-symmetric form from 16384 particles and the far
-        image partners (n >= 2) as one FP64 expansion."""
+        by default the pair-symmetric form from 5120 particles (12288 without
+        partners n >= 1) and the far partners (n >= 2) as one FP64 expansion."""
         flags = (1 if no_symmetric else 0) | (2 if no_far_expansion else 0)
         check(self._lib.rd_set_force_options(self._h, flags))
 
