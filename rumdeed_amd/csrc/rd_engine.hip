@@ -1823,26 +1823,40 @@ static double jump_work(const DevGeom& g, JumpKind kind, int n) {
   return rounds * (g.ic ? 12.0 + 10.0 * g.nic : 17.0);
 }
 
-// The instructions a workgroup of nc chains keeps a CU's SIMDs busy for in a jump,
-// its own start and decision among them (FP64: whole passes of four chains by
-// four chunks, tip two).
-static double jump_time(const DevGeom& g, JumpKind kind, int n, int nc) {
-  if (kind == kJumpFp64) {
-    const int chunks = g.kind == RD_GEOM_TIP ? 2 : 4;
-    n = (n + chunks * kChunk - 1) / (chunks * kChunk) * (chunks * kChunk);
-    nc = (nc + kJump64T - 1) / kJump64T * kJump64T;
+// What the layout of a launch takes from one entry.
+struct JumpLoad {
+  double work;   // jump_work
+  double full;   // the same of whole passes (FP64: four chunks, tip two)
+  double start;  // a workgroup's own start and decision
+  int kind, groups, ndim;
+  bool tip, exact;  // as jump_passes takes a workgroup's chains
+  bool fe;          // planar FE: its workgroups wait for each other
+  JumpLoad(const SimDesc& d, JumpKind k, int n)
+      : work(jump_work(d.g, k, n)), full(work), start(kJumpStart[k == kJumpMany]), kind(k),
+        groups(k == kJumpPool ? PoolForm::kWaves / PoolForm::kSlices : 1), ndim(d.ndim),
+        tip(d.g.kind == RD_GEOM_TIP), exact(jump_series(d.g)), fe(d.mode == RD_EMIT_PLANAR_FE) {
+    const int chunk = kChunk * (tip ? 2 : 4);
+    if (kind == kJumpFp64) full = jump_work(d.g, k, (n + chunk - 1) / chunk * chunk);
   }
-  return nc * jump_work(g, kind, n) + kJumpStart[kind == kJumpMany];
-}
+  // nc chains and the idle places of their passes.
+  int places(int nc) const {
+    if (kind == kJumpFp64) return (nc + kJump64T - 1) / kJump64T * kJump64T;
+    const int q = (nc + groups - 1) / groups, r = q % (tip ? 4 : 8);
+    const int idle = r == 3 || r == 7 ? 1 : r > 4 && !exact ? 8 - r : 0;
+    return idle ? groups * (q + idle) : nc;
+  }
+  // The instructions a workgroup of nc chains keeps a CU's SIMDs busy for in a jump.
+  double time(int nc) const { return places(nc) * full + start; }
+};
 
 // What a launch of the entries' workgroups in their order over `room` places takes,
 // and the longest wait of a simulation's first workgroup for its last one to be
-// given a place, both in instructions (jump_time).
+// given a place, both in instructions.
 struct JumpSpan {
   double time = 0.0, wait = 0.0;
 };
-static JumpSpan jump_span(const rd_ctx* c, const std::vector<Ent>& ents, JumpKind kind, int room,
-                          int per_cu) {
+static JumpSpan jump_span(const std::vector<Ent>& ents, const std::vector<JumpLoad>& loads,
+                          int room, int per_cu) {
   JumpSpan s;
   using Places = std::pair<double, int>;  // places and the time they become free
   std::vector<Places> free{{0.0, room}}, taken;  // latest first
@@ -1852,15 +1866,14 @@ static JumpSpan jump_span(const rd_ctx* c, const std::vector<Ent>& ents, JumpKin
                                  [](double x, const Places& p) { return x > p.first; }),
                 {t, k});
   };
-  for (const Ent& e : ents) {
-    const SimDesc& d = c->slots[e.slot].desc;
-    const double t = d.ndim * per_cu *
-                     jump_time(d.g, kind, e.n_ub, (e.nch + e.segs - 1) / e.segs);
-    const bool waits = e.segs > 1 && d.mode == RD_EMIT_PLANAR_FE;
-    if (waits && e.segs > room) s.wait = INFINITY;  // never resident
+  for (size_t i = 0; i < ents.size(); ++i) {
+    const int segs = ents[i].segs;
+    const double t = (double)loads[i].ndim * per_cu * loads[i].time((ents[i].nch + segs - 1) / segs);
+    const bool waits = segs > 1 && loads[i].fe;
+    if (waits && segs > room) s.wait = INFINITY;  // never resident
     const double first = free.back().first;
     double last = first;
-    for (int need = e.segs; need > 0;) {
+    for (int need = segs; need > 0;) {
       Places& p = free.back();
       const int k = std::min(need, p.second);
       last = p.first;
@@ -1873,7 +1886,7 @@ static JumpSpan jump_span(const rd_ctx* c, const std::vector<Ent>& ents, JumpKin
       }
     }
     if (waits) {
-      give(last + t, e.segs);
+      give(last + t, segs);
       s.wait = std::max(s.wait, last - first);
     } else {
       for (const Places& u : taken) give(u.first + t, u.second);
@@ -1888,19 +1901,17 @@ static JumpSpan jump_span(const rd_ctx* c, const std::vector<Ent>& ents, JumpKin
 // SIMD and jump, in a number that the wavefronts can share evenly, at least two
 // where each particle is read from memory in every jump.  FILL: at least the
 // target, and beyond 16 chains, where a workgroup takes several passes, any
-// number (FP64: whole passes), so that the workgroups fill the device evenly
+// number without idle places, so that the workgroups fill the device evenly
 // (20 000 electrons, 5652 chains, ms: 177 workgroups of 32 14.0, 236 of 24 11.1).
 template <bool FILL>
-static int jump_chains(JumpKind kind, double work, double target) {
-  const double want = target / work;
-  if (FILL && want > 16.0) {
-    const int k = (int)std::min<double>(kJumpLanes, std::ceil(want));
-    return kind == kJumpFp64 ? (k + kJump64T - 1) / kJump64T * kJump64T : k;
-  }
-  const int least = kind == kJumpFp64 ? 4 : kind == kJumpLone ? 1 : 2;
+static int jump_chains(const JumpLoad& load, double target) {
+  const double want = target / load.work;
+  if (FILL && want > 16.0)
+    return std::min(kJumpLanes, load.places((int)std::min<double>(kJumpLanes, std::ceil(want))));
+  const int least = load.kind == kJumpFp64 ? 4 : load.kind == kJumpLone ? 1 : 2;
   int cw = least;
   for (int k : {1, 2, 4, 8, 12, 16, 24, 32, 48, 64}) {
-    if (k < least || (kind == kJumpPool && k == 12)) continue;
+    if (k < least || (load.kind == kJumpPool && k == 12)) continue;
     if (FILL && cw >= want) break;
     if (FILL || k <= want) cw = k;
   }
@@ -1909,15 +1920,15 @@ static int jump_chains(JumpKind kind, double work, double target) {
 
 // A launch per jump: the chains per workgroup with the least time, of the fullest
 // compute unit or the longest workgroup, and that time with the launch
-// (jump_time's instructions).
-static double jump_apart(const rd_ctx* c, const std::vector<Ent>& ents, JumpKind kind, int cus,
+// (instructions).
+static double jump_apart(const std::vector<Ent>& ents, const std::vector<JumpLoad>& loads, int cus,
                          int* chains) {
   double best = INFINITY;
   for (int k = kJumpApart; k >= 4; k -= 4) {
     double total = 0.0, longest = 0.0;
-    for (const Ent& e : ents) {
-      const double t = jump_time(c->slots[e.slot].desc.g, kind, e.n_ub, std::min(k, e.nch));
-      total += t * ((e.nch + k - 1) / k);
+    for (size_t i = 0; i < ents.size(); ++i) {
+      const double t = loads[i].time(std::min(k, ents[i].nch));
+      total += t * ((ents[i].nch + k - 1) / k);
       longest = std::max(longest, t);
     }
     const double time = std::max(std::ceil(total / longest / cus), 1.0) * longest;
@@ -2001,26 +2012,32 @@ static int run_jumps(rd_ctx* c, const std::vector<Ent>& in, int C, int precision
   });
   // Chains per workgroup: from the smallest target that lets every workgroup be
   // resident at once.
+  std::vector<JumpLoad> loads;
+  loads.reserve(ents.size());
+  for (const Ent& e : ents) loads.emplace_back(c->slots[e.slot].desc, kind, e.n_ub);
   int nwg = 0;
   long long words = 0;
-  bool waits = false;  // a simulation whose workgroups wait for each other
+  bool waits = false;    // a simulation whose workgroups wait for each other
+  double longest = 0.0;  // a workgroup's time, at least
   auto lay_out = [&](auto&& chains) {
     nwg = 0;
     words = 0;
     waits = false;
-    for (Ent& e : ents) {
-      const SimDesc& d = c->slots[e.slot].desc;
-      e.cps = chains(jump_work(d.g, kind, e.n_ub));
+    longest = 0.0;
+    for (size_t i = 0; i < ents.size(); ++i) {
+      Ent& e = ents[i];
+      e.cps = chains(loads[i]);
       e.segs = (e.nch + e.cps - 1) / e.cps;
       e.wg0 = nwg;
       nwg += e.segs;
       e.pslots = jump_words(e.segs);
       e.part_off = words;
-      words += (long long)e.pslots * d.ndim;
-      waits |= e.segs > 1 && d.mode == RD_EMIT_PLANAR_FE;
+      words += (long long)e.pslots * loads[i].ndim;
+      waits |= e.segs > 1 && loads[i].fe;
+      longest = std::max(longest, loads[i].ndim * loads[i].time((e.nch + e.segs - 1) / e.segs));
     }
   };
-  lay_out([&](double work) { return jump_chains<false>(kind, work, kJumpTarget); });
+  lay_out([](const JumpLoad& l) { return jump_chains<false>(l, kJumpTarget); });
   // Beyond the device's room: larger targets, by their estimated times, or
   // - the smallest with all workgroups resident (pools of like diodes, lone ones),
   // - one of fewer chains and more workgroups, the large simulations' first and
@@ -2033,15 +2050,16 @@ static int run_jumps(rd_ctx* c, const std::vector<Ent>& in, int C, int precision
     int least = 0;
     auto fill = [&](double target) {
       least = kJumpLanes;
-      lay_out([&](double work) {
-        const int cw = jump_chains<true>(kind, work, target);
+      lay_out([&](const JumpLoad& l) {
+        const int cw = jump_chains<true>(l, target);
         least = std::min(least, cw);
         return cw;
       });
       return nwg <= room;
     };
     auto consider = [&](double target, double handicap) {
-      const JumpSpan span = jump_span(c, ents, kind, room, room / cus);
+      if (longest * (room / cus) * handicap >= best) return;
+      const JumpSpan span = jump_span(ents, loads, room, room / cus);
       if (waits && span.wait > kJumpLate) return;
       if (span.time * handicap < best) {
         best = span.time * handicap;
@@ -2053,7 +2071,7 @@ static int run_jumps(rd_ctx* c, const std::vector<Ent>& in, int C, int precision
     do {
       target *= 1.2;
       fits = fill(target);
-      if (!fits && nwg <= 2 * room) consider(target, 1.0);
+      if (!fits && nwg <= 4 * room) consider(target, 1.0);
     } while (!fits && least < kJumpLanes);
     if (fits) {
       for (target /= 1.2; !fill(target *= 1.05);) {
@@ -2064,13 +2082,13 @@ static int run_jumps(rd_ctx* c, const std::vector<Ent>& in, int C, int precision
     }
     int k = 0;
     spin = spin && best_target > 0.0 &&
-           (!waits || best < maxndim * jump_apart(c, ents, kind, cus, &k));
+           (!waits || best < maxndim * jump_apart(ents, loads, cus, &k));
     if (spin) fill(best_target);
   }
   if (!spin) {
     int k = 0;
-    jump_apart(c, ents, kind, cus, &k);
-    lay_out([&](double) { return k; });
+    jump_apart(ents, loads, cus, &k);
+    lay_out([&](const JumpLoad&) { return k; });
   }
   a.C = C;
   a.later = c->jump_wait >= 0 ? c->jump_wait : kSpinTicks;

@@ -197,8 +197,8 @@ constexpr double kJumpLaunch = 2700.0, kJumpLate = 9.0e6;
 // which it is taken before one of more workgroups: mixed (two workgroups on a CU,
 // whose second one overlaps) and FP64.  Serving streams of 64 / 128 / 24 uneven
 // diodes, simulations an hour in thousands, fitting launches alone / by this
-// rule: mixed 153 / 147, 117 / 143, 86.5 / 85.5 (launches cut off after 24 steps of
-// the search, as they were: 141, 123, 84), FP64 64 and 24 30 / 43, 32.5 / 32.3 (38, 28).
+// rule: mixed 153 / 145, 117 / 143, 86.5 / 86.4 (launches cut off after 24 steps of
+// the search: 145, 123, 84), FP64 64 and 24 30 / 43, 32.5 / 32.3 (38, 28).
 constexpr double kJumpFits[2] = {0.6, 0.9};
 
 // Partial sums of one pair launch are bounded by this many bytes (512 MiB);
