@@ -48,11 +48,11 @@ COPY_BYTES = 1 << 30  # calibration copy: 1 GiB read + 1 GiB written per launch
 # workload and kernel form only.  The writes are the kernel's FP64 partial
 # sums, 3 x 128 blocks x N doubles = 201.33 MB; the reads are the packed
 # particles (32 B each) as the block pairs fetch them, mostly from L2.
-MEASURED_TRAFFIC = {("k_accel_sym32", 65536, 10): {"read": 41.982e6, "write": 201.327e6}}
-# VALU issue of the same dispatch (profiles/snapshot65536_nic10_valu_counters.txt):
-# SQ_INSTS_VALU over 1024 SIMDs x 2.4 GHz x duration / 4 cycles per wave64
-# instruction.
-MEASURED_VALU_ISSUE = {("k_accel_sym32", 65536, 10): 1.012}
+MEASURED_TRAFFIC = {("k_accel_sym32", 65536, 10): {"read": 41.908e6, "write": 201.327e6}}
+# VALU instructions of the same dispatch (profiles/snapshot65536_nic10_valu_counters.txt)
+# per SIMD and 4 cycles at 2.4 GHz.  Not a fraction of a ceiling: FP32 instructions
+# with vector operands issue at up to 1.6 of these, FP64 ones at 0.93, roots at 0.24-0.47.
+MEASURED_VALU_PER_4_CYCLES = {("k_accel_sym32", 65536, 10): 1.051}
 
 
 def cpu_baseline(n_sample: int, nic: int, threads: int):
@@ -417,7 +417,8 @@ def main():
     far = W.far_expansion_used(pos, W.SNAPSHOT_D, nic)
     tot_ms, ker_ms = dd.time_accel("mixed", reps=5)
     flops = W.force_flops(n, nic, "mixed", far_expansion=far)
-    kernel = "k_accel_sym32" if n >= W.SYM_MIN else "k_accel_planar32"
+    sym_min = W.SYM_MIN if nic > 0 else W.SYM_MIN_LIGHT
+    kernel = "k_accel_sym32" if n >= sym_min else "k_accel_planar32"
     nic_pair = min(nic, 1) if far else nic
     achieved = flops / (ker_ms * 1e-3) / 1e12
     # like for like: the same accelerations in mixed precision with each ordered
@@ -475,7 +476,7 @@ def main():
                      "traffic": traffic and traffic["read"] + traffic["write"],
                      "traffic_read_write": traffic,
                      "traffic_unit": "bytes per launch (HBM read + write, counter passes)",
-                     "valu_issue_frac": MEASURED_VALU_ISSUE.get((kernel, n, nic)),
+                     "valu_instructions_per_4_cycles": MEASURED_VALU_PER_4_CYCLES.get((kernel, n, nic)),
                      "kernel": kernel,
                      "flops_per_launch": flops,
                      "image_partners_in_kernel": 1 + 4 * nic_pair,

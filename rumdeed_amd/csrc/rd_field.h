@@ -497,12 +497,12 @@ __device__ __forceinline__ void add_quarters(void* lds, double& fx, double& fy, 
 // of chunks [c0, c1) at the packed target (h1, l1); split: of this wavefront's
 // quarters of them.
 //
-// On the cathode the pair terms are bound by VALU issue (the far series 22
+// On the cathode the pair terms are bound by VALU issue (the far series 23
 // instructions a pair, without 11; two or four targets per lane, which halve and
 // quarter the LDS and scalar reads, measured the same).  65 536 electrons at 256
-// x 256 points: 2.02 -> 1.87 ms with the far series, 1.37 -> 1.18 without, by terms
-// without products or additions of their own (charge in the series, z^2 and q z
-// formed at staging, the direct term added by the product).
+// x 256 points: 2.02 -> 1.90 ms with the far series, 1.37 -> 1.18 without, by terms
+// without products or additions of their own (charge in the series, q z formed at
+// staging, z^2 in the sum under the root, the direct term added by the product).
 __device__ __forceinline__ void field_seg32(const DevGeom& g, bool split, bool act, float4 h1,
                                             float4 l1,
                                             const float4* __restrict__ hi,
